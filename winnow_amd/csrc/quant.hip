@@ -5,57 +5,18 @@
 //   n = max(||x||_2, 1e-10);  y = (x / n) Pi^T;  code = #{boundaries < y}
 // A work-group quantizes sixteen vectors (quantize_kernel on the float64 matrix
 // cores at head_dim 64 and 128, quantize_any_kernel on the vector ALU at 16, 32 and
-// 256). The squared norm and the rotation are
+// 256); many vectors at 64 and 128 run on quant_tile.hip, with the same codes. The squared norm and the rotation are
 // accumulated in float64 from exact fp32 inputs and rounded once to fp32, and
 // x / n is the correctly rounded fp32 quotient, so every code is the bucket of
 // the correctly rounded fp32 y; an fp32 GEMM elsewhere can differ from it only
 // when its own rounding error crosses a boundary.
-#include "wn_common.h"
+#include "wn_quant.h"
 
 namespace wn {
 namespace {
 
 constexpr int kQBlock = 256;                // 4 waves
 constexpr int kVecPerBlock = 16;            // vectors per work-group (the rows of one f64 MFMA tile)
-
-struct QuantSide {
-  const void* x;
-  int64_t sb, sh, sn;  // element strides of (B, H, n, D)
-  const float* pi;
-  const float* bnd;
-  int bw;
-  uint8_t* pages;  // scatter mode
-  int64_t psp, psh;
-  uint16_t* norms;
-  int64_t nsp, nsh;
-  uint8_t* codes_out;  // flat mode
-  float* norms_out;
-};
-
-struct QuantArgs {
-  QuantSide side[2];
-  const int32_t* table;
-  const int32_t* start_pos;
-  int64_t tsb;
-  int64_t total;  // vectors per side = B*H*n
-  int H, n, log2S, num_pages, max_pages, x_dtype, scatter;
-};
-
-// pos[k] = #{b < y[k]} over the 2^bw - 1 ascending boundaries (torch.bucketize,
-// right=False), for N values at once: the N binary searches advance in lockstep, so
-// each level issues N independent LDS reads instead of one dependent read per value.
-template <int N>
-__device__ __forceinline__ void bucketize_n(const float* bnd, int bw, const float (&y)[N], uint32_t (&pos)[N]) {
-#pragma unroll
-  for (int k = 0; k < N; ++k) pos[k] = 0;
-  for (int step = 1 << (bw - 1); step > 0; step >>= 1) {
-    float b[N];
-#pragma unroll
-    for (int k = 0; k < N; ++k) b[k] = bnd[pos[k] + step - 1];
-#pragma unroll
-    for (int k = 0; k < N; ++k) pos[k] += b[k] < y[k] ? step : 0;
-  }
-}
 
 // Byte k of the LSB-first packing of `codes` (D codes of bw bits).
 __device__ __forceinline__ uint8_t packed_byte(const uint8_t* codes, int k, int bw, int D) {
@@ -67,24 +28,6 @@ __device__ __forceinline__ uint8_t packed_byte(const uint8_t* codes, int k, int 
     v |= off >= 0 ? (c << off) : (c >> (-off));
   }
   return uint8_t(v & 0xffu);
-}
-
-// The bw bytes of eight bw-bit codes packed LSB-first, stored at p (p is aligned to
-// the largest power of two dividing bw).
-__device__ __forceinline__ void store_packed8(uint8_t* p, uint64_t v, int bw) {
-  if (bw == 8) {
-    *reinterpret_cast<uint2*>(p) = make_uint2(uint32_t(v), uint32_t(v >> 32));
-  } else if (bw == 4) {
-    *reinterpret_cast<uint32_t*>(p) = uint32_t(v);
-  } else if (bw == 2) {
-    *reinterpret_cast<uint16_t*>(p) = uint16_t(v);
-  } else if (bw == 6) {
-    reinterpret_cast<uint16_t*>(p)[0] = uint16_t(v);
-    reinterpret_cast<uint16_t*>(p)[1] = uint16_t(v >> 16);
-    reinterpret_cast<uint16_t*>(p)[2] = uint16_t(v >> 32);
-  } else {
-    for (int k = 0; k < bw; ++k) p[k] = uint8_t(v >> (8 * k));
-  }
 }
 
 // A work-group quantizes sixteen vectors (sixteen per work-group keep even a
@@ -507,7 +450,13 @@ static int launch_quantize(QuantArgs& a, int sides, int D, hipStream_t st, const
   if (a.total == 0) return WN_OK;
   dim3 grid(unsigned((a.total + kVecPerBlock - 1) / kVecPerBlock), sides);
   if (ev_begin) hipEventRecord(static_cast<hipEvent_t>(ev_begin), st);
-  switch (D) {
+  if (quantize_tiles_ok(a, sides, D)) {
+    const int rc = launch_quantize_tiles(a, sides, D, st);
+    if (rc != WN_OK) {
+      set_error("%s: cannot query the device", what);
+      return rc;
+    }
+  } else switch (D) {
     case 16: hipLaunchKernelGGL(quantize_any_kernel<16>, grid, dim3(kQBlock), 0, st, a); break;
     case 32: hipLaunchKernelGGL(quantize_any_kernel<32>, grid, dim3(kQBlock), 0, st, a); break;
     case 64: hipLaunchKernelGGL(quantize_kernel<64>, grid, dim3(kQBlock), 0, st, a); break;
