@@ -51,7 +51,8 @@ namespace {
 
 constexpr float kPfRescale = 8.0f;
 constexpr int kRowPad = 64;    // q_rot rows per (sequence, kv head) are a multiple of this
-constexpr int kRotRows = 32;   // rows per work-group of the rotate and merge kernels
+constexpr int kRotRows = 32;   // rows of a tile of the rotate and merge kernels
+constexpr int kRotGroups = 768;  // their work-groups at most (three per CU)
 
 struct PrefillArgs {
   const float* q_rot;  // (B*Hkv*nrp, 128)
@@ -948,13 +949,17 @@ __global__ __launch_bounds__(64 * WPB) void pf_tile_kernel(PrefillArgs a) {
 
 // ---------------------------------------------------------------- rotate and merge
 //
-// Both are a kRotRows-row tile times a 128 x 128 rotation per work-group: the matrix
-// M^T ([j][k], 132-float rows) and the rows ([r][k], 132-float rows) in LDS, thread t
-// making rows RT (t >> 4) .. and columns (t & 15) + 16 jj, jj = 0..7, from 16-byte
-// reads along k (the 16 lanes of a column group read 16 different M^T rows whose 4-bank
-// spans do not overlap; lanes sharing rows read the same addresses).
-
-constexpr int kRotStride = 132;  // floats per LDS row (16-byte aligned, bank-skewed)
+// Both multiply rows by a D x D rotation on v_mfma_f32_16x16x4f32 (fp32 operands and
+// sums): y^T = M x^T with A = M, B = sixteen rows. Wave w of a row tile of kRotRows makes
+// output columns 32w .. 32w + 31 and keeps their part of M in registers (A operands, 64
+// at D = 128) over all the row tiles its work-group takes, so M is read from L2 once per
+// work-group and needs no LDS. K-step (s, e), slot k (= lane / 16) is column 16s + 4k + e
+// of x, so that a lane's operands are runs of four consecutive values of a row. Lane
+// 16g + c ends with columns 16t + 4g .. + 3 of row c.
+// Measured at 32,768 rows (2 sequences, 32 heads, 512 tokens, head_dim 128; traces), against
+// the vector-ALU products with M in LDS that they replace: rotate 56.8 -> 25.0 us, merge 32.1
+// -> 23.2 us; a whole call of 8 sequences of 100 tokens over 500 (6 bits) 126 -> 84 us. One,
+// two or three work-groups per CU: rotate 26.0 / 23.2 / 24.9, merge 30.9 / 24.8 / 23.7 us.
 
 struct PfRotArgs {
   const void* q;
@@ -962,66 +967,103 @@ struct PfRotArgs {
   const float* pi;
   float* q_rot;
   float scale;
+  int64_t tiles;  // row tiles: B Hkv nrp / kRotRows (fewer than 2^32 rows)
   int Hkv, n_rep, Q, nrp, q_dtype;
+  int vec;  // rows of q are aligned to four elements
 };
 
-// y[r][jj] = sum_k x[rb + r][k] mt[(t & 15) + 16 jj][k], rb = RT (t >> 4).
-constexpr int RT = kRotRows / 16;  // rows per thread
-__device__ __forceinline__ void rows_times_t(const float* x, const float* mt, int tid, float (&y)[RT][8]) {
-  const int rb = RT * (tid >> 4), jc = tid & 15;
+// Waves that share a row tile, row tiles a work-group of four waves takes at a time.
+template <int D>
+struct RotShape {
+  static constexpr int CW = D / 32, TW = 4 / CW, S = D / 16;
+};
+
+// acc[rt][t] += M x^T: columns 16t + 4g + i of row c of half rt of the tile.
+template <int S>
+__device__ __forceinline__ void rot_product(const f32x4 (&m)[2][S], const f32x4 (&x)[2][S], f32x4 (&acc)[2][2]) {
 #pragma unroll
-  for (int r = 0; r < RT; ++r)
+  for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) y[r][jj] = 0.f;
-#pragma unroll 2
-  for (int k = 0; k < 128; k += 4) {
-    float4 xv[RT], mv[8];
+    for (int t = 0; t < 2; ++t) acc[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int r = 0; r < RT; ++r) xv[r] = *reinterpret_cast<const float4*>(x + (rb + r) * kRotStride + k);
+  for (int s = 0; s < S; ++s)
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) mv[jj] = *reinterpret_cast<const float4*>(mt + (jc + 16 * jj) * kRotStride + k);
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
-    for (int r = 0; r < RT; ++r)
+      for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        y[r][jj] = fmaf(xv[r].x, mv[jj].x, y[r][jj]);
-        y[r][jj] = fmaf(xv[r].y, mv[jj].y, y[r][jj]);
-        y[r][jj] = fmaf(xv[r].z, mv[jj].z, y[r][jj]);
-        y[r][jj] = fmaf(xv[r].w, mv[jj].w, y[r][jj]);
-      }
-  }
+        for (int t = 0; t < 2; ++t)
+          acc[rt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(m[t][s][e], x[rt][s][e], acc[rt][t], 0, 0, 0);
 }
 
-// q_rot rows (sequence blockIdx.z, kv head blockIdx.y, rows kRotRows blockIdx.x ..):
-// scale * q Pi_K^T, zero for rows past n_rep Q. Pi_K is [j][k] already: its rows are
-// staged as they are, with coalesced 16-byte loads.
+// Four elements of a row of q.
+__device__ __forceinline__ f32x4 load_q4(const PfRotArgs& a, int64_t i) {
+  f32x4 v;
+  if (!a.vec) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = load_elem(a.q, i + k, a.q_dtype);
+  } else if (a.q_dtype == WN_F32) {
+    v = *reinterpret_cast<const f32x4*>(static_cast<const float*>(a.q) + i);
+  } else {
+    const uint2 w = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(a.q) + i);
+    const uint16_t h[4] = {uint16_t(w.x), uint16_t(w.x >> 16), uint16_t(w.y), uint16_t(w.y >> 16)};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = a.q_dtype == WN_BF16 ? bf16_to_f32(h[k]) : f16_to_f32(h[k]);
+  }
+  return v;
+}
+
+// Four consecutive elements of out, at a multiple of four (vec: out is aligned to four elements).
+__device__ __forceinline__ void store4(void* out, int64_t i, int dtype, bool vec, f32x4 v) {
+  if (!vec) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) store_elem(out, i + k, dtype, v[k]);
+    return;
+  }
+  if (dtype == WN_F32) {
+    *reinterpret_cast<f32x4*>(static_cast<float*>(out) + i) = v;
+    return;
+  }
+  uint16_t h[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) h[k] = dtype == WN_BF16 ? f32_to_bf16(v[k]) : f32_to_f16(v[k]);
+  *reinterpret_cast<uint2*>(static_cast<uint16_t*>(out) + i) =
+      make_uint2(uint32_t(h[0]) | uint32_t(h[1]) << 16, uint32_t(h[2]) | uint32_t(h[3]) << 16);
+}
+
+// q_rot = scale * q Pi_K^T, zero for rows past n_rep Q of a (sequence, kv head).
+template <int D>
 __global__ __launch_bounds__(256) void pf_rotate_kernel(PfRotArgs a) {
-  __shared__ __align__(16) float mt[128 * kRotStride];
-  __shared__ __align__(16) float x[kRotRows * kRotStride];
-  const int tid = threadIdx.x, kvh = blockIdx.y, b = blockIdx.z, r0 = blockIdx.x * kRotRows;
-  for_strided<128 * 32, 256>(tid, [&](int i) {
-    const int j = i >> 5, k4 = 4 * (i & 31);
-    *reinterpret_cast<float4*>(mt + j * kRotStride + k4) = reinterpret_cast<const float4*>(a.pi)[i];
-  });
+  using Sh = RotShape<D>;
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, w = threadIdx.x >> 6;
+  const int j0 = 32 * (w % Sh::CW);
+  f32x4 m[2][Sh::S];  // rows j of Pi_K
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int s = 0; s < Sh::S; ++s) m[t][s] = *reinterpret_cast<const f32x4*>(a.pi + (j0 + 16 * t + c) * D + 16 * s + 4 * g);
   const int rows = a.n_rep * a.Q;
-  for_strided<kRotRows * 128, 256>(tid, [&](int i) {
-    const int rr = i >> 7, k = i & 127, r = r0 + rr;
-    float v = 0.f;
-    if (r < rows) {
+  for (int64_t tile = int64_t(blockIdx.x) * Sh::TW + w / Sh::CW; tile < a.tiles; tile += int64_t(gridDim.x) * Sh::TW) {
+    const int64_t row0 = tile * kRotRows;
+    const uint32_t unit = uint32_t(row0) / uint32_t(a.nrp);  // kRotRows divides nrp
+    const int r0 = int(uint32_t(row0) % uint32_t(a.nrp)), kvh = int(unit % uint32_t(a.Hkv));
+    const int64_t b = unit / uint32_t(a.Hkv);
+    f32x4 x[2][Sh::S], acc[2][2];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      const int r = r0 + 16 * rt + c;
       const int qi = r / a.n_rep, h = kvh * a.n_rep + r % a.n_rep;
-      v = load_elem(a.q, b * a.qsb + h * a.qsh + qi * a.qsq + k, a.q_dtype);
+      const int64_t o = b * a.qsb + h * a.qsh + qi * a.qsq + 4 * g;
+#pragma unroll
+      for (int s = 0; s < Sh::S; ++s) x[rt][s] = r < rows ? load_q4(a, o + 16 * s) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    x[rr * kRotStride + k] = v;
-  });
-  __syncthreads();
-  float y[RT][8];
-  rows_times_t(x, mt, tid, y);
-  const int rb = RT * (tid >> 4), jc = tid & 15;
-  float* out = a.q_rot + ((int64_t(b) * a.Hkv + kvh) * a.nrp + r0) * 128;
+    rot_product<Sh::S>(m, x, acc);
 #pragma unroll
-  for (int r = 0; r < RT; ++r)
+    for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-    for (int jj = 0; jj < 8; ++jj) out[(rb + r) * 128 + jc + 16 * jj] = y[r][jj] * a.scale;
+      for (int t = 0; t < 2; ++t)
+        *reinterpret_cast<f32x4*>(a.q_rot + (row0 + 16 * rt + c) * D + j0 + 16 * t + 4 * g) = acc[rt][t] * a.scale;
+  }
 }
 
 struct PfMergeArgs {
@@ -1029,100 +1071,95 @@ struct PfMergeArgs {
   const float* part_ml;
   const float* pi_v;
   void* out;  // (B, Hq, Q, D) contiguous
+  int64_t tiles;  // row tiles: B Hkv nrp / kRotRows (fewer than 2^32 rows)
   int out_dtype, Hkv, n_rep, Q, nrp, ncb, nsplit, nr;  // nr: rows per column block
+  int vec;  // out is aligned to four elements
 };
 
-// y[r][j] = sum_k xt[k][rb + r] m[k][jb + j] for the kRotRows rows of a work-group:
-// xt = the rows transposed ([k][r]), m = M as it is stored ([k][j]); thread t makes
-// rows 4 (t / 32) .. +3 (RT2 of them) and columns 4 (t % 32) .. +3.
-constexpr int RT2 = kRotRows / 8;
-__device__ __forceinline__ void rows_times_n(const float* xt, const float* m, int tid, float (&y)[RT2][4]) {
-  const int rb = RT2 * (tid >> 5), jb = 4 * (tid & 31);
-#pragma unroll
-  for (int r = 0; r < RT2; ++r)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) y[r][j] = 0.f;
-#pragma unroll 4
-  for (int k = 0; k < 128; ++k) {
-    float xa[RT2];
-#pragma unroll
-    for (int r = 0; r < RT2; r += 4) {
-      const float4 xv = *reinterpret_cast<const float4*>(xt + k * kRotRows + rb + r);
-      xa[r] = xv.x;
-      xa[r + 1] = xv.y;
-      xa[r + 2] = xv.z;
-      xa[r + 3] = xv.w;
-    }
-    const float4 mv = *reinterpret_cast<const float4*>(m + k * 128 + jb);
-#pragma unroll
-    for (int r = 0; r < RT2; ++r) {
-      y[r][0] = fmaf(xa[r], mv.x, y[r][0]);
-      y[r][1] = fmaf(xa[r], mv.y, y[r][1]);
-      y[r][2] = fmaf(xa[r], mv.z, y[r][2]);
-      y[r][3] = fmaf(xa[r], mv.w, y[r][3]);
-    }
-  }
-}
-
-// Rows (sequence blockIdx.z, kv head blockIdx.y, rows kRotRows blockIdx.x ..): the
-// max-stable merge of each row's split partials (weights 2^(m_s - max m)), 1 / l,
-// then Pi_V ([k][j], staged as stored) and the cast; rows that saw no key are 0
-// (packed_attention.py:206). The splits' maxima are read in one pass and their
-// weighted rows in a second, so neither pass chains a load behind another.
+// The max-stable merge of each row's split partials (weights 2^(m_s - max m)), 1 / l,
+// then Pi_V and the cast; rows that saw no key are 0 (packed_attention.py:206). All
+// threads merge a row tile into LDS, then its waves multiply. The splits' maxima are
+// read in one pass and their weighted rows in a second, so neither pass chains a load
+// behind another.
+template <int D>
 __global__ __launch_bounds__(256) void pf_merge_kernel(PfMergeArgs a) {
-  __shared__ __align__(16) float pv[128 * 128];
-  __shared__ __align__(16) float xt[128 * kRotRows];
-  const int tid = threadIdx.x, kvh = blockIdx.y, b = blockIdx.z, r0 = blockIdx.x * kRotRows;
-  for_strided<128 * 128 / 4, 256>(
-      tid, [&](int i) { reinterpret_cast<float4*>(pv)[i] = reinterpret_cast<const float4*>(a.pi_v)[i]; });
-  {
-    // thread: row rr = tid / TPR, dims DPT (tid % TPR) .. (TPR threads per row)
-    constexpr int TPR = 256 / kRotRows, DPT = 128 / TPR;
-    const int rr = tid / TPR, d0 = DPT * (tid % TPR), r = r0 + rr;
-    const int cb = r / a.nr, ri = r % a.nr;
-    const int64_t row0 = (((int64_t(b) * a.Hkv + kvh) * a.nsplit) * a.ncb + cb) * a.nr + ri;
-    const int64_t srow = int64_t(a.ncb) * a.nr;  // rows between a row's consecutive splits
-    float M = -INFINITY;
+  using Sh = RotShape<D>;
+  constexpr int NR = kRotRows * Sh::TW, STRIDE = D + 4;  // rows at a time; floats per LDS row (bank-skewed)
+  __shared__ __align__(16) float xt[NR * STRIDE];
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15, w = tid >> 6;
+  const int j0 = 32 * (w % Sh::CW);
+  f32x4 m[2][Sh::S];  // columns j of Pi_V ([k][j])
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int s = 0; s < Sh::S; ++s)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m[t][s][e] = a.pi_v[(16 * s + 4 * g + e) * D + j0 + 16 * t + c];
+  const int rows = a.n_rep * a.Q, Hq = a.Hkv * a.n_rep;
+  for (int64_t tile0 = int64_t(blockIdx.x) * Sh::TW; tile0 < a.tiles; tile0 += int64_t(gridDim.x) * Sh::TW) {
+    {
+      // thread: row rr, dims DPT (tid % TPR) .. (TPR threads per row)
+      constexpr int TPR = 256 / NR, DPT = D / TPR;
+      const int rr = tid / TPR, d0 = DPT * (tid % TPR);
+      const int64_t row = tile0 * kRotRows + rr;
+      float den = 0.f, num[DPT];
+#pragma unroll
+      for (int k = 0; k < DPT; ++k) num[k] = 0.f;
+      if (row < a.tiles * kRotRows) {
+        const uint32_t unit = uint32_t(row) / uint32_t(a.nrp);
+        const int r = int(uint32_t(row) % uint32_t(a.nrp));
+        const int64_t part = (int64_t(unit) * a.nsplit * a.ncb + r / a.nr) * a.nr + r % a.nr;
+        const int64_t step = int64_t(a.ncb) * a.nr;  // rows between a row's consecutive splits
+        float M = -INFINITY;
 #pragma unroll 8
-    for (int s = 0; s < a.nsplit; ++s) M = fmaxf(M, a.part_ml[2 * (row0 + s * srow)]);
-    float den = 0.f, num[DPT];
-#pragma unroll
-    for (int k = 0; k < DPT; ++k) num[k] = 0.f;
-    if (M != -INFINITY) {
+        for (int s = 0; s < a.nsplit; ++s) M = fmaxf(M, a.part_ml[2 * (part + s * step)]);
+        if (M != -INFINITY) {
 #pragma unroll 4
-      for (int s = 0; s < a.nsplit; ++s) {
-        const int64_t row = row0 + s * srow;
-        const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * row);
-        const float w = __builtin_amdgcn_exp2f(ml.x - M);  // 0 for a split without keys (m = -inf)
-        den = fmaf(w, ml.y, den);
-        const float4* src = reinterpret_cast<const float4*>(a.part_acc + row * 128 + d0);
+          for (int s = 0; s < a.nsplit; ++s) {
+            const int64_t pr = part + s * step;
+            const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * pr);
+            const float wt = __builtin_amdgcn_exp2f(ml.x - M);  // 0 for a split without keys (m = -inf)
+            den = fmaf(wt, ml.y, den);
+            const float4* src = reinterpret_cast<const float4*>(a.part_acc + pr * D + d0);
 #pragma unroll
-        for (int k = 0; k < DPT / 4; ++k) {
-          const float4 v = src[k];
-          num[4 * k] = fmaf(w, v.x, num[4 * k]);
-          num[4 * k + 1] = fmaf(w, v.y, num[4 * k + 1]);
-          num[4 * k + 2] = fmaf(w, v.z, num[4 * k + 2]);
-          num[4 * k + 3] = fmaf(w, v.w, num[4 * k + 3]);
+            for (int k = 0; k < DPT / 4; ++k) {
+              const float4 v = src[k];
+              num[4 * k] = fmaf(wt, v.x, num[4 * k]);
+              num[4 * k + 1] = fmaf(wt, v.y, num[4 * k + 1]);
+              num[4 * k + 2] = fmaf(wt, v.z, num[4 * k + 2]);
+              num[4 * k + 3] = fmaf(wt, v.w, num[4 * k + 3]);
+            }
+          }
         }
       }
+      const float inv = den > 0.f ? 1.f / den : 0.f;
+#pragma unroll
+      for (int k = 0; k < DPT; k += 4)
+        *reinterpret_cast<f32x4*>(xt + rr * STRIDE + d0 + k) = f32x4{num[k], num[k + 1], num[k + 2], num[k + 3]} * inv;
     }
-    const float inv = den > 0.f ? 1.f / den : 0.f;
+    __syncthreads();
+    const int64_t tile = tile0 + w / Sh::CW;
+    if (tile < a.tiles) {
+      f32x4 x[2][Sh::S], acc[2][2];
 #pragma unroll
-    for (int k = 0; k < DPT; ++k) xt[(d0 + k) * kRotRows + rr] = num[k] * inv;
-  }
-  __syncthreads();
-  float y[RT2][4];
-  rows_times_n(xt, pv, tid, y);
-  const int rb = RT2 * (tid >> 5), jb = 4 * (tid & 31);
-  const int rows = a.n_rep * a.Q, Hq = a.Hkv * a.n_rep;
+      for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-  for (int r = 0; r < RT2; ++r) {
-    const int rg = r0 + rb + r;
-    if (rg >= rows) continue;
-    const int qi = rg / a.n_rep, h = kvh * a.n_rep + rg % a.n_rep;
-    const int64_t o = ((int64_t(b) * Hq + h) * a.Q + qi) * 128 + jb;
+        for (int s = 0; s < Sh::S; ++s)
+          x[rt][s] = *reinterpret_cast<const f32x4*>(xt + ((w / Sh::CW) * kRotRows + 16 * rt + c) * STRIDE + 16 * s + 4 * g);
+      rot_product<Sh::S>(m, x, acc);
+      const uint32_t row0 = uint32_t(tile * kRotRows), unit = row0 / uint32_t(a.nrp);
+      const int kvh = int(unit % uint32_t(a.Hkv));
+      const int64_t b = unit / uint32_t(a.Hkv);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) store_elem(a.out, o + j, a.out_dtype, y[r][j]);
+      for (int rt = 0; rt < 2; ++rt) {
+        const int r = int(row0 % uint32_t(a.nrp)) + 16 * rt + c;
+        if (r >= rows) continue;
+        const int qi = r / a.n_rep, h = kvh * a.n_rep + r % a.n_rep;
+#pragma unroll
+        for (int t = 0; t < 2; ++t) store4(a.out, ((b * Hq + h) * a.Q + qi) * D + j0 + 16 * t + 4 * g, a.out_dtype, a.vec, acc[rt][t]);
+      }
+    }
+    __syncthreads();  // the tile is read; the next one may overwrite it
   }
 }
 
@@ -1276,9 +1313,15 @@ extern "C" int wn_prefill_attention(
   const int nrp = pf_nrp(n_rep, Q);
   const int nr = 16 * k.nct, ncb = nrp / nr;
 
+  const int64_t tiles = int64_t(B) * Hkv * (nrp / kRotRows);
+  const int q4 = q_dtype == WN_F32 ? 16 : 8, o4 = out_dtype == WN_F32 ? 16 : 8;  // bytes of four elements
+  const bool qvec = aligned(q, q4) && q_stride_b % 4 == 0 && q_stride_h % 4 == 0 && q_stride_q % 4 == 0;
+  WN_REQUIRE(tiles * kRotRows < (int64_t(1) << 32), WN_E_INVALID, "prefill: too many query rows");
   PfRotArgs ra{q, q_stride_b, q_stride_h, q_stride_q, pi_k, reinterpret_cast<float*>(ws + lay.qrot),
-               float(double(scale) * 1.4426950408889634), Hkv, n_rep, Q, nrp, q_dtype};
-  hipLaunchKernelGGL(pf_rotate_kernel, dim3(nrp / kRotRows, Hkv, B), dim3(256), 0, st, ra);
+               float(double(scale) * 1.4426950408889634), tiles, Hkv, n_rep, Q, nrp, q_dtype, qvec};
+  // work-groups that take a few row tiles each: Pi is read once per work-group
+  const unsigned rot_groups = unsigned(std::min<int64_t>(tiles, kRotGroups));
+  hipLaunchKernelGGL(pf_rotate_kernel<128>, dim3(rot_groups), dim3(256), 0, st, ra);
 
   PrefillArgs pa;
   pa.q_rot = ra.q_rot;
@@ -1318,7 +1361,8 @@ extern "C" int wn_prefill_attention(
   else hipLaunchKernelGGL(k.fn, dim3(unsigned(groups)), dim3(64 * k.wpb), 0, st, pa);
   if (ev_end) hipEventRecord(static_cast<hipEvent_t>(ev_end), st);
 
-  PfMergeArgs ma{pa.part_acc, pa.part_ml, pi_v, out, out_dtype, Hkv, n_rep, Q, nrp, ncb, num_splits, nr};
-  hipLaunchKernelGGL(pf_merge_kernel, dim3(nrp / kRotRows, Hkv, B), dim3(256), 0, st, ma);
+  PfMergeArgs ma{pa.part_acc, pa.part_ml, pi_v, out, tiles, out_dtype, Hkv, n_rep, Q, nrp, ncb, num_splits, nr,
+                 aligned(out, o4)};
+  hipLaunchKernelGGL(pf_merge_kernel<128>, dim3(rot_groups), dim3(256), 0, st, ma);
   return check_launch("wn_prefill_attention");
 }
