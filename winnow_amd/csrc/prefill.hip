@@ -1229,6 +1229,41 @@ int resident_groups_pf(PfScanFn fn, int wpb) {
 // The shared-tile scan serves shapes with at least tile_wpb query blocks per kv head.
 bool use_tile(const PfKernel& k, int n_rep, int Q) { return pf_nrp(n_rep, Q) / (16 * k.nct) >= k.tile_wpb; }
 
+// The per-wave scan takes about two work-groups per resident slot over the (sequence, kv
+// head, column block) units, each split keeping at least four chunks of the longest
+// history. A shared-tile split is chosen by what it costs, in chunks of one work-group:
+// the rounds of work-groups over the w slots, times a split's chunks and the six that
+// staging its tables takes; a tenth of one round more for the spread of their ends (the
+// last round's only: several rounds even it out); and the partials, written and read
+// once per split (256 rows of 512 bytes per unit at 5 TB/s against 2.9 us a chunk).
+// Measured (us per call, 4 / 4 bits, 32 / 8 heads; two work-groups per slot -> this): 512
+// tokens over 9,000 176 -> 158, 4 x 128 over 4,000 119 -> 100, 300 (28 / 4 heads) over
+// 2,000 77 -> 67; 2 x 512 over 32,768 stays at four splits (831; two: 868).
+int pf_plan(const PfKernel& k, const char* what, int B, int Hq, int Hkv, int Q, int max_len, int* num_splits) {
+  const bool tile = use_tile(k, Hq / Hkv, Q);
+  const int wpb = tile ? k.tile_wpb : k.wpb;
+  const int w = resident_groups_pf(tile ? k.tile : k.fn, wpb);
+  WN_REQUIRE(w > 0, WN_E_LAUNCH, "%s: cannot query the device occupancy", what);
+  const int ncb = pf_nrp(Hq / Hkv, Q) / (16 * k.nct);
+  const int64_t units = int64_t(B > 0 ? B : 1) * Hkv * (tile ? (ncb + wpb - 1) / wpb : ncb);
+  const int64_t chunks = (int64_t(max_len) + 63) / 64;
+  const int64_t most = std::max<int64_t>(1, std::min<int64_t>(256, chunks / 4));
+  if (!tile) {
+    *num_splits = int(std::min<int64_t>((2 * int64_t(w) * wpb + units - 1) / units, most));
+    return WN_OK;
+  }
+  double best = 0.0;
+  for (int64_t ns = 1; ns <= most; ++ns) {
+    const int64_t rounds = (units * ns + w - 1) / w;
+    const double cost = (double(rounds) + 0.1) * double((chunks + ns - 1) / ns + 6) + 0.018 * double(units * ns);
+    if (ns == 1 || cost < best) {
+      best = cost;
+      *num_splits = int(ns);
+    }
+  }
+  return WN_OK;
+}
+
 }  // namespace
 }  // namespace wn
 
@@ -1241,20 +1276,7 @@ extern "C" int wn_prefill_plan(int B, int Hq, int Hkv, int Q, int D, int S, int 
   const PfKernel k = pick_prefill(bw_k, bw_v);
   WN_REQUIRE(D == 128 && S >= 16 && is_pow2(S) && k.fn, WN_E_UNSUPPORTED,
              "wn_prefill_plan: (D=%d, S=%d, bw_k=%d, bw_v=%d) not compiled", D, S, bw_k, bw_v);
-  // about two work-groups per resident slot over the (sequence, kv head, column block
-  // or group of blocks) units, each split keeping at least four chunks of the longest
-  // history
-  const bool tile = use_tile(k, Hq / Hkv, Q);
-  const int wpb = tile ? k.tile_wpb : k.wpb;
-  const int w = resident_groups_pf(tile ? k.tile : k.fn, wpb);
-  WN_REQUIRE(w > 0, WN_E_LAUNCH, "wn_prefill_plan: cannot query the device occupancy");
-  const int ncb = pf_nrp(Hq / Hkv, Q) / (16 * k.nct);
-  const int64_t units = int64_t(B > 0 ? B : 1) * Hkv * (tile ? (ncb + wpb - 1) / wpb : ncb);
-  int64_t ns = (2 * int64_t(tile ? w : w * wpb) + units - 1) / units;
-  const int64_t chunks = (int64_t(max_len) + 63) / 64;
-  ns = std::min<int64_t>(ns, std::max<int64_t>(1, chunks / 4));
-  *num_splits = int(std::max<int64_t>(1, std::min<int64_t>(ns, 256)));
-  return WN_OK;
+  return pf_plan(k, "wn_prefill_plan", B, Hq, Hkv, Q, max_len, num_splits);
 }
 
 extern "C" int64_t wn_prefill_workspace_bytes(int B, int Hq, int Hkv, int Q, int D, int num_splits) {
