@@ -305,6 +305,32 @@ int wn_prefill_attention(
     float scale, int num_splits,
     void* stream, void* ev_begin, void* ev_end);
 
+/* The histories of a batch at once: row (b, h, t) of out (B, Hkv, Lpad, D) contiguous is
+ * wn_dequantize_history's row (h, t) of sequence b, whose pages row b of page_table (row
+ * stride table_stride_b) names. Rows past seq_lens[b] repeat the sequence's last one (an
+ * empty sequence's: any). B * Hkv * Lpad < 2^31; other limits as wn_dequantize_history. */
+int wn_dequantize_histories(const uint8_t* pages, int64_t page_stride, int64_t head_stride,
+                            const uint16_t* norms, int64_t norm_page_stride, int64_t norm_head_stride,
+                            const int32_t* page_table, int64_t table_stride_b, const int32_t* seq_lens,
+                            int B, int Lpad, int Hkv, int S, const float* centroids, const float* pi, int bw,
+                            int D, void* out, int out_dtype, int fast, void* stream);
+
+/* Attention of q over reconstructed histories, the SDPA of _reconstruct_sdpa
+ * (packed_backend.py:211-226): query i of sequence b attends to keys j <= L - Q + i of
+ * the first L = seq_lens[b] rows of k and v; a query that sees none gives 0.
+ *   q     (B, Hq, Q, D), WN_BF16 or WN_F16, element strides multiples of 8
+ *   k, v  (B, Hkv, Lpad, D) contiguous, q's type; rows past seq_lens[b] are not read
+ *   out   (B, Q, Hq, D) contiguous, q's type
+ * Exact 16-bit operands, fp32 scores and softmax, probabilities as pairs of 16-bit values.
+ * D 64 or 128; all operands 16-byte aligned, the workspace (wn_history_workspace_bytes)
+ * 256. num_splits from wn_history_plan (any value 1..4096 is valid). */
+int wn_history_plan(int B, int Hq, int Hkv, int Q, int D, int dtype, int max_len, int* num_splits);
+int64_t wn_history_workspace_bytes(int B, int Hq, int Hkv, int Q, int D, int num_splits);
+int wn_history_attention(const void* q, int dtype, int64_t q_stride_b, int64_t q_stride_h, int64_t q_stride_q,
+                         const void* k, const void* v, const int32_t* seq_lens, void* out, void* workspace,
+                         int64_t workspace_bytes, int B, int Hq, int Hkv, int Q, int D, int64_t Lpad,
+                         float scale, int num_splits, void* stream);
+
 /* Plan of wn_dense_decode_attention (as wn_decode_plan: requested_splits > 0 gives
  * the reference's cdiv split of max_pages; 0 lets the library choose: a balanced
  * plan of persistent waves, pages_per_split = 0, for WN_BF16 and WN_F16 pages, fixed

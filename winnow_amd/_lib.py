@@ -103,6 +103,20 @@ SIGNATURES = {
         _c_p, _c_i, _c_i, _c_i,                     # table row, L, Hkv, S
         _c_p, _c_p, _c_i, _c_i,                     # centroids, Pi, bw, D
         _c_p, _c_i, _c_i, _c_p]),                   # out, out dtype, fast, stream
+    "wn_dequantize_histories": (_c_i, [
+        _c_p, _c_i64, _c_i64,                       # pages, page stride, head stride
+        _c_p, _c_i64, _c_i64,                       # norms, page stride, head stride
+        _c_p, _c_i64, _c_p,                         # table, stride, seq_lens
+        _c_i, _c_i, _c_i, _c_i,                     # B, Lpad, Hkv, S
+        _c_p, _c_p, _c_i, _c_i,                     # centroids, Pi, bw, D
+        _c_p, _c_i, _c_i, _c_p]),                   # out, out dtype, fast, stream
+    "wn_history_plan": (_c_i, [_c_i, _c_i, _c_i, _c_i, _c_i, _c_i, _c_i, ctypes.POINTER(_c_i)]),
+    "wn_history_workspace_bytes": (_c_i64, [_c_i, _c_i, _c_i, _c_i, _c_i, _c_i]),
+    "wn_history_attention": (_c_i, [
+        _c_p, _c_i, _c_i64, _c_i64, _c_i64,         # q, dtype, strides (b, h, q)
+        _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64,       # k, v, seq_lens, out, workspace, bytes
+        _c_i, _c_i, _c_i, _c_i, _c_i, _c_i64,       # B Hq Hkv Q D Lpad
+        _c_f, _c_i, _c_p]),                         # scale, num_splits, stream
     "wn_prefill_plan": (_c_i, [_c_i, _c_i, _c_i, _c_i, _c_i, _c_i, _c_i, _c_i, _c_i, ctypes.POINTER(_c_i)]),
     "wn_prefill_workspace_bytes": (_c_i64, [_c_i, _c_i, _c_i, _c_i, _c_i, _c_i]),
     "wn_prefill_attention": (_c_i, [

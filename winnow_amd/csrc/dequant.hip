@@ -64,6 +64,11 @@ struct DqArgs {
   int log2S;
   int64_t psp, psh;       // paged: packed page / plane strides, bytes
   int64_t nsp, nsh;       // paged: norm page / plane strides, elements
+  // paged, several sequences (lens not null): plane = sequence Hkv + head, the table row of
+  // a sequence tsb entries from the last one's; positions past a length repeat its last row
+  const int32_t* lens;
+  int64_t tsb;
+  uint32_t Hkv;
 };
 
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
@@ -86,11 +91,21 @@ __device__ __forceinline__ void row_pos(const DqArgs& a, int64_t r, uint32_t& pl
   t = r32 - plane * uint32_t(a.L);
 }
 
-// Paged mode: the page holding row r.
+// Paged mode: head and position of row r, and its sequence's table row.
+__device__ __forceinline__ const int32_t* row_paged(const DqArgs& a, int64_t r, uint32_t& plane, uint32_t& t) {
+  row_pos(a, r, plane, t);
+  if (!a.lens) return a.table;
+  const uint32_t b = plane / a.Hkv;
+  plane -= b * a.Hkv;
+  t = min(t, uint32_t(max(a.lens[b], 1) - 1));
+  return a.table + b * a.tsb;
+}
+
+// Paged mode: the page holding row r (an empty sequence's first entry may be -1: page 0).
 __device__ __forceinline__ int32_t row_page(const DqArgs& a, int64_t r) {
   uint32_t plane, t;
-  row_pos(a, r, plane, t);
-  return a.table[t >> a.log2S];
+  const int32_t* trow = row_paged(a, r, plane, t);
+  return max(trow[t >> a.log2S], 0);
 }
 
 // Codes and norm of row r; in paged mode `page` is row_page(a, r).
@@ -98,12 +113,13 @@ template <int NB, bool PAGED>
 __device__ __forceinline__ void row_src(const DqArgs& a, int64_t r, int32_t page, const uint8_t*& p,
                                         const uint16_t*& n) {
   uint32_t plane, t;
-  row_pos(a, r, plane, t);
   if constexpr (PAGED) {
+    row_paged(a, r, plane, t);
     const int64_t slot = t & ((1u << a.log2S) - 1u);
     p = a.packed + page * a.psp + plane * a.psh + slot * NB;
     n = a.norms + page * a.nsp + plane * a.nsh + slot;
   } else {
+    row_pos(a, r, plane, t);
     const int64_t src = int64_t(plane) * a.plane_rows + t;
     p = a.packed + src * NB;
     n = a.norms + src;
@@ -543,4 +559,41 @@ extern "C" int wn_dequantize_history(const uint8_t* pages, int64_t page_stride, 
   a.nsp = norm_page_stride;
   a.nsh = norm_head_stride;
   return launch_dq(a, bw, fast, out_dtype, static_cast<hipStream_t>(stream), "wn_dequantize_history");
+}
+
+extern "C" int wn_dequantize_histories(const uint8_t* pages, int64_t page_stride, int64_t head_stride,
+                                       const uint16_t* norms, int64_t norm_page_stride, int64_t norm_head_stride,
+                                       const int32_t* page_table, int64_t table_stride_b, const int32_t* seq_lens,
+                                       int B, int Lpad, int Hkv, int S, const float* centroids, const float* pi, int bw,
+                                       int D, void* out, int out_dtype, int fast, void* stream) {
+  clear_error();
+  WN_REQUIRE(D == kDqD, WN_E_UNSUPPORTED, "wn_dequantize_histories: head_dim %d (128 only)", D);
+  WN_REQUIRE(B >= 0 && Lpad >= 0 && Hkv > 0 && S > 0 && (S & (S - 1)) == 0, WN_E_INVALID,
+             "wn_dequantize_histories: bad sizes B=%d Lpad=%d Hkv=%d S=%d", B, Lpad, Hkv, S);
+  WN_REQUIRE(out_dtype == WN_F32 || out_dtype == WN_BF16 || out_dtype == WN_F16, WN_E_INVALID,
+             "wn_dequantize_histories: output dtype %d", out_dtype);
+  if (B == 0 || Lpad == 0) return WN_OK;
+  WN_REQUIRE(pages && norms && page_table && seq_lens && centroids && pi && out, WN_E_INVALID,
+             "wn_dequantize_histories: null pointer");
+  WN_REQUIRE(aligned(pages, 16) && page_stride % 16 == 0 && head_stride % 16 == 0 && aligned(out, 16), WN_E_INVALID,
+             "wn_dequantize_histories: pages, their strides and out must be 16-byte aligned");
+  DqArgs a{};
+  a.packed = pages;
+  a.norms = norms;
+  a.pi = pi;
+  a.cb = centroids;
+  a.out = out;
+  a.N = int64_t(B) * Hkv * Lpad;
+  a.L = Lpad;
+  a.plane_rows = Lpad;
+  a.table = page_table;
+  a.log2S = ilog2(S);
+  a.psp = page_stride;
+  a.psh = head_stride;
+  a.nsp = norm_page_stride;
+  a.nsh = norm_head_stride;
+  a.lens = seq_lens;
+  a.tsb = table_stride_b;
+  a.Hkv = uint32_t(Hkv);
+  return launch_dq(a, bw, fast, out_dtype, static_cast<hipStream_t>(stream), "wn_dequantize_histories");
 }

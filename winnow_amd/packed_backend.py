@@ -458,16 +458,80 @@ def _padded_sdpa(query, k, v, lens, scaling):
     return torch.where(live, out, torch.zeros((), dtype=out.dtype, device=out.device))
 
 
+def _plain(t: torch.Tensor) -> bool:
+    """A tensor whose values are all that is wanted of it: no gradient, tangent, batching
+    transform or trace passes through the operator that reads it."""
+    return (type(t) is torch.Tensor and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and torch.autograd.forward_ad.unpack_dual(t).tangent is None and not torch.compiler.is_compiling())
+
+
+def _history_kernel(query, kv: pa.PackedKV, Lmax: int) -> bool:
+    """Whether ``wn_history_attention`` serves the SDPA of a reconstruct step: a 16-bit
+    query at head_dim 64 or 128 on the handle's device, only its values wanted (the
+    library's operator serves gradients, tangents and traces), sizes within its limits."""
+    if query.dtype not in (torch.bfloat16, torch.float16) or query.dim() != 4 or not _plain(query):
+        return False
+    B, Hq, Q, D = query.shape
+    Hkv, lens = kv.num_kv_heads, kv.seq_lens
+    return (D in (64, 128) and kv.head_dim == D and _lib.is_hip(query) and Hq % Hkv == 0 and Q > 0
+            and query.device == kv.k_pages.device == lens.device and lens.dtype == torch.int32 and lens.shape == (B,)
+            and lens.is_contiguous() and kv.page_table.dtype == torch.int32 and kv.page_table.stride(-1) == 1
+            and Hq // Hkv * Q <= 1 << 24 and B * Hkv * Lmax < 1 << 31)
+
+
+def _histories(kv: pa.PackedKV, pages, norms, quant, lens, Lmax: int, dtype) -> torch.Tensor:
+    """(B, Hkv, Lmax, D) histories of the batch; what lies past a length is not meant to be
+    read. head_dim 128 with contiguous rows: one launch; else sequence by sequence."""
+    B, S, D, Hkv = lens.shape[0], kv.page_size, kv.head_dim, kv.num_kv_heads
+    buf = torch.empty(B, Hkv, Lmax, D, dtype=dtype, device=pages.device)
+    if D == 128 and pages.stride(-1) == 1 and pages.stride(-2) == pages.shape[-1] and norms.stride(-1) == 1:
+        with torch.cuda.device(pages.device):
+            _lib.call("wn_dequantize_histories", _lib.ptr(pages), pages.stride(0), pages.stride(1), _lib.ptr(norms),
+                      norms.stride(0), norms.stride(1), _lib.ptr(kv.page_table), kv.page_table.stride(0),
+                      _lib.ptr(kv.seq_lens), B, Lmax, Hkv, S, _lib.ptr(quant.centroids), _lib.ptr(quant.Pi),
+                      quant.bit_width, D, _lib.ptr(buf), _lib.DTYPE_CODE[dtype], 0, _lib.stream_of(pages.device))
+        return buf
+    for b in range(B):
+        if lens[b]:
+            buf[b, :, :int(lens[b])] = dequantize_history(kv, pages, norms, quant, b, dtype)[0]
+    return buf
+
+
+def _history_attention(query, kv: pa.PackedKV, k, v, Lmax: int, scaling):
+    """The offset-causal SDPA of ``_padded_sdpa`` in one HIP operator, as a (B, Hq, Q, D)
+    view of (B, Q, Hq, D) memory, the order in which the model's attention returns it."""
+    B, Hq, Q, D = query.shape
+    Hkv, code = kv.num_kv_heads, _lib.DTYPE_CODE[query.dtype]
+    if query.stride(-1) != 1 or query.data_ptr() % 16 or any(s % 8 for s in query.stride()[:3]):
+        query = query.clone(memory_format=torch.contiguous_format)
+    out = torch.empty(B, Q, Hq, D, dtype=query.dtype, device=query.device)
+    ns = ctypes.c_int(0)
+    with torch.cuda.device(query.device):
+        _lib.call("wn_history_plan", B, Hq, Hkv, Q, D, code, Lmax, ctypes.byref(ns))
+        ws = torch.empty(int(_lib.lib().wn_history_workspace_bytes(B, Hq, Hkv, Q, D, ns.value)), dtype=torch.uint8,
+                         device=query.device)
+        _lib.call("wn_history_attention", _lib.ptr(query), code, query.stride(0), query.stride(1), query.stride(2),
+                  _lib.ptr(k), _lib.ptr(v), _lib.ptr(kv.seq_lens), _lib.ptr(out), _lib.ptr(ws), ws.numel(),
+                  B, Hq, Hkv, Q, D, Lmax, float(scaling), ns.value, _lib.stream_of(query.device))
+    return out.transpose(1, 2)
+
+
 def _reconstruct_sdpa(query, kv: pa.PackedKV, scaling):
     """Dequantize every sequence's history on the GPU into one padded (B, Hkv, Lmax, D)
-    pair, then one offset-causal SDPA over the batch (packed_backend.py:211-226)."""
+    pair, then one offset-causal SDPA over the batch (packed_backend.py:211-226): the HIP
+    operator for 16-bit queries (``_history_kernel``), else the library's."""
     B, Hq, Q, D = query.shape
     lens = _host_lens(kv).to(torch.int64)
     Lmax = int(lens.max()) if B else 0
     if Lmax == 0:
         return torch.zeros(B, Hq, Q, D, dtype=query.dtype, device=query.device)
+    sides = ((kv.k_pages, kv.k_norms, kv.k_quant), (kv.v_pages, kv.v_norms, kv.v_quant))
+    if _history_kernel(query, kv, Lmax):
+        k, v = (_histories(kv, *side, lens, Lmax, query.dtype) for side in sides)
+        return _history_attention(query, kv, k, v, Lmax, scaling)
     hist = []
-    for pages, norms, quant in ((kv.k_pages, kv.k_norms, kv.k_quant), (kv.v_pages, kv.v_norms, kv.v_quant)):
+    for pages, norms, quant in sides:
         buf = torch.zeros(B, kv.num_kv_heads, Lmax, D, dtype=query.dtype, device=query.device)
         for b in range(B):
             if lens[b]:
