@@ -230,6 +230,39 @@ int wn_dequantize(const uint8_t* codes, const uint16_t* norms, int64_t rows,
                   const float* pi, const float* centroids, int bw, int D,
                   void* out, int out_dtype, void* stream);
 
+/* Append to a contiguous packed cache with outlier channels (cache.py:205-219): K and V
+ * (B, H, n, D) quantized as two channel groups each and written at positions pos ..
+ * pos + n - 1 of rows (B, H, capacity). channel_group (D bytes): 1 for the count2 outlier
+ * channels. m (D, D): both rotations, rows in code order (the D - count2 regular ones
+ * first), columns in channel order, zero between the groups. Codes (B, H, capacity, NB)
+ * and fp16 norms (B, H, capacity) per side and group, contiguous. Codes and norms are
+ * wn_quantize's of each group. D 64 or 128; K/V rows 16-byte aligned. */
+int wn_append_split(
+    const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_n, const void* v, int64_t vs_b, int64_t vs_h, int64_t vs_n,
+    int x_dtype, const float* m, const uint8_t* channel_group, int count2, const float* boundaries, int bw,
+    const float* boundaries2, int bw2, uint8_t* k_codes, uint8_t* v_codes, uint16_t* k_norms, uint16_t* v_norms,
+    uint8_t* k_codes2, uint8_t* v_codes2, uint16_t* k_norms2, uint16_t* v_norms2, int B, int H, int n, int D,
+    int64_t capacity, int64_t pos, void* stream);
+
+/* wn_dequantize's accuracy over packed rows, K and V (v_* null: K only) in one launch,
+ * addressed as wn_tq_dequant's. count2 > 0: two channel groups, m and channel_group as
+ * for wn_append_split; count2 = 0: m is the rotation, the *2 operands and channel_group
+ * null. Any D from 1 to 256 whose rows are whole bytes. */
+int wn_dequantize_rows(const uint8_t* k_codes, const uint8_t* v_codes, const uint16_t* k_norms,
+                       const uint16_t* v_norms, int bw, const float* centroids, const uint8_t* k_codes2,
+                       const uint8_t* v_codes2, const uint16_t* k_norms2, const uint16_t* v_norms2, int bw2,
+                       const float* centroids2, int count2, const float* m, const uint8_t* channel_group,
+                       int64_t planes, int64_t L, int64_t plane_rows, int D, void* k_out, void* v_out,
+                       int out_dtype, void* stream);
+
+/* wn_dequantize_histories at wn_dequantize's accuracy and any D from 1 to 256 (rows of
+ * whole bytes, no alignment asked of pages). seq_lens null: every sequence has Lpad. */
+int wn_dequantize_pages(const uint8_t* pages, int64_t page_stride, int64_t head_stride, const uint16_t* norms,
+                        int64_t norm_page_stride, int64_t norm_head_stride, const int32_t* page_table,
+                        int64_t table_stride_b, const int32_t* seq_lens, int B, int Lpad, int Hkv, int S,
+                        const float* centroids, const float* pi, int bw, int D, void* out, int out_dtype,
+                        void* stream);
+
 /* Fused dequantization of packed rows, unpack + codebook gather + inverse rotation
  * + norm rescale in one pass (replaces tq_dequant, turboquant_kv/kernel.py:78-115,
  * and tq_dequant_cuda, csrc/tq_dequant.cu:186-215). planes x L rows: row (p, t)

@@ -103,6 +103,26 @@ SIGNATURES = {
         _c_p, _c_i, _c_i, _c_i,                     # table row, L, Hkv, S
         _c_p, _c_p, _c_i, _c_i,                     # centroids, Pi, bw, D
         _c_p, _c_i, _c_i, _c_p]),                   # out, out dtype, fast, stream
+    "wn_append_split": (_c_i, [
+        _c_p, _c_i64, _c_i64, _c_i64,               # k, strides
+        _c_p, _c_i64, _c_i64, _c_i64, _c_i,         # v, strides, dtype
+        _c_p, _c_p, _c_i, _c_p, _c_i, _c_p, _c_i,   # m, channel_group, count2, boundaries, bw, boundaries2, bw2
+        _c_p, _c_p, _c_p, _c_p,                     # codes and norms of group 0
+        _c_p, _c_p, _c_p, _c_p,                     # of the outliers
+        _c_i, _c_i, _c_i, _c_i, _c_i64, _c_i64,     # B, H, n, D, capacity, pos
+        _c_p]),
+    "wn_dequantize_rows": (_c_i, [
+        _c_p, _c_p, _c_p, _c_p, _c_i, _c_p,         # codes, norms, bw, centroids of group 0
+        _c_p, _c_p, _c_p, _c_p, _c_i, _c_p, _c_i,   # of the outliers, their count
+        _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i,   # m, channel_group, planes, L, plane_rows, D
+        _c_p, _c_p, _c_i, _c_p]),                   # outs, dtype, stream
+    "wn_dequantize_pages": (_c_i, [
+        _c_p, _c_i64, _c_i64,                       # pages, page stride, head stride
+        _c_p, _c_i64, _c_i64,                       # norms, page stride, head stride
+        _c_p, _c_i64, _c_p,                         # table, stride, seq_lens
+        _c_i, _c_i, _c_i, _c_i,                     # B, Lpad, Hkv, S
+        _c_p, _c_p, _c_i, _c_i,                     # centroids, Pi, bw, D
+        _c_p, _c_i, _c_p]),                         # out, out dtype, stream
     "wn_dequantize_histories": (_c_i, [
         _c_p, _c_i64, _c_i64,                       # pages, page stride, head stride
         _c_p, _c_i64, _c_i64,                       # norms, page stride, head stride

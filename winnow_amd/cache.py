@@ -15,17 +15,19 @@ On MI355X:
 * the append is one ``wn_append_kv`` launch for K and V together (quantize, pack
   and write into the contiguous rows: the buffer is addressed as B pages of one
   power-of-two page each, page b = sequence b) when there are no outlier channels
-  and the rows allow it; otherwise ``wn_quantize`` + ``wn_pack`` per channel group
-  (any group width up to 256);
+  and the rows allow it, one ``wn_append_split`` launch with outlier channels at
+  head_dim 64 and 128; otherwise ``wn_quantize`` + ``wn_pack`` per channel group (any
+  group width up to 256);
 * the history comes back through ``wn_tq_dequant`` (the fused kernel, read in place
   from the ``max_cache_len`` buffer) at head_dim 128 without outlier channels, else
-  through ``wn_unpack`` + ``wn_dequantize`` in chunks of ``chunk`` positions.
+  through ``wn_dequantize_rows`` at fp32 accuracy, K and V in one launch.
 
 ``kernel_backend`` keeps the reference's names: ``"triton_fp32"`` and
 ``"native_cuda_fp32"`` select the fused kernel at fp32 accuracy, ``"triton_tf32"``
 the fused kernel's fast mode (one fp16 product per term), ``"torch_fp32"`` the
-chunked standalone kernels, and ``"auto"`` the fused kernel where it applies (fast
-when ``allow_tf32``) and the chunked path elsewhere. The reference's dispatcher
+fp32-accurate rows kernel (the reference's chunked path, recorded under that name;
+``chunk`` is accepted and ignored), and ``"auto"`` the fused kernel where it applies
+(fast when ``allow_tf32``) and the rows kernel elsewhere. The reference's dispatcher
 (``dispatch.py``) is not used: ``native_kernel`` and ``dispatcher`` are accepted
 and ignored, and ``last_dispatch_decision`` records the path taken.
 """
@@ -38,12 +40,13 @@ from transformers.cache_utils import DynamicCache, DynamicLayer
 
 from winnow_amd import _lib
 from winnow_amd.kernel import tq_dequant
-from winnow_amd.packing import pack, packed_bytes, unpack
+from winnow_amd.packing import pack, packed_bytes
 from winnow_amd.quantizer import get_quantizer
 
 KERNEL_BACKENDS = ("auto", "torch_fp32", "triton_fp32", "triton_tf32", "native_cuda_fp32")
 _FUSED_HEAD_DIM = 128   # wn_tq_dequant's head_dim
 _APPEND_HEAD_DIMS = (16, 32, 64, 128, 256)
+_SPLIT_HEAD_DIMS = (64, 128)   # wn_append_split's
 
 
 @dataclass
@@ -72,13 +75,13 @@ class TQPackedLayer(DynamicLayer):
                  use_kernel: bool = True, allow_tf32: bool = True, kernel_backend: str = "auto",
                  native_kernel=None, dispatcher=None):
         super().__init__()
-        del native_kernel, dispatcher  # planner objects of the reference, not used here
+        del native_kernel, dispatcher, chunk  # not used here
         backend = kernel_backend if use_kernel else "torch_fp32"
         if backend not in KERNEL_BACKENDS:
             raise ValueError(f"unknown kernel_backend={kernel_backend!r}")
         self.use_kernel, self.allow_tf32, self.kernel_backend = use_kernel, allow_tf32, backend
         self.last_dispatch_decision: DequantChoice | None = None
-        self._head_dim, self._bits, self._capacity, self._span = head_dim, bit_width, max_cache_len, chunk
+        self._head_dim, self._bits, self._capacity = head_dim, bit_width, max_cache_len
         split = num_outlier_channels > 0 and outlier_bits > bit_width
         self._n_outlier = num_outlier_channels if split else 0
         self._n_regular = head_dim - self._n_outlier
@@ -90,6 +93,7 @@ class TQPackedLayer(DynamicLayer):
         self._outlier_row_bytes = packed_bytes(self._n_outlier, outlier_bits) if split else 0
         self._tokens = 0
         self._outlier_channels = None          # (head_dim,) bool: the outlier channels
+        self._split = None                     # (both rotations, channel groups) of the kernels: _split_operands
         self._k_groups = self._v_groups = None   # lists of _Group: regular, then outlier
         self._append_table = self._append_start = None   # fused append's (B, 1) table, start positions
         self.is_initialized = False
@@ -112,6 +116,7 @@ class TQPackedLayer(DynamicLayer):
             rms = key_states.float().pow(2).mean(dim=(0, 1, 2)).sqrt()
             self._outlier_channels = torch.zeros(D, dtype=torch.bool, device=dev)
             self._outlier_channels[rms.topk(min(self._n_outlier, D)).indices] = True
+            self._split = self._split_operands()
         self._dims = (B, H, D)
         self.is_initialized = True
 
@@ -150,6 +155,37 @@ class TQPackedLayer(DynamicLayer):
                       _lib.ptr(vg.norms), vg.norms.stride(0), vg.norms.stride(1),
                       B, H, n, D, S, B, 1, _lib.stream_of(dev), None, None)
 
+    def _split_operands(self):
+        """(head_dim, head_dim) fp32: the rotations of both channel groups, rows in code order
+        (regular, then outlier), columns in channel order, zero between the groups; and
+        the group of each channel, uint8. Built on the device without a copy back."""
+        order = torch.argsort(self._outlier_channels.to(torch.uint8), stable=True)   # regular channels, then outliers
+        both = torch.block_diag(self._quant.Pi, self._quant_outlier.Pi)
+        m = torch.empty_like(both)
+        m[:, order] = both
+        return m, self._outlier_channels.to(torch.uint8)
+
+    def _split_append_ok(self, k: torch.Tensor, v: torch.Tensor) -> bool:
+        """One wn_append_split launch writes both sides and groups: a compiled head_dim,
+        K/V rows that 16-byte loads read."""
+        return (bool(self._n_outlier) and self._head_dim in _SPLIT_HEAD_DIMS and k.dtype in _lib.DTYPE_CODE
+                and v.dtype == k.dtype and all(
+                    x.stride(-1) == 1 and x.data_ptr() % 16 == 0
+                    and all(s * x.element_size() % 16 == 0 for s in x.stride()[:3]) for x in (k, v)))
+
+    @torch.no_grad()
+    def _append_split(self, k: torch.Tensor, v: torch.Tensor, pos: int) -> None:
+        B, H, n, D = k.shape
+        m, chan = self._split
+        (kg, ko), (vg, vo), q, qo = self._k_groups, self._v_groups, self._quant, self._quant_outlier
+        with torch.cuda.device(k.device):
+            _lib.call("wn_append_split", _lib.ptr(k), *k.stride()[:3], _lib.ptr(v), *v.stride()[:3],
+                      _lib.DTYPE_CODE[k.dtype], _lib.ptr(m), _lib.ptr(chan), self._n_outlier, _lib.ptr(q.boundaries),
+                      self._bits, _lib.ptr(qo.boundaries), self._outlier_bits,
+                      _lib.ptr(kg.codes), _lib.ptr(vg.codes), _lib.ptr(kg.norms), _lib.ptr(vg.norms),
+                      _lib.ptr(ko.codes), _lib.ptr(vo.codes), _lib.ptr(ko.norms), _lib.ptr(vo.norms),
+                      B, H, n, D, self._capacity, pos, _lib.stream_of(k.device))
+
     @torch.no_grad()
     def _append_groups(self, x: torch.Tensor, groups, pos: int) -> None:
         """wn_quantize + wn_pack per channel group, written into [pos, pos + n)."""
@@ -183,34 +219,35 @@ class TQPackedLayer(DynamicLayer):
         return DequantChoice("fused", b == "triton_tf32", f"kernel_backend {b}")
 
     @torch.no_grad()
-    def _history(self, groups, length: int) -> torch.Tensor:
+    def _histories(self, length: int):
+        """K's and V's first ``length`` positions, dequantized."""
         B, H, D = self._dims
-        out = torch.empty(B, H, length, D, dtype=self.dtype, device=self.device)
+        k, v = (torch.empty(B, H, length, D, dtype=self.dtype, device=self.device) for _ in range(2))
         choice = self._choose()
         self.last_dispatch_decision = choice
         if length == 0:
-            return out
+            return k, v
         if choice.backend == "fused":
-            g = groups[0]
-            tq_dequant(g.codes[:, :, :length], g.norms[:, :, :length], self._quant.centroids, self._quant.Pi,
-                       self._bits, D, out=out, allow_tf32=choice.fast)
-            return out
-        quants = [(self._quant, self._bits, self._n_regular)] + \
-            ([(self._quant_outlier, self._outlier_bits, self._n_outlier)] if self._n_outlier else [])
-        for s in range(0, length, self._span):
-            e = min(s + self._span, length)
-            pieces = []
-            for g, (q, bw, dim) in zip(groups, quants):
-                part = torch.empty(B, H, e - s, dim, dtype=self.dtype, device=self.device)
-                q.dequantize_into(unpack(g.codes[:, :, s:e].contiguous(), bw, dim), g.norms[:, :, s:e], part)
-                pieces.append(part)
-            if self._n_outlier:
-                sl = out[:, :, s:e]
-                sl[..., ~self._outlier_channels] = pieces[0]
-                sl[..., self._outlier_channels] = pieces[1]
-            else:
-                out[:, :, s:e] = pieces[0]
-        return out
+            for g, out in ((self._k_groups[0], k), (self._v_groups[0], v)):
+                tq_dequant(g.codes[:, :, :length], g.norms[:, :, :length], self._quant.centroids, self._quant.Pi,
+                           self._bits, D, out=out, allow_tf32=choice.fast)
+            return k, v
+        exact = self.dtype in _lib.DTYPE_CODE   # else through fp32
+        ok, ov = (k, v) if exact else (k.float(), v.float())
+        kg, vg, q = self._k_groups[0], self._v_groups[0], self._quant
+        m, second = q.Pi, (None, None, None, None, 0, None, 0)
+        chan = None
+        if self._n_outlier:
+            m, chan = self._split
+            ko, vo, qo = self._k_groups[1], self._v_groups[1], self._quant_outlier
+            second = (_lib.ptr(ko.codes), _lib.ptr(vo.codes), _lib.ptr(ko.norms), _lib.ptr(vo.norms),
+                      self._outlier_bits, _lib.ptr(qo.centroids), self._n_outlier)
+        with torch.cuda.device(self.device):
+            _lib.call("wn_dequantize_rows", _lib.ptr(kg.codes), _lib.ptr(vg.codes), _lib.ptr(kg.norms),
+                      _lib.ptr(vg.norms), self._bits, _lib.ptr(q.centroids), *second, _lib.ptr(m), _lib.ptr(chan),
+                      B * H, length, self._capacity, D, _lib.ptr(ok), _lib.ptr(ov), _lib.DTYPE_CODE[ok.dtype],
+                      _lib.stream_of(self.device))
+        return (ok, ov) if exact else (ok.to(self.dtype), ov.to(self.dtype))
 
     # ---------------------------------------------------------------- cache protocol
     def update(self, key_states, value_states, *args, **kwargs):
@@ -222,11 +259,13 @@ class TQPackedLayer(DynamicLayer):
                                f"Raise max_cache_len.")
         if self._fused_append_ok(key_states):
             self._append_fused(key_states, value_states, self._tokens)
+        elif self._split_append_ok(key_states, value_states):
+            self._append_split(key_states, value_states, self._tokens)
         else:
             self._append_groups(key_states, self._k_groups, self._tokens)
             self._append_groups(value_states, self._v_groups, self._tokens)
         self._tokens += n
-        return self._history(self._k_groups, self._tokens), self._history(self._v_groups, self._tokens)
+        return self._histories(self._tokens)
 
     def get_seq_length(self, *a, **k) -> int:
         return self._tokens

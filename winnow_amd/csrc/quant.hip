@@ -1,5 +1,5 @@
 // TurboQuant quantize / bit-pack / page scatter (the KV append path) and the
-// standalone pack, unpack and dequantize ops, for gfx950.
+// standalone pack and unpack ops, for gfx950.
 //
 // quantize (turboquant_kv/cache.py:108-115):
 //   n = max(||x||_2, 1e-10);  y = (x / n) Pi^T;  code = #{boundaries < y}
@@ -410,36 +410,6 @@ __global__ void unpack_kernel(const uint8_t* packed, int64_t rows, int D, int bw
   out[e] = uint8_t(v & ((1u << bw) - 1u));
 }
 
-// out[r, j] = (sum_d c[code[r, d]] Pi[d, j]) * n[r] at a run-time head_dim <= 256.
-__global__ __launch_bounds__(kRtMaxD) void dequantize_rt_kernel(const uint8_t* codes, const uint16_t* norms,
-                                                                const float* pi, const float* cb, int bw, int D,
-                                                                void* out, int out_dtype) {
-  __shared__ float y[kRtMaxD];
-  const int64_t r = blockIdx.x;
-  const int j = threadIdx.x;
-  y[j] = cb[codes[r * D + j] & ((1u << bw) - 1u)];
-  __syncthreads();
-  float o = 0.f;
-  for (int d = 0; d < D; ++d) o = fmaf(y[d], pi[d * D + j], o);
-  store_elem(out, r * D + j, out_dtype, o * f16_to_f32(norms[r]));
-}
-
-// out[r, j] = (sum_d c[code[r, d]] Pi[d, j]) * n[r]  (cache.py:125-131)
-template <int D>
-__global__ __launch_bounds__(D) void dequantize_kernel(const uint8_t* codes, const uint16_t* norms,
-                                                      const float* pi, const float* cb, int bw, void* out,
-                                                      int out_dtype) {
-  __shared__ float y[D];
-  const int64_t r = blockIdx.x;
-  const int j = threadIdx.x;
-  y[j] = cb[codes[r * D + j] & ((1u << bw) - 1u)];
-  __syncthreads();
-  float o = 0.f;
-#pragma unroll 8
-  for (int d = 0; d < D; ++d) o = fmaf(y[d], pi[d * D + j], o);
-  store_elem(out, r * D + j, out_dtype, o * f16_to_f32(norms[r]));
-}
-
 }  // namespace
 }  // namespace wn
 
@@ -567,25 +537,42 @@ extern "C" int wn_unpack(const uint8_t* packed, int64_t rows, int D, int bw, uin
   return check_launch("wn_unpack");
 }
 
-extern "C" int wn_dequantize(const uint8_t* codes, const uint16_t* norms, int64_t rows, const float* pi,
-                             const float* centroids, int bw, int D, void* out, int out_dtype, void* stream) {
+extern "C" int wn_append_split(
+    const void* k, int64_t ks_b, int64_t ks_h, int64_t ks_n, const void* v, int64_t vs_b, int64_t vs_h, int64_t vs_n,
+    int x_dtype, const float* m, const uint8_t* channel_group, int count2, const float* boundaries, int bw,
+    const float* boundaries2, int bw2, uint8_t* k_codes, uint8_t* v_codes, uint16_t* k_norms, uint16_t* v_norms,
+    uint8_t* k_codes2, uint8_t* v_codes2, uint16_t* k_norms2, uint16_t* v_norms2, int B, int H, int n, int D,
+    int64_t capacity, int64_t pos, void* stream) {
   clear_error();
-  WN_REQUIRE(rows >= 0 && valid_bw(bw), WN_E_INVALID, "dequantize: rows=%lld bw=%d", (long long)rows, bw);
-  WN_REQUIRE(D >= 1 && D <= kRtMaxD, WN_E_UNSUPPORTED, "dequantize: head_dim %d (1 .. %d)", D, kRtMaxD);
-  WN_REQUIRE(out_dtype >= WN_F32 && out_dtype <= WN_BF16, WN_E_INVALID, "dequantize: dtype %d", out_dtype);
-  if (rows == 0) return WN_OK;
-  WN_REQUIRE(rows < (int64_t(1) << 31), WN_E_INVALID, "dequantize: too many rows");
-  WN_REQUIRE(codes && norms && pi && centroids && out, WN_E_INVALID, "dequantize: null operand");
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 grid(static_cast<unsigned>(rows));
-  switch (D) {
-    case 16: hipLaunchKernelGGL(dequantize_kernel<16>, grid, dim3(16), 0, st, codes, norms, pi, centroids, bw, out, out_dtype); break;
-    case 32: hipLaunchKernelGGL(dequantize_kernel<32>, grid, dim3(32), 0, st, codes, norms, pi, centroids, bw, out, out_dtype); break;
-    case 64: hipLaunchKernelGGL(dequantize_kernel<64>, grid, dim3(64), 0, st, codes, norms, pi, centroids, bw, out, out_dtype); break;
-    case 128: hipLaunchKernelGGL(dequantize_kernel<128>, grid, dim3(128), 0, st, codes, norms, pi, centroids, bw, out, out_dtype); break;
-    case 256: hipLaunchKernelGGL(dequantize_kernel<256>, grid, dim3(256), 0, st, codes, norms, pi, centroids, bw, out, out_dtype); break;
-    default:
-      hipLaunchKernelGGL(dequantize_rt_kernel, grid, dim3(D), 0, st, codes, norms, pi, centroids, bw, D, out, out_dtype);
-  }
-  return check_launch("wn_dequantize");
+  WN_REQUIRE(B >= 0 && H > 0 && n >= 0 && pos >= 0 && pos + n <= capacity && capacity < (int64_t(1) << 31), WN_E_INVALID,
+             "append_split: bad sizes B=%d H=%d n=%d at %lld of %lld", B, H, n, (long long)pos, (long long)capacity);
+  WN_REQUIRE(D == 64 || D == 128, WN_E_UNSUPPORTED, "append_split: head_dim %d (64 or 128)", D);
+  WN_REQUIRE(x_dtype >= WN_F32 && x_dtype <= WN_BF16, WN_E_INVALID, "append_split: dtype code %d", x_dtype);
+  WN_REQUIRE(valid_bw(bw) && valid_bw(bw2) && count2 > 0 && count2 < D && (D - count2) * bw % 8 == 0 &&
+                 count2 * bw2 % 8 == 0,
+             WN_E_INVALID, "append_split: %d outlier channels at %d bits beside %d", count2, bw2, bw);
+  if (int64_t(B) * n == 0) return WN_OK;
+  WN_REQUIRE(k && v && m && channel_group && boundaries && boundaries2 && k_codes && v_codes && k_norms && v_norms &&
+                 k_codes2 && v_codes2 && k_norms2 && v_norms2,
+             WN_E_INVALID, "append_split: null operand");
+  WN_REQUIRE(aligned(m, 16), WN_E_INVALID, "append_split: the rotations need 16-byte aligned rows");
+  QuantArgs a{};
+  a.side[0] = QuantSide{k, ks_b, ks_h, ks_n, m, boundaries, bw, k_codes, 0, 0, k_norms, 0, 0, nullptr, nullptr,
+                        boundaries2, bw2, k_codes2, k_norms2};
+  a.side[1] = QuantSide{v, vs_b, vs_h, vs_n, m, boundaries, bw, v_codes, 0, 0, v_norms, 0, 0, nullptr, nullptr,
+                        boundaries2, bw2, v_codes2, v_norms2};
+  a.total = int64_t(B) * H * n;
+  a.H = H;
+  a.n = n;
+  a.x_dtype = x_dtype;
+  a.scatter = 1;
+  a.chan = channel_group;
+  a.split = D - count2;
+  a.pos0 = int(pos);
+  a.cap = capacity;
+  WN_REQUIRE(quantize_split_ok(a, 2, D), WN_E_INVALID,
+             "append_split: K/V need 16-byte aligned rows and fewer than 2^31 vectors");
+  const int rc = launch_quantize_split(a, 2, D, static_cast<hipStream_t>(stream));
+  WN_REQUIRE(rc == WN_OK, rc, "append_split: cannot query the device");
+  return check_launch("wn_append_split");
 }

@@ -33,6 +33,14 @@
 // norms of 128 or more), take the float64 path for every code. The codes of a pass sit
 // in LDS as bytes, so that whole rows are packed and stored by neighbouring lanes.
 //
+// With outlier channels (G2; the contiguous cache) a vector is two: its regular and its
+// outlier channels, each with its own norm, rotation, boundaries and width. Pi is then
+// the matrix of both rotations, rows in code order (regular first), columns in channel
+// order, zero between the groups; the norms, thresholds, grids and exact dot products
+// are taken per group, and the rows are packed byte by byte (a group's codes need not
+// fill eights). A prompt of 2,048 tokens (2 sequences, 8 heads; 120 channels at 4 bits, 8 at
+// 8) took sixteen launches and copies, a single token 25 us now, the prompt 53 us.
+//
 // Measured (K and V of 8 kv heads in one launch, head_dim 128, quantize_kernel -> this):
 // 8,191 tokens 4 bits bf16 128 -> 30 us, 8 bits 133 -> 47 us, 4 bits fp32 119 -> 34 us;
 // 65,536 tokens 4 bits bf16 947 -> 186 us (1.8 TB/s). The vector ALU bounds it: about
@@ -49,7 +57,9 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
-constexpr int kTileWaves = 16;   // waves of a work-group
+// waves of a work-group (two groups of channels: eight, whose registers they need)
+template <bool G2>
+constexpr int tile_waves() { return G2 ? 8 : 16; }
 constexpr int kTileVecs = 16;    // vectors a wave takes per pass (an MFMA column tile)
 constexpr int kCells = 512;      // cells of the boundary grid
 constexpr int kListMax = 256;    // flagged pairs a wave lists; with more it recomputes the whole pass
@@ -100,8 +110,9 @@ __device__ __forceinline__ float elem(const Raw8<DT>& r, int k) {
 // float64 sum of squares of a lane's elements reduced over the four lanes of a vector,
 // in quantize_kernel's order: D/16 consecutive elements in turn, then the sixteen
 // partial sums by halves.
-template <int DT, int KS>
-__device__ __forceinline__ double sum_squares(const Raw8<DT> (&x)[KS]) {
+// G2: the elements of one group only, `in` naming the lane's elements 8s + k in it.
+template <int DT, int KS, bool G2>
+__device__ __forceinline__ double sum_squares(const Raw8<DT> (&x)[KS], uint32_t in) {
   constexpr int EPT = 2 * KS, PPL = 8 / EPT;  // elements per partial sum, partial sums per eight elements
   double p[KS][PPL];
 #pragma unroll
@@ -112,7 +123,8 @@ __device__ __forceinline__ double sum_squares(const Raw8<DT> (&x)[KS]) {
 #pragma unroll
       for (int k = 0; k < EPT; ++k) {
         const double e = double(elem<DT>(x[s], EPT * h + k));
-        ss = fma(e, e, ss);
+        const double f = !G2 || (in >> (8 * s + EPT * h + k) & 1) ? e : 0.0;
+        ss = fma(f, f, ss);
       }
       __builtin_amdgcn_sched_barrier(0);
       p[s][h] = ss;
@@ -136,7 +148,7 @@ struct RowInfo {
   int64_t x;     // element offset of x
   int64_t page;  // byte offset of the packed row, or element offset of its codes; -1: not written
   int64_t norm;  // element offset of the norm
-  float n;       // the norm
+  float n[2];    // the norms of the two groups (one group: the first)
 };
 
 template <int D>
@@ -153,35 +165,46 @@ __device__ __forceinline__ uint8_t* code8(TileWave<D>& w, int r, int k) {
   return w.code[r] + 8 * (k ^ ((r >> 1) & (D / 8 - 1)));
 }
 
-template <int D, int DT>
-__global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArgs a) {
+template <int D, int DT, bool G2>
+__global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(QuantArgs a) {
+  constexpr int WV = tile_waves<G2>();
   constexpr int KS = D / 32;  // K-steps of 32 input dims
   constexpr int U = D / 32;   // eights of output dims per lane (two MFMA row tiles each)
-  constexpr int NR = kTileVecs, NTHR = 64 * kTileWaves;
+  constexpr int NR = kTileVecs, NTHR = 64 * WV;
   constexpr bool F32 = DT == WN_F32;
+  constexpr int NG = G2 ? 2 : 1;
   __shared__ __align__(16) h8 ph[2 * U][KS][64], pl[2 * U][KS][64];
-  __shared__ __align__(8) Cell cells[kCells];
-  __shared__ float bnd[256];
+  __shared__ __align__(8) Cell cells[NG][kCells];
+  __shared__ float bnd[NG][256];
   __shared__ float rowsq[D];
-  __shared__ TileWave<D> waves[kTileWaves];
+  __shared__ TileWave<D> waves[WV];
 
   const QuantSide& sd = a.side[blockIdx.y];
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int wig = __builtin_amdgcn_readfirstlane(tid >> 6);
   TileWave<D>& wv = waves[wig];
-  const int bw = sd.bw, nb = (1 << bw) - 1;
+  const int bw = sd.bw, split = G2 ? a.split : D;
+  uint32_t outl = 0;  // bit 8s + k: channel 32s + 8g + k is an outlier
+  if constexpr (G2) {
+#pragma unroll
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) outl |= (a.chan[32 * s + 8 * g + k] ? 1u : 0u) << (8 * s + k);
+  }
   // passes are dealt to the work-groups in turn, so that a launch of few passes still
   // spreads over the CUs
-  const int64_t passes = (a.total + NR - 1) / NR, stride = int64_t(gridDim.x) * kTileWaves;
+  const int64_t passes = (a.total + NR - 1) / NR, stride = int64_t(gridDim.x) * WV;
   int64_t pass = int64_t(wig) * gridDim.x + blockIdx.x;
-  for (int i = tid; i < nb; i += NTHR) bnd[i] = sd.bnd[i];
+#pragma unroll
+  for (int q = 0; q < NG; ++q)
+    for (int i = tid; i < (1 << (q ? sd.bw2 : bw)) - 1; i += NTHR) bnd[q][i] = (q ? sd.bnd2 : sd.bnd)[i];
   for (int i = tid; i < D; i += NTHR) rowsq[i] = 0.f;
   __syncthreads();
   // operand (t, s, lane 16g + c): row r = c of tile t = 2u + h is output dim
   // D/4 (c >> 2) + 8u + 4h + (c & 3), k-slots of group g the input dims 32s + 8g ..
 #pragma unroll
-  for (int it = 0; it < (2 * U * KS + kTileWaves - 1) / kTileWaves; ++it) {
-    const int item = it * kTileWaves + wig, t = item / KS, s = item % KS;
+  for (int it = 0; it < (2 * U * KS + WV - 1) / WV; ++it) {
+    const int item = it * WV + wig, t = item / KS, s = item % KS;
     if (item < 2 * U * KS) {
       const int dim = (D / 4) * (c >> 2) + 8 * (t >> 1) + 4 * (t & 1) + (c & 3);
       const float4* p = reinterpret_cast<const float4*>(sd.pi + dim * D + 32 * s + 8 * g);
@@ -202,27 +225,35 @@ __global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArg
     }
   }
   __syncthreads();
-  float rmax = 0.f;  // largest squared row norm (a NaN row is left out: its own dims' y are NaN, hence flagged)
+  float eps[NG], inv_w[NG], at0[NG];
 #pragma unroll
-  for (int i = 0; i < D; i += 64) rmax = fmaxf(rmax, rowsq[i + lane]);
-  rmax = wave_max(rmax);
-  const float eps = rmax < 16384.f ? (D * 0x1p-23f + 0x1p-20f) * 1.01f * sqrtf(rmax) : NAN;
-  // cells of width cw: cell 0 ends at the first boundary, the last one starts at the last
-  const float b0 = bnd[0], b1 = bnd[nb - 1];
-  const float cw = (b1 - b0) / float(kCells - 2);
-  const bool grid_ok = cw > 0.f && cw < INFINITY && fabsf(b0) < INFINITY && eps < INFINITY;
-  const float inv_w = grid_ok ? 8.f / cw : 0.f;  // 8: bytes of a cell
-  const float lo0 = b0 - cw, at0 = -lo0 * inv_w;
-  for (int i = tid; i < kCells; i += NTHR) {
-    const float reach = eps + 0.05f * cw;  // 0.05 cw: rounding of the cell number and of the edges
-    Cell e{NAN, 0};
-    if (grid_ok) {
-      const uint32_t below = i == 0 ? 0 : count_below(bnd, bw, lo0 + i * cw - reach);
-      const uint32_t upto = i == kCells - 1 ? nb : count_below(bnd, bw, lo0 + (i + 1) * cw + reach);
-      e.base = below;
-      e.b = upto == below ? INFINITY : upto == below + 1 ? bnd[below] : NAN;
+  for (int q = 0; q < NG; ++q) {
+    const int qbw = q ? sd.bw2 : bw, nb = (1 << qbw) - 1;
+    const float* bd = bnd[q];
+    float rmax = 0.f;  // largest squared row norm (a NaN row is left out: its own dims' y are NaN, hence flagged)
+#pragma unroll
+    for (int i = 0; i < D; i += 64)
+      if (!G2 || (i + lane >= split) == (q == 1)) rmax = fmaxf(rmax, rowsq[i + lane]);
+    rmax = wave_max(rmax);
+    eps[q] = rmax < 16384.f ? (D * 0x1p-23f + 0x1p-20f) * 1.01f * sqrtf(rmax) : NAN;
+    // cells of width cw: cell 0 ends at the first boundary, the last one starts at the last
+    const float b0 = bd[0], b1 = bd[nb - 1];
+    const float cw = (b1 - b0) / float(kCells - 2);
+    const bool grid_ok = cw > 0.f && cw < INFINITY && fabsf(b0) < INFINITY && eps[q] < INFINITY;
+    inv_w[q] = grid_ok ? 8.f / cw : 0.f;  // 8: bytes of a cell
+    const float lo0 = b0 - cw;
+    at0[q] = -lo0 * inv_w[q];
+    for (int i = tid; i < kCells; i += NTHR) {
+      const float reach = eps[q] + 0.05f * cw;  // 0.05 cw: rounding of the cell number and of the edges
+      Cell e{NAN, 0};
+      if (grid_ok) {
+        const uint32_t below = i == 0 ? 0 : count_below(bd, qbw, lo0 + i * cw - reach);
+        const uint32_t upto = i == kCells - 1 ? nb : count_below(bd, qbw, lo0 + (i + 1) * cw + reach);
+        e.base = below;
+        e.b = upto == below ? INFINITY : upto == below + 1 ? bd[below] : NAN;
+      }
+      cells[q][i] = e;
     }
-    cells[i] = e;
   }
   __syncthreads();  // the only block-wide barriers: waves run independently from here
 
@@ -236,7 +267,9 @@ __global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArg
       o.x = b * sd.sb + h * sd.sh + i * sd.sn;
       int64_t page = -1, norm = 0;
       if (vec < a.total) {
-        if (!a.scatter) {
+        if (G2) {
+          page = norm = (int64_t(b) * a.H + h) * a.cap + a.pos0 + i;  // the row's number
+        } else if (!a.scatter) {
           page = vec * D;
           norm = vec;
         } else {
@@ -253,26 +286,30 @@ __global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArg
       o.norm = norm;
     }
     wave_lds_sync();
-    float r, thr;
+    float r[NG], thr[NG];
     h8 xh[KS], xl[F32 ? KS : 1];
     {
       Raw8<DT> x[KS];
       const int64_t xo = wv.row[c].x + 8 * g;
 #pragma unroll
       for (int s = 0; s < KS; ++s) x[s] = load8<DT>(sd.x, xo + 32 * s);
-      const float n = fmaxf(float(sqrt(sum_squares<DT, KS>(x))), 1e-10f);
-      if (g == 0) wv.row[c].n = n;
-      int e;
-      frexpf(n, &e);
-      const bool sane = n < 0x1p100f;
-      const float sc = sane ? ldexpf(1.f, 8 - e) : 0.f;
-      r = sane ? ldexpf(1.f / n, e - 16) : 0.f;
-      thr = sane ? eps : NAN;  // NaN: every code is flagged
+      float sc[NG];
+#pragma unroll
+      for (int q = 0; q < NG; ++q) {
+        const float n = fmaxf(float(sqrt(sum_squares<DT, KS, G2>(x, q ? outl : ~outl))), 1e-10f);
+        if (g == 0) wv.row[c].n[q] = n;
+        int e;
+        frexpf(n, &e);
+        const bool sane = n < 0x1p100f;
+        sc[q] = sane ? ldexpf(1.f, 8 - e) : 0.f;
+        r[q] = sane ? ldexpf(1.f / n, e - 16) : 0.f;
+        thr[q] = sane ? eps[q] : NAN;  // NaN: every code is flagged
+      }
 #pragma unroll
       for (int s = 0; s < KS; ++s)
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-          const float z = elem<DT>(x[s], k) * sc;
+          const float z = elem<DT>(x[s], k) * (G2 && (outl >> (8 * s + k) & 1) ? sc[NG - 1] : sc[0]);
           xh[s][k] = _Float16(z);
           if constexpr (F32) xl[s][k] = _Float16(z - float(xh[s][k]));
         }
@@ -298,7 +335,10 @@ __global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArg
           if constexpr (F32) low[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(p, xl[s], low[h], 0, 0, 0);
         }
       }
-      const float rw = r * inv_w;  // inv_w, at0: in bytes of the table
+      float rw[NG];  // inv_w, at0: in bytes of the table
+#pragma unroll
+      for (int q = 0; q < NG; ++q) rw[q] = r[q] * inv_w[q];
+      const int j0 = (D / 4) * g + 8 * u;  // the lane's first code of the eight
       uint32_t word[2];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -306,16 +346,20 @@ __global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArg
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           acc[h][i] += low[h][i];
+          const int q = G2 && j0 + 4 * h + i >= split;
           // the cell number, below 0 and past the end clamped; a NaN reads some cell
-          const float at = __builtin_amdgcn_fmed3f(fmaf(acc[h][i], rw, at0), 0.f, 8.f * kCells - 1.f);
-          e[i] = *reinterpret_cast<const Cell*>(reinterpret_cast<const char*>(cells) + (uint32_t(at) & (8 * kCells - 8)));
+          const float at = __builtin_amdgcn_fmed3f(fmaf(acc[h][i], q ? rw[NG - 1] : rw[0], q ? at0[NG - 1] : at0[0]), 0.f,
+                                                   8.f * kCells - 1.f);
+          e[i] = *reinterpret_cast<const Cell*>(reinterpret_cast<const char*>(cells[0]) + (uint32_t(at) & (8 * kCells - 8)) +
+                                                (q ? 8 * kCells : 0));
         }
         word[h] = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float d = fmaf(acc[h][i], r, -e[i].b);  // y - b
+          const int q = G2 && j0 + 4 * h + i >= split;
+          const float d = fmaf(acc[h][i], q ? r[NG - 1] : r[0], -e[i].b);  // y - b
           word[h] |= (e[i].base + (d > 0.f ? 1u : 0u)) << (8 * i);
-          const uint64_t near = __ballot(!(fabsf(d) >= thr));
+          const uint64_t near = __ballot(!(fabsf(d) >= (q ? thr[NG - 1] : thr[0])));
           if (near) {  // wave-uniform, taken for one in ten at 4 bits
             const int at = flagged + int(__builtin_amdgcn_mbcnt_hi(uint32_t(near >> 32),
                                                                    __builtin_amdgcn_mbcnt_lo(uint32_t(near), 0)));
@@ -334,7 +378,8 @@ __global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArg
       const int j = min(j0 + c, items - 1);
       const int id = all ? j : int(wv.list[j]);
       const int rr = id / D, dim = id % D;
-      const float n = wv.row[rr].n, rn = 1.f / n;
+      const int q2 = G2 && dim >= split;  // the group
+      const float n = wv.row[rr].n[q2], rn = 1.f / n;
       const bool divide = __any(!(n < 0x1p100f));  // wave-uniform
       const int64_t xo = wv.row[rr].x + 8 * g;
       const float* prow = sd.pi + dim * D + 8 * g;
@@ -354,20 +399,44 @@ __global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArg
         for (int k = 0; k < 8; ++k) {
           const float xv = elem<DT>(x, k), q = xv * rn;
           z[k] = fmaf(fmaf(-q, n, xv), rn, q);
+          if (G2 && int(outl >> (8 * s + k) & 1) != q2) z[k] = 0.f;
         }
         if (divide) {
           asm volatile("" ::: "memory");  // a branch: the divisions are not formed for a select
 #pragma unroll
-          for (int k = 0; k < 8; ++k) z[k] = elem<DT>(x, k) / n;
+          for (int k = 0; k < 8; ++k) z[k] = G2 && int(outl >> (8 * s + k) & 1) != q2 ? 0.f : elem<DT>(x, k) / n;
         }
 #pragma unroll
         for (int k = 0; k < 8; ++k) sum = fma(double(z[k]), double(p[k]), sum);
       }
       sum += __shfl_xor(sum, 16, 64);
       sum += __shfl_xor(sum, 32, 64);
-      if (g == 0) code8<D>(wv, rr, dim >> 3)[dim & 7] = uint8_t(count_below(bnd, bw, float(sum)));
+      if (g == 0) code8<D>(wv, rr, dim >> 3)[dim & 7] = uint8_t(count_below(bnd[q2], q2 ? sd.bw2 : bw, float(sum)));
     }
     wave_lds_sync();
+    if constexpr (G2) {
+      // byte by byte: the bytes of both groups' rows, neighbouring lanes neighbouring bytes
+      const int nb1 = split * bw / 8, nb2 = (D - split) * sd.bw2 / 8, nball = nb1 + nb2;
+      for (int i = lane; i < NR * nball; i += 64) {
+        const int rr = i / nball, k = i % nball, q = k >= nb1;
+        const int64_t row = wv.row[rr].page;
+        if (row < 0) continue;
+        const int w = q ? sd.bw2 : bw, first = q ? split : 0, end = q ? D : split, bit0 = 8 * (q ? k - nb1 : k);
+        uint32_t v = 0;
+        for (int d = bit0 / w; first + d < end && d * w < bit0 + 8; ++d) {
+          const int j = first + d, sh = d * w - bit0;
+          const uint32_t cd = code8<D>(wv, rr, j >> 3)[j & 7];
+          v |= sh >= 0 ? cd << sh : cd >> -sh;
+        }
+        if (q) sd.pages2[row * nb2 + k - nb1] = uint8_t(v);
+        else sd.pages[row * nb1 + k] = uint8_t(v);
+      }
+      if (lane < NR && wv.row[lane].page >= 0) {
+        sd.norms[wv.row[lane].norm] = f32_to_f16(wv.row[lane].n[0]);
+        sd.norms2[wv.row[lane].norm] = f32_to_f16(wv.row[lane].n[1]);
+      }
+      continue;
+    }
     // whole rows: D/8 lanes each pack and store eight codes
     constexpr int LPR = D / 8, RPI = 64 / LPR;
 #pragma unroll
@@ -378,7 +447,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArg
       const uint2 w = *reinterpret_cast<const uint2*>(code8<D>(wv, rr, part));
       if (!a.scatter) {
         *reinterpret_cast<uint2*>(sd.codes_out + page + 8 * part) = w;
-        if (part == 0) sd.norms_out[wv.row[rr].norm] = wv.row[rr].n;
+        if (part == 0) sd.norms_out[wv.row[rr].norm] = wv.row[rr].n[0];
         continue;
       }
       uint8_t* dst = sd.pages + page + part * bw;
@@ -392,18 +461,18 @@ __global__ __launch_bounds__(64 * kTileWaves) void quantize_tile_kernel(QuantArg
         for (int k = 0; k < 8; ++k) pk |= uint64_t((k < 4 ? w.x : w.y) >> (8 * (k & 3)) & 0xffu) << (bw * k);
         store_packed8(dst, pk, bw);
       }
-      if (part == 0) sd.norms[wv.row[rr].norm] = f32_to_f16(wv.row[rr].n);
+      if (part == 0) sd.norms[wv.row[rr].norm] = f32_to_f16(wv.row[rr].n[0]);
     }
   }
 }
 
 using TileFn = void (*)(QuantArgs);
 
-template <int D>
+template <int D, bool G2>
 TileFn pick_tile(int dtype) {
-  return dtype == WN_F32   ? quantize_tile_kernel<D, WN_F32>
-         : dtype == WN_F16 ? quantize_tile_kernel<D, WN_F16>
-                           : quantize_tile_kernel<D, WN_BF16>;
+  return dtype == WN_F32   ? quantize_tile_kernel<D, WN_F32, G2>
+         : dtype == WN_F16 ? quantize_tile_kernel<D, WN_F16, G2>
+                           : quantize_tile_kernel<D, WN_BF16, G2>;
 }
 
 bool rows_aligned(const QuantSide& s, int es) {
@@ -428,16 +497,31 @@ bool quantize_tiles_ok(const QuantArgs& a, int sides, int D) {
   return a.total * sides >= (wide ? 16384 : 12288);
 }
 
-int launch_quantize_tiles(const QuantArgs& a, int sides, int D, hipStream_t st) {
-  const TileFn fn = D == 64 ? pick_tile<64>(a.x_dtype) : pick_tile<128>(a.x_dtype);
+static int launch_tiles(TileFn fn, int waves, const QuantArgs& a, int sides, hipStream_t st) {
   // one work-group per CU; its passes are dealt out from there
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return WN_E_LAUNCH;
   const int64_t groups = std::min<int64_t>((a.total + kTileVecs - 1) / kTileVecs, std::max(1, cus / sides));
-  hipLaunchKernelGGL(fn, dim3(unsigned(groups), sides), dim3(64 * kTileWaves), 0, st, a);
+  hipLaunchKernelGGL(fn, dim3(unsigned(groups), sides), dim3(64 * waves), 0, st, a);
   return WN_OK;
+}
+
+int launch_quantize_tiles(const QuantArgs& a, int sides, int D, hipStream_t st) {
+  return launch_tiles(D == 64 ? pick_tile<64, false>(a.x_dtype) : pick_tile<128, false>(a.x_dtype), tile_waves<false>(), a, sides, st);
+}
+
+bool quantize_split_ok(const QuantArgs& a, int sides, int D) {
+  if ((D != 64 && D != 128) || a.total >= (int64_t(1) << 31)) return false;
+  const int es = a.x_dtype == WN_F32 ? 4 : 2;
+  for (int i = 0; i < sides; ++i)
+    if (!rows_aligned(a.side[i], es)) return false;
+  return true;
+}
+
+int launch_quantize_split(const QuantArgs& a, int sides, int D, hipStream_t st) {
+  return launch_tiles(D == 64 ? pick_tile<64, true>(a.x_dtype) : pick_tile<128, true>(a.x_dtype), tile_waves<true>(), a, sides, st);
 }
 
 }  // namespace wn

@@ -18,6 +18,11 @@ struct QuantSide {
   int64_t nsp, nsh;
   uint8_t* codes_out;  // flat mode
   float* norms_out;
+  // outlier channels (launch_quantize_split): boundaries, width, rows and norms of the second group
+  const float* bnd2;
+  int bw2;
+  uint8_t* pages2;
+  uint16_t* norms2;
 };
 
 struct QuantArgs {
@@ -27,6 +32,10 @@ struct QuantArgs {
   int64_t tsb;
   int64_t total;  // vectors per side = B*H*n
   int H, n, log2S, num_pages, max_pages, x_dtype, scatter;
+  // launch_quantize_split: group of each channel, codes of group 0, rows per (sequence, head), first position
+  const uint8_t* chan;
+  int split, pos0;
+  int64_t cap;
 };
 
 // pos[k] = #{b < y[k]} over the 2^bw - 1 ascending boundaries (torch.bucketize,
@@ -66,5 +75,9 @@ __device__ __forceinline__ void store_packed8(uint8_t* p, uint64_t v, int bw) {
 // quant_tile.hip: whether its kernel serves these operands, and its launch (0: launched).
 bool quantize_tiles_ok(const QuantArgs& a, int sides, int D);
 int launch_quantize_tiles(const QuantArgs& a, int sides, int D, hipStream_t st);
+// The same kernel with two groups of channels, rows of a contiguous cache (quant.hip's
+// wn_append_split).
+bool quantize_split_ok(const QuantArgs& a, int sides, int D);
+int launch_quantize_split(const QuantArgs& a, int sides, int D, hipStream_t st);
 
 }  // namespace wn

@@ -414,9 +414,9 @@ def _host_table(kv) -> torch.Tensor:
 def dequantize_history(kv: pa.PackedKV, pages, norms, quant, b: int, dtype) -> torch.Tensor:
     """(1, Hkv, L, D) reconstruction of sequence b's history, on the GPU (packed_backend.py:192-208).
 
-    head_dim 128 with contiguous page rows: one ``wn_dequantize_history`` launch reads
-    the pool pages through the table row. Other shapes gather the rows, unpack and
-    dequantize with the standalone kernels."""
+    Contiguous page rows: one launch reads the pool pages through the table row,
+    ``wn_dequantize_history`` at head_dim 128 and ``wn_dequantize_pages`` at the others.
+    Other layouts gather the rows, unpack and dequantize with the standalone kernels."""
     L = int(_host_lens(kv)[b])
     S, D, Hkv = kv.page_size, kv.head_dim, pages.shape[1]
     odt = dtype if dtype in _lib.DTYPE_CODE else torch.float32
@@ -430,6 +430,8 @@ def dequantize_history(kv: pa.PackedKV, pages, norms, quant, b: int, dtype) -> t
                       _lib.ptr(norms), norms.stride(0), norms.stride(1), _lib.ptr(kv.page_table[b]), L, Hkv, S,
                       _lib.ptr(quant.centroids), _lib.ptr(quant.Pi), quant.bit_width, D, _lib.ptr(out),
                       _lib.DTYPE_CODE[odt], 0, _lib.stream_of(pages.device))
+        elif _paged_rows(kv, pages, norms):
+            _dequantize_pages(kv, pages, norms, quant, kv.page_table[b:b + 1], None, L, out)
         else:
             ids = _host_table(kv)[b, :-(-L // S)].to(torch.int64).to(pages.device)
             rows = pages[ids].transpose(0, 1).reshape(Hkv, -1, pages.shape[-1])[:, :L].contiguous()
@@ -439,6 +441,22 @@ def dequantize_history(kv: pa.PackedKV, pages, norms, quant, b: int, dtype) -> t
                       _lib.ptr(quant.centroids), quant.bit_width, D, _lib.ptr(out), _lib.DTYPE_CODE[odt],
                       _lib.stream_of(pages.device))
     return out.to(dtype)
+
+
+def _paged_rows(kv: pa.PackedKV, pages, norms) -> bool:
+    """Whether ``wn_dequantize_pages`` can address these pages."""
+    S, D, table = kv.page_size, kv.head_dim, kv.page_table
+    return (D <= 256 and S & (S - 1) == 0 and pages.stride(-1) == 1 and pages.stride(-2) == pages.shape[-1]
+            and norms.stride(-1) == 1 and table.dtype == torch.int32 and table.stride(-1) == 1
+            and table.device == pages.device)
+
+
+def _dequantize_pages(kv: pa.PackedKV, pages, norms, quant, table, lens, Lpad: int, out) -> None:
+    """``out`` (len(table), Hkv, Lpad, D) of the sequences whose table rows are given."""
+    _lib.call("wn_dequantize_pages", _lib.ptr(pages), pages.stride(0), pages.stride(1), _lib.ptr(norms), norms.stride(0),
+              norms.stride(1), _lib.ptr(table), table.stride(0), _lib.ptr(lens), table.shape[0], Lpad, pages.shape[1],
+              kv.page_size, _lib.ptr(quant.centroids), _lib.ptr(quant.Pi), quant.bit_width, kv.head_dim, _lib.ptr(out),
+              _lib.DTYPE_CODE[out.dtype], _lib.stream_of(pages.device))
 
 
 def _offset_causal(lens: torch.Tensor, Q: int, Lmax: int, device):
@@ -482,7 +500,7 @@ def _history_kernel(query, kv: pa.PackedKV, Lmax: int) -> bool:
 
 def _histories(kv: pa.PackedKV, pages, norms, quant, lens, Lmax: int, dtype) -> torch.Tensor:
     """(B, Hkv, Lmax, D) histories of the batch; what lies past a length is not meant to be
-    read. head_dim 128 with contiguous rows: one launch; else sequence by sequence."""
+    read. Contiguous page rows: one launch; else sequence by sequence."""
     B, S, D, Hkv = lens.shape[0], kv.page_size, kv.head_dim, kv.num_kv_heads
     buf = torch.empty(B, Hkv, Lmax, D, dtype=dtype, device=pages.device)
     if D == 128 and pages.stride(-1) == 1 and pages.stride(-2) == pages.shape[-1] and norms.stride(-1) == 1:
@@ -491,6 +509,10 @@ def _histories(kv: pa.PackedKV, pages, norms, quant, lens, Lmax: int, dtype) -> 
                       norms.stride(0), norms.stride(1), _lib.ptr(kv.page_table), kv.page_table.stride(0),
                       _lib.ptr(kv.seq_lens), B, Lmax, Hkv, S, _lib.ptr(quant.centroids), _lib.ptr(quant.Pi),
                       quant.bit_width, D, _lib.ptr(buf), _lib.DTYPE_CODE[dtype], 0, _lib.stream_of(pages.device))
+        return buf
+    if D != 128 and _paged_rows(kv, pages, norms):
+        with torch.cuda.device(pages.device):
+            _dequantize_pages(kv, pages, norms, quant, kv.page_table, kv.seq_lens, Lmax, buf)
         return buf
     for b in range(B):
         if lens[b]:
