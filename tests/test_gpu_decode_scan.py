@@ -1,0 +1,57 @@
+"""The decode row scan on the 16-bit matrix cores at the widths and sizes where a chunk,
+a page or a split ends, against the same attention in float64.
+
+The scan multiplies fp16 pairs (H + L carries a value to 2^-22 of itself) and accumulates
+in fp32, so a score is off by at most 2^-19 sum|q k| (both factors, 128 products' sums), a weight by twice that relative to itself with the exponential's own
+error, and an output by that share of the largest value; the values' own split and the
+rotation back add 2^-17 of the largest value. The bound below is that, from the case's data.
+"""
+from __future__ import annotations
+
+import pytest
+import torch
+
+from cases import build, to_device
+from oracle import attention as oa
+
+pytestmark = pytest.mark.gpu
+
+
+def _float64(q, kv, scale):
+    """(attention in float64 over the rotated codes, the bound above)."""
+    B, Hq, _, D = q.shape
+    rep = Hq // kv.num_kv_heads
+    out = torch.zeros(B, Hq, 1, D, dtype=torch.float64)
+    qr = q.double() @ kv.k_quant.Pi.double().T
+    smax = vmax = 0.0
+    for b in range(B):
+        if int(kv.seq_lens[b]) == 0:
+            continue
+        kc, kn = oa._gather_history(kv.k_pages, kv.k_norms, kv, b)
+        vc, vn = oa._gather_history(kv.v_pages, kv.v_norms, kv, b)
+        k = oa._centroids(kc, kv.k_quant, D).double() * kn.double()[..., None]
+        v = oa._centroids(vc, kv.v_quant, D).double() * vn.double()[..., None]
+        k, v = (x.repeat_interleave(rep, 0) for x in (k, v))
+        p = torch.softmax((k @ qr[b].transpose(-1, -2)).squeeze(-1) * scale, -1)
+        out[b, :, 0] = (p[:, None] @ v).squeeze(1) @ kv.v_quant.Pi.double()
+        smax = max(smax, float((k.abs() @ qr[b].abs().transpose(-1, -2)).max()) * scale)
+        vmax = max(vmax, float(v.norm(dim=-1).max()))
+    return out, (2 * 2.0 ** -19 * smax + 2.0 ** -17) * vmax
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,bwk,bwv", [(16, 28, 4, 8, 8), (64, 8, 8, 8, 8), (32, 64, 8, 8, 8), (16, 12, 2, 4, 8),
+                                              (128, 4, 2, 4, 8), (16, 28, 4, 4, 4)])
+def test_scan_edges(S, Hq, Hkv, bwk, bwv, D=128):
+    lens = (0, 1, 63, 64, 65, 130, 2049)
+    q, kv = build(700 + S + bwk, len(lens), Hq, Hkv, D, lens, S, bwk, bw_v=bwv)
+    scale = oa.default_scale(D)
+    ref, tol = _float64(q, kv, scale)
+    from winnow_amd import packed_attention as pa
+    for splits in (None, 1, 7):
+        print(f"S={S} {Hq}/{Hkv} heads {bwk}/{bwv} bits D={D} splits={splits}", flush=True)
+        got = pa.packed_decode_attention(q.cuda(), to_device(kv, "cuda"), scale, num_splits=splits,
+                                         out_dtype=torch.float32).cpu().double()
+        assert torch.isfinite(got).all()
+        err = float((got - ref).abs().max())
+        assert err <= tol, (err, tol)
+        assert (got[0] == 0).all()

@@ -38,6 +38,7 @@
 // reference kernel packed_attention_triton.py:51-134).
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 #include <utility>
 
 #include "wn_decode.h"
@@ -805,7 +806,7 @@ __global__ __launch_bounds__(64 * WPB) void decode_rows_kernel(DecodeArgs a) {
 // ------------------------------------------------------------------ 16-bit matrix-core scan
 //
 // The page scan on v_mfma_f32_16x16x32_f16 (16 times the MAC rate of the fp32 4x4x1
-// MFMA on gfx950), for 2, 3, 4, 5 and 6-bit codes. Every fp32 factor x is carried as
+// MFMA on gfx950), for 2, 3, 4, 5 and 6-bit codes, 8-bit ones, and 4 with 8. Every fp32 factor x is carried as
 // an fp16 pair x = H + L (H = fp16(x), L = fp16(x - H)) after an exact power-of-two
 // scaling that keeps both in fp16's normal range; products of fp16 values are exact
 // in the fp32 accumulators and each factor keeps 22 bits, so scores and values keep
@@ -815,6 +816,10 @@ __global__ __launch_bounds__(64 * WPB) void decode_rows_kernel(DecodeArgs a) {
 // [H0, L0, H1, L1]; two entries loaded side by side are an 8-slot MFMA operand, and
 // the other operand carries its factor twice per code ([f0, f0, f1, f1, ...]), so
 // the k-slots pair each code's H and L with the same factor. Lane l = 16g + c.
+// An 8-bit pair table would not fit LDS: 8-bit codes have a table of single codes,
+// [H, L] in 4 bytes, replicated once per lane of the wave as the TF32-class scan's
+// 4-bit table is (entry (code, r) at byte 256 code + 4 r of a 64 KB slot: one SDWA move
+// forms its address), and four of its entries are an operand.
 //
 //   scores   tile r (tokens 16r .. 16r+15 of the chunk) x 16 columns x 32 k-slots
 //            per MFMA. Row c of
@@ -889,12 +894,15 @@ __device__ __forceinline__ void read_unconditionally(float (&x)[N]) {
   for (int i = 0; i < N; ++i) asm volatile("" : "+v"(x[i]));
 }
 
-// H | L << 16 of x with H = fp16(x) and L = fp16(x - H), both rounded toward zero.
+// H | L << 16 of x with H = fp16(x) and L = fp16(x - H), both rounded to nearest: H + L is
+// x to 2^-22 of itself and without bias (rounded toward zero it is to 2^-20, and every
+// weight and codebook value comes out a little too small: at 8/8 bits, 9,000 tokens, the
+// output's error against float64 was 4.6e-7 of its norm, now 3.8e-7; the fp32-product scan's
+// is 3.6e-7). One conversion instruction per pair either way.
 __device__ __forceinline__ uint32_t split_word(float x) {
-  typedef __fp16 h2 __attribute__((ext_vector_type(2)));
-  const h2 hi = __builtin_amdgcn_cvt_pkrtz(x, 0.f);
-  const float r = x - (float)hi[0];
-  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x, r));
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  const float r = x - float(_Float16(x));
+  return __builtin_bit_cast(uint32_t, h2{_Float16(x), _Float16(r)});
 }
 
 // Table entry of two codebook values: [H(2^8 lo), L(2^8 lo), H(2^8 hi), L(2^8 hi)].
@@ -912,25 +920,78 @@ __device__ __forceinline__ int2 table16_codes(int i) {
   if constexpr (BW == 4) return make_int2((i >> 5) & 15, i >> 9);
   else return make_int2(i & ((1 << BW) - 1), i >> BW);
 }
+// The 8-bit table: 256 entries of 256 B, one word for each lane of a wave. Wave v of the
+// group stages 256 / waves of them: lane l loads code E v + (l mod E), and each b128 store
+// writes four entries' rows, a row's word fetched from the lane that holds it. (A load and
+// a split for every stored word, 64 a thread for 8/8, took 0.8 us longer in a scan of 12
+// heads of at most 300 tokens: 15.4 us against 14.7.)
 template <int BW, int NTHR>
-using Table16Loads = CodePairs<table16_entries<BW>(), NTHR>;
+struct Table16Loads : CodePairs<table16_entries<BW>(), NTHR> {};
+template <int NTHR>
+struct Table16Loads<8, NTHR> {
+  static constexpr int E = 256 / (NTHR / 64);  // entries per wave
+  static_assert(E % 4 == 0 && E <= 64, "a wave's entries: whole b128 stores, one lane each");
+  float v;
+};
 template <int BW, int NTHR>
 __device__ __forceinline__ Table16Loads<BW, NTHR> load_table16(const float* cb, int tid) {
-  static_assert(BW == 4 || pair_coded<BW>(), "16-bit tables are pair tables");
-  return load_code_pairs<table16_entries<BW>(), NTHR>(cb, tid, [](int i) { return table16_codes<BW>(i); });
+  if constexpr (BW == 8) {
+    constexpr int E = Table16Loads<8, NTHR>::E;
+    return {cb[E * (tid >> 6) + (tid & (E - 1))]};
+  } else {
+    static_assert(BW == 4 || pair_coded<BW>(), "16-bit tables are pair tables");
+    return {load_code_pairs<table16_entries<BW>(), NTHR>(cb, tid, [](int i) { return table16_codes<BW>(i); })};
+  }
 }
 template <int BW, int NTHR>
 __device__ __forceinline__ void store_table16(const Table16Loads<BW, NTHR>& p, char* dst, int tid) {
-  store_code_pairs(p, reinterpret_cast<uint2*>(dst), tid, [](float lo, float hi) { return split_pair(lo, hi); });
+  if constexpr (BW == 8) {
+    constexpr int E = Table16Loads<8, NTHR>::E;
+    const int lane = tid & 63, row = lane >> 4;
+    const int v = int(split_word(p.v * kCbScale));
+    uint4* t = reinterpret_cast<uint4*>(dst + 256 * E * (tid >> 6)) + lane;
+#pragma unroll
+    for (int k = 0; k < E / 4; ++k) {
+      const uint32_t x = __shfl(v, 4 * k + row);
+      t[64 * k] = make_uint4(x, x, x, x);
+    }
+  } else {
+    store_code_pairs(p, reinterpret_cast<uint2*>(dst), tid, [](float lo, float hi) { return split_pair(lo, hi); });
+  }
+}
+
+// The 8-bit table as one lane reads it: address registers 4 lane | slot << 16, one per
+// byte position of a code word.
+struct Tab8 {
+  const char* lds;
+  uint32_t r[4];
+};
+template <int K>
+__device__ __forceinline__ uint32_t entry8(Tab8& tab, uint32_t x) {
+  tab.r[K] = put_byte1<K>(tab.r[K], x);
+  return *reinterpret_cast<const uint32_t*>(tab.lds + tab.r[K]);
+}
+
+// The 16-bit scan's table of BW-bit codes at LDS offset off.
+template <int BW>
+using Tab16 = std::conditional_t<BW == 8, Tab8, Tab<BW>>;
+template <int BW>
+__device__ __forceinline__ Tab16<BW> make_tab16(const char* lds, int off, int lane) {
+  if constexpr (BW == 8) {
+    const uint32_t r = uint32_t(4 * lane) | (uint32_t(off >> 16) << 16);
+    return Tab8{lds, {r, r, r, r}};
+  } else {
+    return make_tab<BW>(lds, off, lane);
+  }
 }
 
 // Table reads in flight ahead of their MFMA in the 16-bit scan: eight steps where
 // the widths leave the registers for them (2 and 4 bits, whose pieces are whole
-// bytes), two with a 6-bit side (its kernels sit at 256 VGPRs; fewer reads in flight
-// measured 2 % faster at config 5), else four.
+// bytes), two with a 6 or 8-bit side (their kernels sit at 256 VGPRs; fewer reads in
+// flight measured 2 % faster at config 5), else four.
 template <int BWK, int BWV>
 constexpr int mx_lookahead() {
-  return (BWK == 2 || BWK == 4) && (BWV == 2 || BWV == 4) ? 8 : (BWK == 6 || BWV == 6) ? 2 : 4;
+  return (BWK == 2 || BWK == 4) && (BWV == 2 || BWV == 4) ? 8 : (BWK >= 6 || BWV >= 6) ? 2 : 4;
 }
 
 // Two table entries side by side as an 8-slot operand.
@@ -1048,12 +1109,15 @@ __device__ __forceinline__ void load_k16(const DecodeArgs& a, int kvh, int lane,
             uint32_t((c0 + 16 * t) & smask) * uint32_t(NBK);
     }
     const uint8_t* q = blk + lane_off;
-    if constexpr (QB == 16) {
-      const uint4 x = *reinterpret_cast<const uint4*>(q);
-      r.w[t * QW] = x.x;
-      r.w[t * QW + 1] = x.y;
-      r.w[t * QW + 2] = x.z;
-      r.w[t * QW + 3] = x.w;
+    if constexpr (QB % 16 == 0) {
+#pragma unroll
+      for (int i = 0; i < QB / 16; ++i) {
+        const uint4 x = reinterpret_cast<const uint4*>(q)[i];
+        r.w[t * QW + 4 * i] = x.x;
+        r.w[t * QW + 4 * i + 1] = x.y;
+        r.w[t * QW + 4 * i + 2] = x.z;
+        r.w[t * QW + 4 * i + 3] = x.w;
+      }
     } else if constexpr (QB % 8 == 0) {
 #pragma unroll
       for (int i = 0; i < QB / 8; ++i) {
@@ -1094,7 +1158,7 @@ __device__ __forceinline__ float add_half(float x) {
 // h * kTileStride + 16r + 4g + i; with kTileHalves the part of q' L at word
 // (h + NH) * kTileStride + ...), before the 2^-(e+8) scale.
 template <int BWK, int BWV, int NG>
-__device__ __forceinline__ void score_phase_mx(const RowBuf<BWK, BWV>& K, Tab<BWK>& cbk, const h8 (&qb)[8], int lane,
+__device__ __forceinline__ void score_phase_mx(const RowBuf<BWK, BWV>& K, Tab16<BWK>& cbk, const h8 (&qb)[8], int lane,
                                                uint32_t* pt) {
   constexpr int NH = 4 * NG, QW = BWK, LA = mx_lookahead<BWK, BWV>();
   f32x4 d[4];
@@ -1104,8 +1168,14 @@ __device__ __forceinline__ void score_phase_mx(const RowBuf<BWK, BWV>& K, Tab<BW
   uint2 e[LA + 1][2];
   auto look = [&](auto kc, uint2 (&o)[2]) {
     constexpr int k = decltype(kc)::value, s = k >> 2, r = k & 3;
-    o[0] = piece_pair<BWK, 2 * s>(K.w + r * QW, cbk);
-    o[1] = piece_pair<BWK, 2 * s + 1>(K.w + r * QW, cbk);
+    if constexpr (BWK == 8) {
+      const uint32_t w = K.w[r * QW + s];
+      o[0] = make_uint2(entry8<0>(cbk, w), entry8<1>(cbk, w));
+      o[1] = make_uint2(entry8<2>(cbk, w), entry8<3>(cbk, w));
+    } else {
+      o[0] = piece_pair<BWK, 2 * s>(K.w + r * QW, cbk);
+      o[1] = piece_pair<BWK, 2 * s + 1>(K.w + r * QW, cbk);
+    }
   };
   static_for<0, LA>([&](auto kc) { look(kc, e[decltype(kc)::value]); });
   __builtin_amdgcn_sched_barrier(0);
@@ -1208,17 +1278,22 @@ __device__ __forceinline__ void softmax_phase_mx(float sc, uint32_t nk_h, uint32
 // Values of a chunk: 4 K-steps (16 tokens each) x 8 M-tiles (one dim of each lane's
 // eight), one MFMA each; lookups run LA steps ahead.
 template <int BWK, int BWV, int NG>
-__device__ __forceinline__ void value_phase_mx(RowBuf<BWK, BWV>& V, Tab<BWV>& cbv, const uint32_t* pt, int lane,
+__device__ __forceinline__ void value_phase_mx(RowBuf<BWK, BWV>& V, Tab16<BWV>& cbv, const uint32_t* pt, int lane,
                                                f32x4 (&acc)[8]) {
   constexpr int NH = 4 * NG, VW = VWords<BWV>::N, LA = mx_lookahead<BWK, BWV>();
   const int c = lane & 15, g = lane >> 4;
-  if constexpr (BWV != 4) merge_value_pairs<BWK, BWV>(V, lane);
+  if constexpr (BWV != 4 && BWV != 8) merge_value_pairs<BWK, BWV>(V, lane);
   const uint32_t sel = c < NH ? 0x01000100u : c < 2 * NH ? 0x03020302u : 0x0c0c0c0cu;
   const uint32_t* prow = pt + (c % NH) * kTileStride + 4 * g;
   // step k = 8ks + mt
   auto look = [&](auto kc, uint2 (&o)[2]) {
     constexpr int k = decltype(kc)::value, ks = k >> 3, mt = k & 7;
-    if constexpr (BWV == 4) {
+    if constexpr (BWV == 8) {
+      // code mt of tokens 4ks .. 4ks + 3 of the V buffer, one entry each
+      const uint32_t* w = V.w + 4 * ks * VW + (mt >> 2);
+      o[0] = make_uint2(entry8<mt & 3>(cbv, w[0]), entry8<mt & 3>(cbv, w[VW]));
+      o[1] = make_uint2(entry8<mt & 3>(cbv, w[2 * VW]), entry8<mt & 3>(cbv, w[3 * VW]));
+    } else if constexpr (BWV == 4) {
       // 4-bit: byte mt/2 of the merged bytes of token pairs (0,1), (2,3) of K-step ks
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
@@ -1639,11 +1714,17 @@ __device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh
   else write_partial_mx<NG>(a, st, prow, lane);
 }
 
+// LDS of a work-group: the tables (4 and 8-bit ones in 64 KB slots of their own, slot 1
+// beside a pair-coded table, as in RowsLds), then one tile per wave.
+template <int BW>
+constexpr int table16_bytes() { return BW == 8 ? 256 * 64 * 4 : table_bytes<BW>(); }
 template <int BWK, int BWV, int NG, int WPB>
 struct Rows16Lds {
-  static constexpr int k_off = RowsLds<BWK, BWV, NG, WPB>::k_off;
-  static constexpr int v_off = RowsLds<BWK, BWV, NG, WPB>::v_off;
-  static constexpr int tiles = RowsLds<BWK, BWV, NG, WPB>::tiles;
+  static constexpr bool ks = BWK == 4 || BWK == 8, vs = BWV == 4 || BWV == 8;
+  static constexpr int k_off = ks && !vs ? kPairTableBytes : 0;
+  static constexpr int v_off = vs ? kPairTableBytes : ks ? 0 : table16_bytes<BWK>();
+  static constexpr int k_end = k_off + table16_bytes<BWK>(), v_end = v_off + table16_bytes<BWV>();
+  static constexpr int tiles = k_end > v_end ? k_end : v_end;
   static constexpr int tile_bytes = (kTileHalves<NG> ? 2 : 1) * 4 * NG * kTileStride * 4;
   static constexpr int pace = tiles + WPB * tile_bytes;  // one word per wave (Pace)
   static constexpr int total = pace + 4 * WPB;
@@ -1668,8 +1749,8 @@ __global__ __launch_bounds__(64 * WPB) void decode_rows16_kernel(DecodeArgs a) {
   const Pace pace = make_pace<WPB>(reinterpret_cast<uint32_t*>(lds + Lay::pace), wig);
   __syncthreads();  // the only block-wide barrier: waves run independently from here
   uint32_t* ptile = reinterpret_cast<uint32_t*>(lds + Lay::tiles + wig * Lay::tile_bytes);
-  Tab<BWK> cbk = make_tab<BWK>(lds, Lay::k_off, lane);
-  Tab<BWV> cbv = make_tab<BWV>(lds, Lay::v_off, lane);
+  Tab16<BWK> cbk = make_tab16<BWK>(lds, Lay::k_off, lane);
+  Tab16<BWV> cbv = make_tab16<BWV>(lds, Lay::v_off, lane);
   if (live) {
     rw.run(a, w, lane, [&](int b, int kvh, int t_lo, int t_hi, int64_t prow, uint32_t left) {
       scan_range16<BWK, BWV, NG, false>(a, b, kvh, t_lo, t_hi, prow, lane, cbk, cbv, ptile, pace, left);
@@ -1758,8 +1839,10 @@ SplitKernel rows16_kernel() {
   return k;
 }
 
-// The 16-bit scan's width pairs: pair-table widths (2, 3, 4, 5, 6 bits) alike for K
-// and V, and 4/6, 6/4.
+// The 16-bit scan's width pairs: 2, 3, 4, 5, 6 and 8 bits alike for K and V, 4/6, 6/4
+// and 4/8. 8 bits joined when their table went to single codes: 32 sequences of 1,000 to
+// 4,096 tokens, 28 query heads over 4 kv heads, 8/8, take 34 us in this scan (200 MB at
+// 6 TB/s) against 45 us in the fp32-product one.
 template <int NG>
 SplitKernel rows16_for(int bw_k, int bw_v) {
   if (bw_k == bw_v) {
@@ -1769,7 +1852,10 @@ SplitKernel rows16_for(int bw_k, int bw_v) {
       case 4: return rows16_kernel<4, 4, NG>();
       case 5: return rows16_kernel<5, 5, NG>();
       case 6: return rows16_kernel<6, 6, NG>();
+      case 8: return rows16_kernel<8, 8, NG>();
     }
+  } else if (bw_k == 4 && bw_v == 8) {
+    return rows16_kernel<4, 8, NG>();
   } else if (bw_k == 4 && bw_v == 6) {
     return rows16_kernel<4, 6, NG>();
   } else if (bw_k == 6 && bw_v == 4) {
