@@ -39,11 +39,14 @@ def _float64(q, kv, scale):
     return out, (2 * 2.0 ** -19 * smax + 2.0 ** -17) * vmax
 
 
-@pytest.mark.parametrize("S,Hq,Hkv,bwk,bwv", [(16, 28, 4, 8, 8), (64, 8, 8, 8, 8), (32, 64, 8, 8, 8), (16, 12, 2, 4, 8),
-                                              (128, 4, 2, 4, 8), (16, 28, 4, 4, 4)])
-def test_scan_edges(S, Hq, Hkv, bwk, bwv, D=128):
-    lens = (0, 1, 63, 64, 65, 130, 2049)
-    q, kv = build(700 + S + bwk, len(lens), Hq, Hkv, D, lens, S, bwk, bw_v=bwv)
+@pytest.mark.parametrize("D,S,Hq,Hkv,bwk,bwv", [(128, 16, 28, 4, 8, 8), (128, 64, 8, 8, 8, 8), (128, 32, 64, 8, 8, 8),
+                                                (128, 16, 12, 2, 4, 8), (128, 128, 4, 2, 4, 8), (128, 16, 28, 4, 4, 4),
+                                                # head_dim 64: two tokens to a row, up to four heads of a kv head
+                                                (64, 16, 8, 2, 4, 4), (64, 32, 12, 4, 4, 4), (64, 128, 3, 3, 8, 8),
+                                                (64, 16, 4, 2, 5, 5), (64, 64, 8, 2, 6, 4), (64, 16, 6, 2, 3, 3)])
+def test_scan_edges(D, S, Hq, Hkv, bwk, bwv):
+    lens = (0, 1, 2, 63, 64, 65, 127, 128, 129, 130, 257, 2049)
+    q, kv = build(700 + S + bwk + D, len(lens), Hq, Hkv, D, lens, S, bwk, bw_v=bwv)
     scale = oa.default_scale(D)
     ref, tol = _float64(q, kv, scale)
     from winnow_amd import packed_attention as pa
@@ -55,3 +58,22 @@ def test_scan_edges(S, Hq, Hkv, bwk, bwv, D=128):
         err = float((got - ref).abs().max())
         assert err <= tol, (err, tol)
         assert (got[0] == 0).all()
+
+
+def test_norms_off_the_word(Hq=8, Hkv=2, D=64, S=16):
+    """head_dim 64 reads the norms of two tokens in one word: norms that begin on an odd
+    element, and plans asked for by number, give the same attention."""
+    from winnow_amd import packed_attention as pa
+    lens = (5, 300, 64)
+    q, kv = build(41, len(lens), Hq, Hkv, D, lens, S, 4)
+    scale = oa.default_scale(D)
+    ref, tol = _float64(q, kv, scale)
+    dev = to_device(kv, "cuda")
+    for name in ("k_norms", "v_norms"):
+        n = getattr(dev, name)
+        room = torch.zeros(n.numel() + 1, dtype=n.dtype, device=n.device)
+        room[1:] = n.flatten()
+        setattr(dev, name, room[1:].view(n.shape))
+    for splits in (None, 3):
+        got = pa.packed_decode_attention(q.cuda(), dev, scale, num_splits=splits, out_dtype=torch.float32).cpu().double()
+        assert float((got - ref).abs().max()) <= tol

@@ -6,7 +6,8 @@
 //                        balanced scan partitions by
 //   2. page scan         the row-per-lane matrix-core scan (decode_rows.hip) where
 //                        it applies (head_dim 128, a width pair it compiles, and
-//                        n_rep that 2^s virtual heads per kv head bring to <= 8),
+//                        n_rep that 2^s virtual heads per kv head bring to <= 8;
+//                        head_dim 64 with n_rep <= 4, two tokens to a row),
 //                        else decode_split_kernel (wn_split.h): one work-group per
 //                        (split, kv head, sequence), score phase (lane = token),
 //                        online softmax, value phase (16 lanes per token row),
@@ -15,6 +16,7 @@
 //                        of its partials, 1/l, a Pi_V, cast to the output type
 // Algebra follows turboquant_kv/packed_attention.py:260-334 (the schedule the
 // reference kernel packed_attention_triton.py:51-159 implements).
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <map>
@@ -410,7 +412,7 @@ int valu_groups(int n_rep) {
 // tf32: the TF32-class row scan where it is compiled (4 and 6-bit K and V, alike or
 // mixed, on the row scan: n_rep up to 8, or up to 16 in virtual kv heads of eight),
 // else the same choice as without it.
-SplitKernel choose_scan(int Hq, int Hkv, int D, int S, int bw_k, int bw_v, bool tf32 = false) {
+SplitKernel choose_scan(int Hq, int Hkv, int D, int S, int bw_k, int bw_v, bool tf32 = false, bool norm_words = true) {
   SplitKernel sk;
   const int n_rep = Hq / Hkv;
   const int shift = row_shift(n_rep);
@@ -422,6 +424,12 @@ SplitKernel choose_scan(int Hq, int Hkv, int D, int S, int bw_k, int bw_v, bool 
       sk.kvdiv = 1 << shift;
     }
   }
+  // head_dim 64, two tokens to a row, for up to four heads of a kv head (the scan's eight
+  // columns are heads x 2 tokens), pages of whole blocks of eight rows, and norms that
+  // can be read by the word: 48 us against the vector-ALU scan's 87 with 32 heads over 8
+  // (16 sequences of 3,000 to 12,000 tokens, 4/4 bits), 67 against 84 with 16 over 8
+  // (32 of 8,000, 6/6), level at 300 tokens (40 and 42, host time).
+  if (D == 64 && S >= 16 && norm_words && rows_allowed()) sk = pick_split_pair(bw_k, bw_v, n_rep);
   if (!sk.fn) {
     const int g = valu_groups(n_rep);
     const int nrp = pad_nrep(n_rep / g);
@@ -515,6 +523,20 @@ static void fixed_plan(int B, int units_per_seq, int mp, int* pages_per_split, i
   *num_splits = int((mp + pps - 1) / pps);
 }
 
+// Fixed splits for the row scan of head_dim 64: at most kPairWaves waves, the chip's two
+// per SIMD, each of whole chunks of 128 tokens. Every wave costs about 12 us before its
+// first product, so a second round of them is dear: 2,048 / 3,072 / 4,096 waves take
+// 48 / 53 / 49 us (16 sequences of 3,000 to 12,000 tokens, 8 kv heads) and
+// 67 / 90 / 78 us (32 of 8,000).
+static constexpr int64_t kPairWaves = 2048;
+static void pair_plan(int B, int Hkv, int S, int mp, int* pages_per_split, int* num_splits) {
+  const int64_t units = int64_t(B > 0 ? B : 1) * Hkv, chunk = S < 128 ? 128 / S : 1;
+  const int64_t want = std::max<int64_t>(kPairWaves / units, 1);
+  const int64_t pps = std::min<int64_t>(((mp + want - 1) / want + chunk - 1) / chunk * chunk, mp);
+  *pages_per_split = int(pps);
+  *num_splits = int((mp + pps - 1) / pps);
+}
+
 namespace {
 int decode_plan(int B, int Hq, int Hkv, int D, int S, int bw_k, int bw_v, int max_pages, int requested_splits,
                 int* pages_per_split, int* num_splits, bool tf32) {
@@ -533,6 +555,10 @@ int decode_plan(int B, int Hq, int Hkv, int D, int S, int bw_k, int bw_v, int ma
     return WN_OK;
   }
   const SplitKernel sk = choose_scan(Hq, Hkv, D, S, bw_k, bw_v, tf32);
+  if (sk.pair) {
+    pair_plan(B, Hkv, S, mp, pages_per_split, num_splits);
+    return WN_OK;
+  }
   if (sk.fn && sk.rows) {  // row scan: balanced persistent waves
     const int w = resident_waves(sk);
     WN_REQUIRE(w > 0, WN_E_LAUNCH, "wn_decode_plan: cannot query the device occupancy");
@@ -614,11 +640,13 @@ int decode_attention(
   WN_REQUIRE(k_stride_p >= 0 && k_stride_p < 2 * lim && v_stride_p >= 0 && v_stride_p < 2 * lim, WN_E_INVALID,
              "decode: page strides of 2^32 bytes or more");
 
-  const SplitKernel sk = choose_scan(Hq, Hkv, D, S, bw_k, bw_v, tf32);
+  const bool norm_words = aligned(k_norms, 4) && aligned(v_norms, 4) &&
+                          (kn_stride_p | kn_stride_h | vn_stride_p | vn_stride_h) % 2 == 0;
+  const SplitKernel sk = choose_scan(Hq, Hkv, D, S, bw_k, bw_v, tf32, norm_words);
   RotFn rot = pick_rot_d(D, max(sk.nrep, 1));
   WN_REQUIRE(sk.fn && rot, WN_E_UNSUPPORTED, "decode: (D=%d, bw_k=%d, bw_v=%d) not compiled", D, bw_k,
              bw_v);
-  WN_REQUIRE(!balanced || sk.rows, WN_E_INVALID,
+  WN_REQUIRE(!balanced || (sk.rows && !sk.pair), WN_E_INVALID,
              "decode: a balanced plan (pages_per_split 0) needs the row scan; ask wn_decode_plan");
 
   const WsLayout lay = ws_layout(B, Hq, Hkv, D, pages_per_split, num_splits);

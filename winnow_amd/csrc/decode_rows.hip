@@ -36,6 +36,7 @@
 // computes.
 // Algebra: turboquant_kv/packed_attention.py:260-334 (the schedule of the
 // reference kernel packed_attention_triton.py:51-134).
+#include <cfloat>
 #include <cstdlib>
 #include <cstring>
 #include <type_traits>
@@ -284,7 +285,7 @@ __device__ __forceinline__ const uint8_t* global_ptr(uint64_t x) {
 // 8p..8p+7 of token c0+4q+G (G = lane/16, p = lane%16). c0 is a multiple of 16 and
 // pages hold >= 16 tokens, so the four quads of 16-token block j share the page of
 // lane 16j (pid_lane is the page of token c0+lane).
-template <int BWK, int BWV, bool RAW = false>
+template <int BWK, int BWV, bool RAW = false, bool PAIR = false>
 __device__ __forceinline__ void load_v(const DecodeArgs& a, int kvh, int lane, int c0, int pid_lane,
                                        RowBuf<BWK, BWV>& r, bool live = true, const uint64_t* ba = nullptr) {
   constexpr int NBV = 16 * BWV, VW = RowBuf<BWK, BWV>::VW;
@@ -298,7 +299,7 @@ __device__ __forceinline__ void load_v(const DecodeArgs& a, int kvh, int lane, i
     constexpr int j = decltype(jc)::value;
     const uint8_t* blk;
     if (ba) {  // the block's address, formed by block_bases
-      blk = global_ptr(ba[j]);
+      blk = global_ptr(ba[PAIR ? 2 * j : j]);
     } else {
       const uint32_t pid_j = __builtin_amdgcn_readlane(pid_lane, 16 * j);  // a live page id, >= 0
       blk = a.v_pages + uint64_t(pid_j) * uint64_t(a.vsp) + (kvh >> a.kvshift) * a.vsh +
@@ -308,7 +309,8 @@ __device__ __forceinline__ void load_v(const DecodeArgs& a, int kvh, int lane, i
     static_for<0, 4>([&](auto qc) {
       constexpr int qq = decltype(qc)::value;
       uint32_t t[VW];
-      load_vcodes<BWV, RAW>(vj + 4 * qq * NBV, p & 1, t);
+      if constexpr (PAIR && qq >= 2) load_vcodes<BWV, RAW>(global_ptr(ba[2 * j + 1]) + lane_off + 4 * (qq - 2) * NBV, p & 1, t);
+      else load_vcodes<BWV, RAW>(vj + 4 * qq * NBV, p & 1, t);
 #pragma unroll
       for (int x = 0; x < VW; ++x) r.w[(4 * j + qq) * VW + x] = t[x];
     });
@@ -1073,15 +1075,16 @@ __device__ __forceinline__ int tile_token(int c) { return 4 * (c & 3) + (c >> 2)
 // 64-bit multiply-adds (page id x page stride, slot x row bytes; base = the pages plus
 // the kv head's offset) and the blocks' addresses are read from lanes 0, 16, 32 and 48.
 // Page strides are below 2^32 bytes (checked on the host).
-template <int NB>
+// N = 8: of its eight 8-row blocks, for rows of two tokens (a 16-token page holds eight).
+template <int NB, int N = 4>
 __device__ __forceinline__ void block_bases(uint64_t base, uint32_t sp, int pid, int c0, int lane, int smask,
-                                            uint64_t (&out)[4]) {
-  const uint32_t slot = uint32_t((c0 + lane) & smask) & ~15u;
+                                            uint64_t (&out)[N]) {
+  const uint32_t slot = uint32_t((c0 + lane) & smask) & ~uint32_t(64 / N - 1);
   const uint64_t x = base + uint64_t(uint32_t(pid)) * sp + uint64_t(slot * uint32_t(NB));
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(x), 16 * t);
-    const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(x >> 32), 16 * t);
+  for (int t = 0; t < N; ++t) {
+    const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(x), 64 / N * t);
+    const uint32_t hi = __builtin_amdgcn_readlane(uint32_t(x >> 32), 64 / N * t);
     out[t] = uint64_t(hi) << 32 | lo;
   }
 }
@@ -1089,7 +1092,7 @@ __device__ __forceinline__ void block_bases(uint64_t base, uint32_t sp, int pid,
 // K side of chunk [c0, c0+64) for the 16-bit scan: quarter g of the rows of the
 // tile tokens (one whole 16-token page block per load instruction) and both norms of
 // token c0 + lane, whose page is pid_lane.
-template <int BWK, int BWV>
+template <int BWK, int BWV, bool PAIR = false>
 __device__ __forceinline__ void load_k16(const DecodeArgs& a, int kvh, int lane, int c0, int pid_lane,
                                          RowBuf<BWK, BWV>& r, bool live = true, const uint64_t* ba = nullptr) {
   constexpr int NBK = 16 * BWK, QB = 4 * BWK, QW = BWK, KW = RowBuf<BWK, BWV>::KW;
@@ -1097,12 +1100,13 @@ __device__ __forceinline__ void load_k16(const DecodeArgs& a, int kvh, int lane,
   // the tile's 16 tokens share a page (c0 + 16t is a multiple of 16 and S >= 16): a
   // wave-uniform block base plus this lane's fixed 32-bit offset in it (0 when the
   // chunk is past the range, as in load_v)
-  const uint32_t lane_off = live ? uint32_t(tile_token(lane & 15) * NBK + QB * (lane >> 4)) : 0u;
+  const int row = tile_token(lane & 15);
+  const uint32_t lane_off = live ? uint32_t((PAIR ? row & 7 : row) * NBK + QB * (lane >> 4)) : 0u;
   static_for<0, 4>([&](auto rc) {
     constexpr int t = decltype(rc)::value;
     const uint8_t* blk;
     if (ba) {  // the block's address, formed by block_bases
-      blk = global_ptr(ba[t]);
+      blk = global_ptr(!PAIR ? ba[t] : row < 8 ? ba[2 * t] : ba[2 * t + 1]);
     } else {
       const uint32_t pid_t = __builtin_amdgcn_readlane(pid_lane, 16 * t);  // a live page id, >= 0
       blk = a.k_pages + uint64_t(pid_t) * uint64_t(a.ksp) + (kvh >> a.kvshift) * a.ksh +
@@ -1132,8 +1136,14 @@ __device__ __forceinline__ void load_k16(const DecodeArgs& a, int kvh, int lane,
   });
   // page ids are >= 0 and the norm strides below 2^31 (checked on the host): one
   // 32 x 32 -> 64-bit multiply-add per offset
-  const uint32_t slot = uint32_t((c0 + lane) & smask);
   const uint32_t pid = uint32_t(pid_lane), kvr = uint32_t(kvh >> a.kvshift);
+  if constexpr (PAIR) {  // the two tokens' norms in one word (4-byte aligned: checked on the host)
+    const uint32_t slot = uint32_t(2 * (c0 + lane)) & uint32_t(smask);
+    r.w[KW] = *reinterpret_cast<const uint32_t*>(a.k_norms + (uint64_t(pid) * uint32_t(a.knp) + (kvr * uint32_t(a.knh) + slot)));
+    r.w[KW + 1] = *reinterpret_cast<const uint32_t*>(a.v_norms + (uint64_t(pid) * uint32_t(a.vnp) + (kvr * uint32_t(a.vnh) + slot)));
+    return;
+  }
+  const uint32_t slot = uint32_t((c0 + lane) & smask);
   r.w[KW] = a.k_norms[uint64_t(pid) * uint32_t(a.knp) + (kvr * uint32_t(a.knh) + slot)];
   r.w[KW + 1] = a.v_norms[uint64_t(pid) * uint32_t(a.vnp) + (kvr * uint32_t(a.vnh) + slot)];
 }
@@ -1207,20 +1217,29 @@ __device__ __forceinline__ void score_phase_mx(const RowBuf<BWK, BWV>& K, Tab16<
 
 // Online softmax of one chunk (lane = token) from the score tile; p n_V 2^-gs goes
 // back to the same words as H | L << 16.
-template <int NG>
-__device__ __forceinline__ void softmax_phase_mx(float sc, uint32_t nk_h, uint32_t nv_h, bool valid, int lane,
+template <int NG, bool PAIR = false>
+__device__ __forceinline__ void softmax_phase_mx(float sc, uint32_t nk_h, uint32_t nv_h, int left, int lane,
                                                  uint32_t* pt, MxState<NG>& st) {
   constexpr int H = 4 * NG;
   const int off = 16 * (lane >> 4) + 4 * (lane & 3) + ((lane >> 2) & 3);  // word of token lane
-  const float nk = half_lo(nk_h) * sc;
-  const float nv = valid ? half_lo(nv_h) : 0.f;
+  // head i weighs token T of this lane, T = 0 except for PAIR's second four heads
+  constexpr int NT = PAIR ? 2 : 1;
+  bool valid[NT];
+  float nk[NT], nvt[NT], nv = 0.f;
+#pragma unroll
+  for (int T = 0; T < NT; ++T) {
+    valid[T] = left > T;
+    nk[T] = half_lo(nk_h >> (16 * T)) * sc;
+    nvt[T] = valid[T] ? half_lo(nv_h >> (16 * T)) : 0.f;
+    nv = T ? fmaxf(nv, nvt[T]) : nvt[T];
+  }
   float sv[H];
   if constexpr (kTileHalves<NG>) {
 #pragma unroll
     for (int i = 0; i < H; ++i) {
       const float x = __builtin_bit_cast(float, pt[i * kTileStride + off]) +
                       __builtin_bit_cast(float, pt[(i + H) * kTileStride + off]);
-      sv[i] = valid ? x * nk : -INFINITY;
+      sv[i] = valid[PAIR ? i / 4 : 0] ? x * nk[PAIR ? i / 4 : 0] : -INFINITY;
     }
   } else {
     float x[H];
@@ -1228,7 +1247,7 @@ __device__ __forceinline__ void softmax_phase_mx(float sc, uint32_t nk_h, uint32
     for (int i = 0; i < H; ++i) x[i] = __builtin_bit_cast(float, pt[i * kTileStride + off]);
     read_unconditionally(x);
 #pragma unroll
-    for (int i = 0; i < H; ++i) sv[i] = valid ? x[i] * nk : -INFINITY;
+    for (int i = 0; i < H; ++i) sv[i] = valid[PAIR ? i / 4 : 0] ? x[i] * nk[PAIR ? i / 4 : 0] : -INFINITY;
   }
   // value scale: 2^kRescale * max(n_V) * 2^-gs < 2^15, i.e. every n_V < 2^(7 + gs); the
   // scale only grows, so the wave's maximum is taken only when a norm reaches the limit
@@ -1255,7 +1274,9 @@ __device__ __forceinline__ void softmax_phase_mx(float sc, uint32_t nk_h, uint32
     float alpha_c = 1.f;
 #pragma unroll
     for (int i = 0; i < H; ++i) {
-      const float m_new = fmaxf(st.m[i], wave_max_dpp(sv[i]));
+      float m_new = fmaxf(st.m[i], wave_max_dpp(sv[i]));
+      // a range of one token has none of PAIR's second heads': finite, so their weights are 0
+      if constexpr (PAIR) m_new = fmaxf(m_new, -FLT_MAX);
       const float alpha = __builtin_amdgcn_exp2f(st.m[i] - m_new);  // 0 on the first chunk
       st.m[i] = m_new;
       st.l[i] *= alpha;
@@ -1265,12 +1286,14 @@ __device__ __forceinline__ void softmax_phase_mx(float sc, uint32_t nk_h, uint32
 #pragma unroll
     for (int mm = 0; mm < 8; ++mm) st.acc[mm] *= alpha_c;
   }
-  const float nvs = ldexpf(nv, -st.gs);
+  float nvs[NT];
+#pragma unroll
+  for (int T = 0; T < NT; ++T) nvs[T] = ldexpf(nvt[T], -st.gs);
 #pragma unroll
   for (int i = 0; i < H; ++i) {
     const float p = __builtin_amdgcn_exp2f(d[i]);  // 0 for masked tokens
     st.l[i] += p;
-    pt[i * kTileStride + off] = split_word(p * nvs);
+    pt[i * kTileStride + off] = split_word(p * nvs[PAIR ? i / 4 : 0]);
   }
   wave_lds_sync();
 }
@@ -1593,20 +1616,69 @@ __device__ __forceinline__ void write_partial_mx(const DecodeArgs& a, MxState<NG
   }
 }
 
+// The partial of a PAIR range: head h's two halves, (even tokens) virtual head h in rows
+// of lane groups 0 and 1 and (odd tokens) virtual head 4 + h in groups 2 and 3, brought to
+// the larger maximum and added: one 64-dim partial row a head, as the merge expects.
+__device__ __forceinline__ void write_partial_pair(const DecodeArgs& a, MxState<2>& st, int64_t prow, int lane) {
+  constexpr int D = 64;
+  const float f = ldexpf(1.f, st.gs - 8);
+  const int c = lane & 15, g = lane >> 4;
+  float m[4], l[4], w0 = 0.f, w1 = 0.f;
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    m[h] = fmaxf(st.m[h], st.m[4 + h]);
+    const float e0 = __builtin_amdgcn_exp2f(st.m[h] - m[h]), e1 = __builtin_amdgcn_exp2f(st.m[4 + h] - m[h]);
+    l[h] = wave_sum(st.l[h]) * e0 + wave_sum(st.l[4 + h]) * e1;
+    w0 = (c & 3) == h ? e0 * f : w0;
+    w1 = (c & 3) == h ? e1 * f : w1;
+  }
+  const int64_t row0 = prow * a.n_rep;
+#pragma unroll
+  for (int mm = 0; mm < 8; ++mm)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float x = add_half<8>(st.acc[mm][i]);
+      st.acc[mm][i] = x * w0 + __shfl(x, (lane + 36) & 63) * w1;
+    }
+  if (g < 2 && c < a.n_rep) {
+    float* dst = a.part_acc + (row0 + c) * D + 32 * g;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      *reinterpret_cast<float4*>(dst + 8 * i) = make_float4(st.acc[0][i], st.acc[1][i], st.acc[2][i], st.acc[3][i]);
+      *reinterpret_cast<float4*>(dst + 8 * i + 4) = make_float4(st.acc[4][i], st.acc[5][i], st.acc[6][i], st.acc[7][i]);
+    }
+  }
+  if (lane == 0) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      if (h < a.n_rep) {
+        a.part_ml[2 * (row0 + h)] = m[h];
+        a.part_ml[2 * (row0 + h) + 1] = l[h];
+      }
+    }
+  }
+}
+
 // scan_range on the 16x16x32 fp16 MFMA; TF: the TF32-class products (4 or 6-bit
 // codes, TabTf tables). left_after: the wave's chunks after this range (pacing).
-template <int BWK, int BWV, int NG, bool TF, class TabK, class TabV>
-__device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh, int t_lo, int t_hi, int64_t prow,
+template <int BWK, int BWV, int NG, bool TF, bool PAIR, class TabK, class TabV>
+__device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh, int t_lo, int tok_hi, int64_t prow,
                                              int lane, TabK& cbk, TabV& cbv, uint32_t* ptile, const Pace& pace,
                                              uint32_t left_after) {
   static_assert(!TF || ((BWK == 4 || BWK == 6) && (BWV == 4 || BWV == 6)), "TF32-class scan: 4 or 6-bit K and V");
+  static_assert(!PAIR || (NG == 2 && !TF), "row pairs: two head groups of the 16-bit scan");
   constexpr int D = 128, NH = 4 * NG;
-  const int page_hi = (t_hi + (1 << a.log2S) - 1) >> a.log2S;
+  // rows of 128 codes: t_lo, t_hi and page slots below count rows, a token each or (PAIR)
+  // two; a range starts at a page, so at an even token
+  const int log2S = PAIR ? a.log2S - 1 : a.log2S;
+  const int t_hi = PAIR ? (tok_hi + 1) >> 1 : tok_hi;
+  if constexpr (PAIR) t_lo >>= 1;
+  const int page_hi = (t_hi + (1 << log2S) - 1) >> log2S;
   const int n = (t_hi - t_lo + 63) >> 6;
   const int c = lane & 15, g = lane >> 4;
   const int32_t* trow = a.table + b * a.tsb;
   auto pid_of = [&](int ch) {
-    const int col = min((t_lo + 64 * ch + lane) >> a.log2S, page_hi - 1);
+    const int col = min((t_lo + 64 * ch + lane) >> log2S, page_hi - 1);
     return trow[col];
   };
   // the first two chunks' page ids are loaded together with the query below
@@ -1618,11 +1690,15 @@ __device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh
   float qv[32];
   float amax = 0.f;
   {
+    // PAIR: virtual head 4 T + h is head h over the row's token T, so its query is zero
+    // in the other token's half of the row
     const float4* qp = reinterpret_cast<const float4*>(
-        a.q_rot + ((int64_t(b) * a.Hkv + kvh) * NH + (c % NH)) * D + 32 * g);
+        PAIR ? a.q_rot + ((int64_t(b) * a.Hkv + kvh) * 4 + (c & 3)) * 64 + 32 * (g & 1)
+             : a.q_rot + ((int64_t(b) * a.Hkv + kvh) * NH + (c % NH)) * D + 32 * g);
+    const bool other = PAIR && ((c >> 2) & 1) != (g >> 1);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
-      const float4 x = qp[s];
+      const float4 x = other ? make_float4(0.f, 0.f, 0.f, 0.f) : qp[s];
       qv[4 * s] = x.x;
       qv[4 * s + 1] = x.y;
       qv[4 * s + 2] = x.z;
@@ -1660,7 +1736,7 @@ __device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh
   }
   st.gs = 0;
   using Buf = RowBuf<BWK, BWV>;
-  const int smask = (1 << a.log2S) - 1;
+  const int smask = (1 << log2S) - 1;
   const uint64_t kbase = uint64_t(a.k_pages) + uint64_t(kvh >> a.kvshift) * uint64_t(a.ksh);
   const uint64_t vbase = uint64_t(a.v_pages) + uint64_t(kvh >> a.kvshift) * uint64_t(a.vsh);
   int pid_next;
@@ -1669,6 +1745,7 @@ __device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh
   // on only some paths, the compiler's wait counts for a chunk's rows would have to
   // cover the paths that skipped them, and each step would wait for every load in
   // flight, the next chunk's V rows included, before it could start.
+  constexpr int NB = PAIR ? 8 : 4;  // blocks of 16 rows, or of 8 (half a page at S = 16)
   auto step = [&](int ch, Buf& X, Buf& Y, Buf& Z) {
     const int c0 = t_lo + 64 * ch;
     const int pid_after = pid_of(ch + 2);
@@ -1677,18 +1754,18 @@ __device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh
     pace.publish(left);
     const uint32_t partner_left = pace.partner_left();
     // addresses of the next chunk's four 16-token blocks, for its K and its V rows
-    uint64_t kb[4], vb[4];
-    block_bases<16 * BWK>(kbase, uint32_t(a.ksp), pid_next, c0 + 64, lane, smask, kb);
-    load_k16(a, kvh, lane, c0 + 64, pid_next, Z, more, kb);
+    uint64_t kb[NB], vb[NB];
+    block_bases<16 * BWK, NB>(kbase, uint32_t(a.ksp), pid_next, c0 + 64, lane, smask, kb);
+    load_k16<BWK, BWV, PAIR>(a, kvh, lane, c0 + 64, pid_next, Z, more, kb);
     if constexpr (TF) {
       score_phase_tf<BWK, BWV, NG>(X, cbk, qb, lane, ptile);
       softmax_phase_tf<NG>(sc, X.w[Buf::KW], X.w[Buf::KW + 1], c0 + lane < t_hi, lane, ptile, st);
     } else {
       score_phase_mx<BWK, BWV, NG>(X, cbk, qb, lane, ptile);
-      softmax_phase_mx<NG>(sc, X.w[Buf::KW], X.w[Buf::KW + 1], c0 + lane < t_hi, lane, ptile, st);
+      softmax_phase_mx<NG, PAIR>(sc, X.w[Buf::KW], X.w[Buf::KW + 1], tok_hi - (PAIR ? 2 : 1) * (c0 + lane), lane, ptile, st);
     }
-    block_bases<16 * BWV>(vbase, uint32_t(a.vsp), pid_next, c0 + 64, lane, smask, vb);
-    load_v<BWK, BWV, kRawV<BWV>>(a, kvh, lane, c0 + 64, pid_next, X, more, vb);
+    block_bases<16 * BWV, NB>(vbase, uint32_t(a.vsp), pid_next, c0 + 64, lane, smask, vb);
+    load_v<BWK, BWV, kRawV<BWV>, PAIR>(a, kvh, lane, c0 + 64, pid_next, X, more, vb);
     if constexpr (TF) value_phase_tf<BWK, BWV, NG>(Y, cbv, ptile, lane, st.acc);
     else value_phase_mx<BWK, BWV, NG>(Y, cbv, ptile, lane, st.acc);
     pid_next = pid_after;
@@ -1696,8 +1773,16 @@ __device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh
   };
 
   Buf b0, b1, b2;
-  load_k16(a, kvh, lane, t_lo, pid0, b0);
-  load_v<BWK, BWV, kRawV<BWV>>(a, kvh, lane, t_lo, pid0, b1);
+  if constexpr (PAIR) {
+    uint64_t kb[NB], vb[NB];
+    block_bases<16 * BWK, NB>(kbase, uint32_t(a.ksp), pid0, t_lo, lane, smask, kb);
+    block_bases<16 * BWV, NB>(vbase, uint32_t(a.vsp), pid0, t_lo, lane, smask, vb);
+    load_k16<BWK, BWV, true>(a, kvh, lane, t_lo, pid0, b0, true, kb);
+    load_v<BWK, BWV, kRawV<BWV>, true>(a, kvh, lane, t_lo, pid0, b1, true, vb);
+  } else {
+    load_k16(a, kvh, lane, t_lo, pid0, b0);
+    load_v<BWK, BWV, kRawV<BWV>>(a, kvh, lane, t_lo, pid0, b1);
+  }
   pid_next = pid1;
   wait_vmem_all();
   // whole turns of the three buffers in a loop without early exits (a loop header
@@ -1711,6 +1796,7 @@ __device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh
   if (ch < n) step(ch, b0, b1, b2);
   if (ch + 1 < n) step(ch + 1, b2, b0, b1);
   if constexpr (TF) write_partial_tf<NG>(a, st, prow, lane);
+  else if constexpr (PAIR) write_partial_pair(a, st, prow, lane);
   else write_partial_mx<NG>(a, st, prow, lane);
 }
 
@@ -1731,7 +1817,11 @@ struct Rows16Lds {
   static_assert(total <= 160 * 1024, "LDS of a work-group exceeds 160 KB");
 };
 
-template <int BWK, int BWV, int NG, int WPB>
+// PAIR: head_dim 64 as rows of 128 codes, two tokens to a row (they lie side by side in a
+// page), for up to four heads of a kv head: the two head groups are the heads over the
+// row's first and second token, with queries that are zero in the other half. Everything
+// up to a range's partial is the scan of a 128-wide head of eight heads.
+template <int BWK, int BWV, int NG, int WPB, bool PAIR>
 __global__ __launch_bounds__(64 * WPB) void decode_rows16_kernel(DecodeArgs a) {
   using Lay = Rows16Lds<BWK, BWV, NG, WPB>;
   __shared__ __align__(16) char lds[Lay::total];
@@ -1753,7 +1843,7 @@ __global__ __launch_bounds__(64 * WPB) void decode_rows16_kernel(DecodeArgs a) {
   Tab16<BWV> cbv = make_tab16<BWV>(lds, Lay::v_off, lane);
   if (live) {
     rw.run(a, w, lane, [&](int b, int kvh, int t_lo, int t_hi, int64_t prow, uint32_t left) {
-      scan_range16<BWK, BWV, NG, false>(a, b, kvh, t_lo, t_hi, prow, lane, cbk, cbv, ptile, pace, left);
+      scan_range16<BWK, BWV, NG, false, PAIR>(a, b, kvh, t_lo, t_hi, prow, lane, cbk, cbv, ptile, pace, left);
     });
   }
   pace.publish(0);
@@ -1782,7 +1872,7 @@ __global__ __launch_bounds__(64 * WPB) void decode_rows_tf_kernel(DecodeArgs a) 
   TabTf<BWV> cbv = make_tab_tf<BWV>(lds, Lay::v_off, lane);
   if (live) {
     rw.run(a, w, lane, [&](int b, int kvh, int t_lo, int t_hi, int64_t prow, uint32_t left) {
-      scan_range16<BWK, BWV, NG, true>(a, b, kvh, t_lo, t_hi, prow, lane, cbk, cbv, ptile, pace, left);
+      scan_range16<BWK, BWV, NG, true, false>(a, b, kvh, t_lo, t_hi, prow, lane, cbk, cbv, ptile, pace, left);
     });
   }
   pace.publish(0);
@@ -1826,14 +1916,15 @@ SplitKernel rows_for(int bw_k, int bw_v) {
   return SplitKernel{};
 }
 
-template <int BWK, int BWV, int NG>
+template <int BWK, int BWV, int NG, bool PAIR>
 SplitKernel rows16_kernel() {
   constexpr int wpb = 8;  // two waves per SIMD: the 16-bit scan needs up to 256 VGPRs
   SplitKernel k;
-  k.fn = decode_rows16_kernel<BWK, BWV, NG, wpb>;
+  k.fn = decode_rows16_kernel<BWK, BWV, NG, wpb, PAIR>;
   k.block = 64 * wpb;
   k.wpb = wpb;
-  k.nrep = 4 * NG;
+  k.nrep = PAIR ? 4 : 4 * NG;
+  k.pair = PAIR;
   k.log2_units = true;
   k.rows = true;
   return k;
@@ -1843,23 +1934,23 @@ SplitKernel rows16_kernel() {
 // and 4/8. 8 bits joined when their table went to single codes: 32 sequences of 1,000 to
 // 4,096 tokens, 28 query heads over 4 kv heads, 8/8, take 34 us in this scan (200 MB at
 // 6 TB/s) against 45 us in the fp32-product one.
-template <int NG>
+template <int NG, bool PAIR = false>
 SplitKernel rows16_for(int bw_k, int bw_v) {
   if (bw_k == bw_v) {
     switch (bw_k) {
-      case 2: return rows16_kernel<2, 2, NG>();
-      case 3: return rows16_kernel<3, 3, NG>();
-      case 4: return rows16_kernel<4, 4, NG>();
-      case 5: return rows16_kernel<5, 5, NG>();
-      case 6: return rows16_kernel<6, 6, NG>();
-      case 8: return rows16_kernel<8, 8, NG>();
+      case 2: return rows16_kernel<2, 2, NG, PAIR>();
+      case 3: return rows16_kernel<3, 3, NG, PAIR>();
+      case 4: return rows16_kernel<4, 4, NG, PAIR>();
+      case 5: return rows16_kernel<5, 5, NG, PAIR>();
+      case 6: return rows16_kernel<6, 6, NG, PAIR>();
+      case 8: return rows16_kernel<8, 8, NG, PAIR>();
     }
   } else if (bw_k == 4 && bw_v == 8) {
-    return rows16_kernel<4, 8, NG>();
+    return rows16_kernel<4, 8, NG, PAIR>();
   } else if (bw_k == 4 && bw_v == 6) {
-    return rows16_kernel<4, 6, NG>();
+    return rows16_kernel<4, 6, NG, PAIR>();
   } else if (bw_k == 6 && bw_v == 4) {
-    return rows16_kernel<6, 4, NG>();
+    return rows16_kernel<6, 4, NG, PAIR>();
   }
   return SplitKernel{};
 }
@@ -1906,6 +1997,11 @@ SplitKernel pick_split_rows_tf(int bw_k, int bw_v, int n_rep) {
   const int ng = n_rep >= 1 && n_rep <= 4 ? 1 : n_rep >= 5 && n_rep <= 8 ? 2 : 0;
   if (ng == 0 || !rows16_allowed()) return SplitKernel{};
   return ng == 1 ? rows_tf_for<1>(bw_k, bw_v) : rows_tf_for<2>(bw_k, bw_v);
+}
+
+SplitKernel pick_split_pair(int bw_k, int bw_v, int n_rep) {
+  if (n_rep < 1 || n_rep > 4 || !rows16_allowed()) return SplitKernel{};
+  return rows16_for<2, true>(bw_k, bw_v);
 }
 
 SplitKernel pick_split_rows(int bw_k, int bw_v, int n_rep) {

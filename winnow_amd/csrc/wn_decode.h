@@ -37,7 +37,8 @@ struct SplitKernel {
   int wpb = 1;    // independent waves per work-group (row scan); grid counts waves / wpb
   int nrep = 0;   // query-head rows per kv head the kernel reads from q_rot
   bool log2_units = false;  // scores/maxima in log2 units (q_rot scaled by log2 e)
-  bool rows = false;        // the row-per-lane matrix-core scan (balanced plans allowed)
+  bool rows = false;        // the row-per-lane matrix-core scan (balanced plans allowed unless pair)
+  bool pair = false;        // row scan of head_dim 64, two tokens to a row: fixed plans
   int kvshift = 0;          // row scan: each kv head runs as 2^kvshift virtual heads of n_rep >> kvshift
   int kvdiv = 1;            // virtual heads per kv head (1 << kvshift on the row scan)
 };
@@ -48,6 +49,11 @@ struct SplitKernel {
 // splits or balanced persistent waves), or an empty SplitKernel when
 // (bw_k, bw_v, n_rep) is not compiled.
 SplitKernel pick_split_rows(int bw_k, int bw_v, int n_rep);
+
+// The 16-bit row scan of head_dim 64, page sizes >= 16, up to four query heads per kv
+// head and fixed plans, or an empty SplitKernel. It reads two norms in one word: norm
+// bases 4-byte aligned, norm strides even.
+SplitKernel pick_split_pair(int bw_k, int bw_v, int n_rep);
 
 // The TF32-class row scan (single fp16 operands, fp32 accumulation; allow_tf32) for
 // 4 and 6-bit K and V (alike or mixed) and up to eight query heads per kv head, or an
