@@ -250,7 +250,22 @@ class TQPackedLayer(DynamicLayer):
         return (ok, ov) if exact else (ok.to(self.dtype), ov.to(self.dtype))
 
     # ---------------------------------------------------------------- cache protocol
+    def _check_step(self, k: torch.Tensor, v: torch.Tensor) -> None:
+        """The kernels address the buffers by K's sizes: K and V have one shape, the buffers'
+        batch, heads and head_dim (``reset`` keeps the buffers), and lie on their device."""
+        if k.dim() != 4 or v.shape != k.shape:
+            raise ValueError(f"TQPackedLayer: K {tuple(k.shape)} and V {tuple(v.shape)} must be (B, H, n, D) alike")
+        if v.device != k.device:
+            raise ValueError(f"TQPackedLayer: K on {k.device}, V on {v.device}")
+        if not self.is_initialized:
+            return
+        if (k.shape[0], k.shape[1], k.shape[3]) != self._dims:
+            raise ValueError(f"TQPackedLayer: K and V {tuple(k.shape)} do not fit a cache of (B, H, D) = {self._dims}")
+        if k.device != self.device:
+            raise ValueError(f"TQPackedLayer: K and V on {k.device}, the cache on {self.device}")
+
     def update(self, key_states, value_states, *args, **kwargs):
+        self._check_step(key_states, value_states)
         if not self.is_initialized:
             self.lazy_initialization(key_states, value_states)
         n = key_states.shape[-2]
