@@ -151,3 +151,17 @@ def test_pages(D, bw):
             nrm = dkv.v_norms[dkv.page_table[b, :-(-L // 16)].long()].transpose(0, 1).reshape(2, -1)[:, :L]
             want = _closed(unpack(rows.contiguous(), bw, D), nrm, dkv.v_quant)
             assert ((one.double() - want).abs() <= 2e-6 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("D,bw", [(64, 4), (32, 5)])
+def test_pages_of_whole_sequences(D, bw):
+    """Without lengths every sequence has Lpad rows, each through its own table row."""
+    from winnow_amd import packed_backend as pb
+    B, L = 3, 50
+    _, kv = build(600 + D, B, 4, 2, D, (L,) * B, 16, bw)
+    dkv = to_device(kv, DEV)
+    side = (dkv.k_pages, dkv.k_norms, dkv.k_quant)
+    got = torch.empty(B, 2, L, D, device=DEV)
+    pb._dequantize_pages(dkv, *side, dkv.page_table, None, L, got)
+    for b in range(B):
+        assert torch.equal(got[b], pb.dequantize_history(dkv, *side, b, torch.float32)[0])

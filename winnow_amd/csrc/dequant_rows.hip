@@ -54,7 +54,7 @@ struct RowsArgs {
   int64_t plane_rows;    // rows between planes in codes and norms
   // pages (group 0 only, table not null): plane = sequence H + head
   const int32_t* table;
-  const int32_t* lens;   // null: one sequence
+  const int32_t* lens;   // null: every sequence has L rows
   int64_t tsb, psp, psh, nsp, nsh;
   uint32_t H;
   int log2S, D, out_dtype, vec;
@@ -108,13 +108,10 @@ __global__ __launch_bounds__(64 * RowsShape<KD>::W) void dequant_rows_kernel(Row
       uint32_t plane = rc / a.L, t = rc % a.L;
       int64_t o, no;
       if (a.table) {
-        const int32_t* trow = a.table;
-        if (a.lens) {  // rows past a length repeat the last one
-          const uint32_t b = plane / a.H;
-          plane -= b * a.H;
-          t = min(t, uint32_t(max(a.lens[b], 1) - 1));
-          trow += b * a.tsb;
-        }
+        const uint32_t b = plane / a.H;
+        plane -= b * a.H;
+        if (a.lens) t = min(t, uint32_t(max(a.lens[b], 1) - 1));  // rows past a length repeat the last one
+        const int32_t* trow = a.table + b * a.tsb;
         const int64_t page = max(trow[t >> a.log2S], 0), slot = t & ((1u << a.log2S) - 1u);
         o = page * a.psp + plane * a.psh + slot * a.grp[0].nb;
         no = page * a.nsp + plane * a.nsh + slot;
