@@ -101,3 +101,46 @@ def test_reconstruct_route_with_and_without_the_operator(D, bw):
     assert torch.allclose(got.float(), want.float(), atol=2e-2 * want.abs().max().item(), rtol=2e-2)
     want.float().sum().backward()
     assert torch.isfinite(wanted.grad).all()
+
+
+def test_a_trace_is_refused():
+    """The histories come through the C ABI, which no trace records: a traced step raises
+    where the library's operator is reached, it does not leave a graph without the attention."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from winnow_amd import packed_backend as pb
+    lens = (100, 3, 250)
+    _, kv = build(500, len(lens), 8, 2, 64, lens, 16, 4)
+    dkv = to_device(kv, DEV)
+    q = torch.randn(3, 8, 5, 64, generator=torch.Generator().manual_seed(2)).to(DEV, torch.bfloat16)
+
+    def step(x):
+        return pb._reconstruct_sdpa(x, dkv, 0.1)
+    with pytest.raises((TypeError, RuntimeError)):
+        torch.jit.trace(step, q, check_trace=False)
+    with pytest.raises((TypeError, RuntimeError)):
+        make_fx(step)(q)
+
+
+def test_transforms_and_autocast_keep_the_library_operator():
+    """vmap over queries, forward-mode tangents, and autocast to the other 16-bit type."""
+    import torch.autograd.forward_ad as fwd
+    from winnow_amd import packed_backend as pb
+    lens, Q = (100, 3, 250), 5
+    _, kv = build(501, len(lens), 8, 2, 64, lens, 16, 4)
+    dkv = to_device(kv, DEV)
+    g = torch.Generator().manual_seed(3)
+    many = torch.randn(2, 3, 8, Q, 64, generator=g).to(DEV, torch.bfloat16)
+    want = torch.stack([pb._reconstruct_sdpa(x, dkv, 0.1) for x in many]).float()
+    got = torch.vmap(lambda x: pb._reconstruct_sdpa(x, dkv, 0.1))(many).float()
+    assert torch.allclose(got, want, atol=2e-2 * want.abs().max().item(), rtol=2e-2)
+    with fwd.dual_level():
+        out, tangent = fwd.unpack_dual(pb._reconstruct_sdpa(fwd.make_dual(many[0], many[1]), dkv, 0.1))
+    assert torch.allclose(out.float(), want[0], atol=2e-2 * want.abs().max().item(), rtol=2e-2)
+    h = 0.125
+    along = (pb._reconstruct_sdpa((many[0] + h * many[1]).float(), dkv, 0.1)
+             - pb._reconstruct_sdpa((many[0] - h * many[1]).float(), dkv, 0.1)) / (2 * h)
+    assert torch.allclose(tangent.float(), along, atol=5e-2 * along.abs().max().item())
+    with torch.autocast("cuda", dtype=torch.float16):
+        cast = pb._reconstruct_sdpa(many[0], dkv, 0.1)
+    assert cast.dtype == torch.float16   # as the library's operator gives it
+    assert torch.allclose(cast.float(), want[0], atol=2e-2 * want.abs().max().item(), rtol=2e-2)

@@ -31,6 +31,8 @@ from collections import Counter
 import numpy as np
 import torch
 import torch.nn.functional as F
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 from winnow_amd import _lib
 from winnow_amd import packed_attention as pa
@@ -478,10 +480,22 @@ def _padded_sdpa(query, k, v, lens, scaling):
 
 def _plain(t: torch.Tensor) -> bool:
     """A tensor whose values are all that is wanted of it: no gradient, tangent, batching
-    transform or trace passes through the operator that reads it."""
+    transform, trace or mode passes through the operator that reads it, and no autocast
+    would read it as another type."""
     return (type(t) is torch.Tensor and not (t.requires_grad and torch.is_grad_enabled())
             and not torch._C._functorch.is_functorch_wrapped_tensor(t)
-            and torch.autograd.forward_ad.unpack_dual(t).tangent is None and not torch.compiler.is_compiling())
+            and torch.autograd.forward_ad.unpack_dual(t).tangent is None and not _observed()
+            and not (torch.is_autocast_enabled(t.device.type) and torch.get_autocast_dtype(t.device.type) != t.dtype))
+
+
+def _observed() -> bool:
+    """Whether something records or rewrites the torch operators called here: a compiler, a
+    trace (``torch.jit.trace``, ``make_fx``, export), a dispatch mode, or a function mode
+    other than a default device's."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
+            or torch._ops._len_torch_dispatch_stack_pre_dispatch() > 0
+            or (torch._C._len_torch_function_stack() > 0
+                and not all(isinstance(m, DeviceContext) for m in _get_current_function_mode_stack())))
 
 
 def _history_kernel(query, kv: pa.PackedKV, Lmax: int) -> bool:
