@@ -77,3 +77,29 @@ def test_norms_off_the_word(Hq=8, Hkv=2, D=64, S=16):
     for splits in (None, 3):
         got = pa.packed_decode_attention(q.cuda(), dev, scale, num_splits=splits, out_dtype=torch.float32).cpu().double()
         assert float((got - ref).abs().max()) <= tol
+
+
+@pytest.mark.parametrize("D,S,Hq,Hkv,bwk,bwv,tf32", [(128, 16, 28, 4, 8, 8, False), (128, 16, 8, 8, 4, 8, False),
+                                                     (128, 32, 16, 4, 4, 4, False), (128, 16, 16, 2, 6, 6, False),
+                                                     (128, 16, 8, 8, 4, 6, True), (64, 16, 8, 2, 4, 4, False),
+                                                     (64, 32, 12, 4, 8, 8, False), (64, 16, 3, 3, 2, 2, False)])
+def test_value_norms_of_any_size(D, S, Hq, Hkv, bwk, bwv, tf32):
+    """V norms times a power of two (exact in fp16 here) give the same attention times that
+    power, bit for bit: the scan scales its 16-bit weights by the norms' own exponent,
+    so small norms lose nothing. Norms of a head_dim of 64 or 128 lie within 4 and 20."""
+    from winnow_amd import packed_attention as pa
+    lens = (1, 70, 300, 1500)
+    q, kv = build(800 + S + bwv + D, len(lens), Hq, Hkv, D, lens, S, bwk, bw_v=bwv)
+    scale = oa.default_scale(D)
+    dev = to_device(kv, "cuda")
+    norms, outs = dev.v_norms.clone(), {}
+    for e in (0, -15, 11):
+        dev.v_norms.copy_((norms.float() * 2.0 ** e).half())
+        assert torch.equal(dev.v_norms.float(), norms.float() * 2.0 ** e)
+        outs[e] = pa.packed_decode_attention(q.cuda(), dev, scale, out_dtype=torch.float32, allow_tf32=tf32) * 2.0 ** -e
+    assert float(outs[0].abs().max()) > 0
+    for e in (-15, 11):
+        assert torch.equal(outs[e], outs[0])
+    dev.v_norms.zero_()
+    out = pa.packed_decode_attention(q.cuda(), dev, scale, out_dtype=torch.float32, allow_tf32=tf32)
+    assert (out == 0).all()

@@ -810,9 +810,12 @@ __global__ __launch_bounds__(64 * WPB) void decode_rows_kernel(DecodeArgs a) {
 // The page scan on v_mfma_f32_16x16x32_f16 (16 times the MAC rate of the fp32 4x4x1
 // MFMA on gfx950), for 2, 3, 4, 5 and 6-bit codes, 8-bit ones, and 4 with 8. Every fp32 factor x is carried as
 // an fp16 pair x = H + L (H = fp16(x), L = fp16(x - H)) after an exact power-of-two
-// scaling that keeps both in fp16's normal range; products of fp16 values are exact
-// in the fp32 accumulators and each factor keeps 22 bits, so scores and values keep
-// fp32 accuracy.
+// scaling that takes the largest of a factor's values to the top of fp16's range: values
+// above 2^-3 keep 22 bits, smaller ones an error of 2^-25, 2^-32 or less of the largest.
+// Products of fp16 values are exact in the fp32 accumulators, so scores and values keep
+// fp32 accuracy. Error of fp32 outputs against float64 (rms over 48 sequences' heads): 8/8 bits, 28
+// heads over 4, 300 / 9,000 tokens 5.1e-7 / 6.3e-7 (the fp32-product scan 5.2e-7 / 6.5e-7);
+// head_dim 64, 4/4 bits 4.6e-7 / 6.0e-7 (the vector-ALU scan 6.1e-7 / 7.7e-7).
 //
 // A codebook table entry holds (H, L) of 2^8 c for each of its two codes,
 // [H0, L0, H1, L1]; two entries loaded side by side are an 8-slot MFMA operand, and
@@ -844,7 +847,8 @@ __global__ __launch_bounds__(64 * WPB) void decode_rows_kernel(DecodeArgs a) {
 //            H or L of p n_V 2^-gs of the column's head for those tokens. 8 x 4 = 32 MFMAs
 //            per chunk; output lane 16g+c register i holds dim 32g + 8i + mt, column c.
 //   scales   scores are multiplied by 2^-(e+8) before the softmax; pv' = p n_V 2^-gs
-//            with gs the smallest shift that keeps 256 max(n_V) 2^-gs < 2^15 (raised,
+//            with gs the smallest shift, negative for small norms, that keeps
+//            256 max(n_V) 2^-gs < 2^15 (raised,
 //            with an exact rescale of the accumulators, when a chunk needs it); the
 //            partials are multiplied by 2^(gs-8) when written.
 
@@ -897,10 +901,11 @@ __device__ __forceinline__ void read_unconditionally(float (&x)[N]) {
 }
 
 // H | L << 16 of x with H = fp16(x) and L = fp16(x - H), both rounded to nearest: H + L is
-// x to 2^-22 of itself and without bias (rounded toward zero it is to 2^-20, and every
-// weight and codebook value comes out a little too small: at 8/8 bits, 9,000 tokens, the
-// output's error against float64 was 4.6e-7 of its norm, now 3.8e-7; the fp32-product scan's
-// is 3.6e-7). One conversion instruction per pair either way.
+// x to 2^-22 of itself where |x| >= 2^-3 (below that to 2^-25, half of L's last place) and
+// without bias (rounded toward zero it is to 2^-20, and every weight and codebook value
+// comes out a little too small: at 8/8 bits, 9,000 tokens, the output's error against
+// float64 was 4.6e-7 of its norm that way and 3.8e-7 this way). One conversion
+// instruction per pair either way.
 __device__ __forceinline__ uint32_t split_word(float x) {
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
   const float r = x - float(_Float16(x));
@@ -1215,6 +1220,29 @@ __device__ __forceinline__ void score_phase_mx(const RowBuf<BWK, BWV>& K, Tab16<
   wave_lds_sync();
 }
 
+// Value scale: 2^kRescale * max(n_V) * 2^-gs < 2^15, i.e. every n_V < 2^(7 + gs), with the
+// smallest such gs, negative for small norms: an fp16 pair keeps 22 bits of a weight only
+// above 2^-3 (its low half ends at 2^-24), so the weights of a range go as far up as they
+// fit. The scale only grows, so the wave's maximum is taken only when a norm reaches
+// the limit: in the first chunk with a norm above 0 (no fp16 value lies between
+// 0 and kMinScale's limit, 2^-24), rarely after it.
+// Measured with gs >= 0 instead (fp32 outputs, 8/8 bits, 300 tokens): V norms of 0.1, 0.01 and
+// 0.001 left errors of 9e-7, 7e-6 and 8e-5 of the output's norm, 5e-7 with this one. The
+// maximum of the first chunk costs a wave about 0.1 us.
+constexpr int kMinScale = -31;
+template <int NG>
+__device__ __forceinline__ void raise_value_scale(float nv, MxState<NG>& st) {
+  if (__any(nv >= ldexpf(1.f, 7 + st.gs))) {  // wave-uniform, rare
+    int ge;
+    frexpf(wave_max_nonneg(nv), &ge);
+    const int gs_need = ge - 7;
+    const float f = ldexpf(1.f, st.gs - gs_need);
+#pragma unroll
+    for (int mm = 0; mm < 8; ++mm) st.acc[mm] *= f;
+    st.gs = gs_need;
+  }
+}
+
 // Online softmax of one chunk (lane = token) from the score tile; p n_V 2^-gs goes
 // back to the same words as H | L << 16.
 template <int NG, bool PAIR = false>
@@ -1249,17 +1277,7 @@ __device__ __forceinline__ void softmax_phase_mx(float sc, uint32_t nk_h, uint32
 #pragma unroll
     for (int i = 0; i < H; ++i) sv[i] = valid[PAIR ? i / 4 : 0] ? x[i] * nk[PAIR ? i / 4 : 0] : -INFINITY;
   }
-  // value scale: 2^kRescale * max(n_V) * 2^-gs < 2^15, i.e. every n_V < 2^(7 + gs); the
-  // scale only grows, so the wave's maximum is taken only when a norm reaches the limit
-  if (__any(nv >= ldexpf(1.f, 7 + st.gs))) {  // wave-uniform, rare
-    int ge;
-    frexpf(wave_max_nonneg(nv), &ge);
-    const int gs_need = max(0, ge - 7);
-    const float f = ldexpf(1.f, st.gs - gs_need);
-#pragma unroll
-    for (int mm = 0; mm < 8; ++mm) st.acc[mm] *= f;
-    st.gs = gs_need;
-  }
+  raise_value_scale(nv, st);
   // the reference maxima move when a score exceeds its head's by more than kRescale:
   // one test of the largest excess over the heads (masked tokens give -inf; the first
   // chunk, with every maximum at -inf, always moves)
@@ -1457,15 +1475,7 @@ __device__ __forceinline__ void softmax_phase_tf(float sc, uint32_t nk_h, uint32
   read_unconditionally(x);
 #pragma unroll
   for (int i = 0; i < H; ++i) sv[i] = valid ? x[i] * nk : -INFINITY;
-  if (__any(nv >= ldexpf(1.f, 7 + st.gs))) {  // wave-uniform, rare
-    int ge;
-    frexpf(wave_max_nonneg(nv), &ge);
-    const int gs_need = max(0, ge - 7);
-    const float f = ldexpf(1.f, st.gs - gs_need);
-#pragma unroll
-    for (int mm = 0; mm < 8; ++mm) st.acc[mm] *= f;
-    st.gs = gs_need;
-  }
+  raise_value_scale(nv, st);
   float d[H], dmax = -INFINITY;
 #pragma unroll
   for (int i = 0; i < H; ++i) {
@@ -1734,7 +1744,7 @@ __device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh
     st.m[i] = -INFINITY;
     st.l[i] = 0.f;
   }
-  st.gs = 0;
+  st.gs = kMinScale;
   using Buf = RowBuf<BWK, BWV>;
   const int smask = (1 << log2S) - 1;
   const uint64_t kbase = uint64_t(a.k_pages) + uint64_t(kvh >> a.kvshift) * uint64_t(a.ksh);
