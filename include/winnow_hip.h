@@ -354,7 +354,8 @@ int wn_dequantize_histories(const uint8_t* pages, int64_t page_stride, int64_t h
  *   q     (B, Hq, Q, D), WN_BF16 or WN_F16, element strides multiples of 8
  *   k, v  (B, Hkv, Lpad, D) contiguous, q's type; rows past seq_lens[b] are not read
  *   out   (B, Q, Hq, D) contiguous, q's type
- * Exact 16-bit operands, fp32 scores and softmax, probabilities as pairs of 16-bit values.
+ * Exact 16-bit operands, fp32 scores and softmax, probabilities as sums of 16-bit values (three
+ * for WN_BF16, two for WN_F16).
  * D 64 or 128; all operands 16-byte aligned, the workspace (wn_history_workspace_bytes)
  * 256. num_splits from wn_history_plan (any value 1..4096 is valid). */
 int wn_history_plan(int B, int Hq, int Hkv, int Q, int D, int dtype, int max_len, int* num_splits);

@@ -144,3 +144,37 @@ def test_transforms_and_autocast_keep_the_library_operator():
         cast = pb._reconstruct_sdpa(many[0], dkv, 0.1)
     assert cast.dtype == torch.float16   # as the library's operator gives it
     assert torch.allclose(cast.float(), want[0], atol=2e-2 * want.abs().max().item(), rtol=2e-2)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+def test_probabilities_keep_fp32_precision(D, dtype):
+    """Values of both signs whose weighted sum nearly cancels show the weights' own errors
+    beside the output's rounding. fp32 weights are off by about 2^-22 of themselves (the scores here
+    are exact in fp32, so that leaves their scaling and the exponential), the result by at
+    most 2^-20 of the weighted sum of magnitudes; a single token of large score and no
+    value makes the other weights small."""
+    from winnow_amd import packed_attention as pa
+    from winnow_amd import packed_backend as pb
+    B, Hq, Hkv, Q, L = 16, 8, 2, 4, 24
+    g = torch.Generator().manual_seed(D)
+    q = torch.randint(-8, 9, (B, Hq, Q, D), generator=g).to(dtype) / 8
+    k = torch.zeros(B, Hkv, L, D)
+    k[..., :6] = torch.randint(-8, 9, (B, Hkv, L, 6), generator=g) / 4
+    k[:, :, 0, 6] = 24                       # the token of no value; q's channel 6 is 1
+    q[..., 6] = 1
+    v = torch.randint(0, 2, (B, Hkv, L, D), generator=g) * 128.0 - 64
+    v[:, :, 0] = 0
+    k, v = k.to(dtype), v.to(dtype)
+    kv = pa.PackedKV(torch.empty(0, Hkv, 16, D, dtype=torch.uint8, device=DEV), None, None, None, None,
+                     torch.full((B,), L, dtype=torch.int32, device=DEV), None, None, D)
+    scale = 0.25
+    got = pb._history_attention(q.to(DEV), kv, k.to(DEV), v.to(DEV), L, scale).cpu().double()
+    kk, vv = (x.double().repeat_interleave(Hq // Hkv, 1) for x in (k, v))
+    s = scale * (q.double() @ kk.transpose(-1, -2))
+    s.masked_fill_(torch.arange(L) > (L - Q + torch.arange(Q))[:, None], -float("inf"))
+    p = torch.softmax(s, -1)
+    ref, size = p @ vv, p @ vv.abs()
+    half = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    worst = ((got - ref).abs() / (half * ref.abs() + 2.0 ** -20 * size)).max().item()
+    assert worst <= 1, f"{worst:.2f} of the bound"

@@ -12,8 +12,11 @@
 // v_mfma_f32_16x16x32_{bf16,f16} and no score leaves the work-group.
 //
 // Precision is that of the fp32 products: q, K and V are exact operands, scores and
-// softmax are fp32, and each probability goes to its product as a pair hi + lo of 16-bit
-// values (16 bits for bf16, 22 for fp16).
+// softmax are fp32, and each probability goes to its product as a sum of 16-bit values:
+// three for bf16 (24 bits), two for fp16, taken up by 2^7 to the top of fp16's range (22
+// bits of those above 2^-10 of the largest, 2^-32 of the largest below). A bf16 pair (16
+// bits) took 80.6 us for the call below and left up to three times the error that fp32
+// weights have where a sum of both signs cancels.
 //
 // Work-group: eight waves take eight neighbouring 32-row query blocks (row r = qi n_rep +
 // h) of one (sequence, kv head, split) and share its 64-token chunks through two LDS tile
@@ -23,8 +26,8 @@
 // [dim][token] rows of 144 bytes; row c of score tile t is token 32 (t >> 1) + 8 (c >> 2)
 // + 4 (t & 1) + (c & 3), so that lane 16g + c ends the scores with the eight tokens that
 // are its k-slots of a value K-step.
-// Measured (that call, 8-bit K and V): 952 -> 81 us, of which the two batched dequants
-// 21 us each, this scan 38 us and the merge 7 us (traces); the same distance from 64 bits.
+// Measured (that call, 8-bit K and V): 952 -> 84 us, of which the two batched dequants
+// 21 us each, this scan 42 us and the merge 7 us; the same distance from 64 bits.
 #include <algorithm>
 #include <map>
 #include <mutex>
@@ -75,19 +78,29 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c, 0, 0, 0);
 }
 
-// Two values as a pair of 16-bit ones, rounded to nearest, and what each rounding left.
+// Terms of a probability in the 16-bit type, and the log2 it is taken up by (its largest, 2^8,
+// ends below 2^15).
 template <bool BF>
-__device__ __forceinline__ void split2(float x, float y, uint32_t& hi, uint32_t& lo) {
+constexpr int kHtTerms = BF ? 3 : 2;
+template <bool BF>
+constexpr float kHtLift = BF ? 0.f : 7.f;
+
+// Two values as 16-bit ones, rounded to nearest, and, term by term, what the rounding left.
+template <bool BF>
+__device__ __forceinline__ void split_terms(float x, float y, uint32_t (&o)[kHtTerms<BF>]) {
   if constexpr (BF) {
     typedef __bf16 b2 __attribute__((ext_vector_type(2)));
     typedef float f2 __attribute__((ext_vector_type(2)));
-    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x, y}, b2));
-    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x - __builtin_bit_cast(float, hi << 16),
-                                                                 y - __builtin_bit_cast(float, hi & 0xffff0000u)}, b2));
+#pragma unroll
+    for (int i = 0; i < kHtTerms<BF>; ++i) {
+      o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2{x, y}, b2));
+      x -= __builtin_bit_cast(float, o[i] << 16);
+      y -= __builtin_bit_cast(float, o[i] & 0xffff0000u);
+    }
   } else {
     const _Float16 a = _Float16(x), b = _Float16(y);
-    hi = uint32_t(__builtin_bit_cast(uint16_t, a)) | uint32_t(__builtin_bit_cast(uint16_t, b)) << 16;
-    lo = tf_word(x - float(a), y - float(b));
+    o[0] = uint32_t(__builtin_bit_cast(uint16_t, a)) | uint32_t(__builtin_bit_cast(uint16_t, b)) << 16;
+    o[1] = tf_word(x - float(a), y - float(b));
   }
 }
 
@@ -145,6 +158,8 @@ template <int D, bool BF>
 __global__ __launch_bounds__(64 * kHtWaves) void history_kernel(HistArgs a) {
   using T = HistTile<D>;
   constexpr int KS = D / 32, MT = D / 16, LA = 4;  // K-steps, value M-tiles, operand reads in flight
+  constexpr int NT = kHtTerms<BF>;
+  constexpr float lift = kHtLift<BF>;
   __shared__ __align__(16) char lds[2 * T::Set];
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int wig = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -230,7 +245,7 @@ __global__ __launch_bounds__(64 * kHtWaves) void history_kernel(HistArgs a) {
           __builtin_amdgcn_sched_barrier(0);
         });
       }
-      u32x4 ph[2][2], pl[2][2];  // value operands: tokens 32 ks + 8g .. + 7 of column tile ct
+      u32x4 pt[NT][2][2];  // value operands, by term: tokens 32 ks + 8g .. + 7 of column tile ct
 #pragma unroll
       for (int ct = 0; ct < 2; ++ct) {
         const bool fresh = m[ct] == -INFINITY;
@@ -241,12 +256,13 @@ __global__ __launch_bounds__(64 * kHtWaves) void history_kernel(HistArgs a) {
         for (int t = 0; t < 4; ++t)
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float y = fmaf(d[ct][t][i], a.scale, -m0);
+            const float y = fmaf(d[ct][t][i], a.scale, lift - m0);
             x[4 * t + i] = full || 32 * (t >> 1) + 4 * (t & 1) + i <= last ? y : -INFINITY;
             top = fmaxf(top, x[4 * t + i]);
           }
         top = fmaxf(top, __shfl_xor(top, 16, 64));
         top = fmaxf(top, __shfl_xor(top, 32, 64));
+        top -= lift;
         const bool move = top > kHtRescale || (fresh && top > -INFINITY);
         if (__any(move)) {  // wave-uniform
           const float shift = move ? top : 0.f;
@@ -265,10 +281,10 @@ __global__ __launch_bounds__(64 * kHtWaves) void history_kernel(HistArgs a) {
             const int k = 8 * ks + 2 * j;
             const float p0 = __builtin_amdgcn_exp2f(x[k]), p1 = __builtin_amdgcn_exp2f(x[k + 1]);
             l[ct] += p0 + p1;
-            uint32_t hi, lo;
-            split2<BF>(p0, p1, hi, lo);
-            ph[ct][ks][j] = hi;
-            pl[ct][ks][j] = lo;
+            uint32_t w[NT];
+            split_terms<BF>(p0, p1, w);
+#pragma unroll
+            for (int i = 0; i < NT; ++i) pt[i][ct][ks][j] = w[i];
           }
       }
       {  // step k = MT ks + mt: tokens 32 ks + 8g .. of dim 16 mt + c
@@ -286,9 +302,9 @@ __global__ __launch_bounds__(64 * kHtWaves) void history_kernel(HistArgs a) {
             __builtin_amdgcn_sched_barrier(0);
           }
 #pragma unroll
-          for (int ct = 0; ct < 2; ++ct) acc[ct][mt] = mfma16<BF>(e[j], ph[ct][ks], acc[ct][mt]);
+          for (int i = 0; i < NT; ++i)
 #pragma unroll
-          for (int ct = 0; ct < 2; ++ct) acc[ct][mt] = mfma16<BF>(e[j], pl[ct][ks], acc[ct][mt]);
+            for (int ct = 0; ct < 2; ++ct) acc[ct][mt] = mfma16<BF>(e[j], pt[i][ct][ks], acc[ct][mt]);
           __builtin_amdgcn_sched_barrier(0);
         });
       }
