@@ -352,7 +352,8 @@ int wn_dequantize_histories(const uint8_t* pages, int64_t page_stride, int64_t h
  * (packed_backend.py:211-226): query i of sequence b attends to keys j <= L - Q + i of
  * the first L = seq_lens[b] rows of k and v; a query that sees none gives 0.
  *   q     (B, Hq, Q, D), WN_BF16 or WN_F16, element strides multiples of 8
- *   k, v  (B, Hkv, Lpad, D) contiguous, q's type; rows past seq_lens[b] are not read
+ *   k, v  (B, Hkv, Lpad, D) contiguous, q's type; rows past seq_lens[b] are not read (a
+ *         length above Lpad counts as Lpad)
  *   out   (B, Q, Hq, D) contiguous, q's type
  * Exact 16-bit operands, fp32 scores and softmax, probabilities as sums of 16-bit values (three
  * for WN_BF16, two for WN_F16).

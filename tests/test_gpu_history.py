@@ -178,3 +178,20 @@ def test_probabilities_keep_fp32_precision(D, dtype):
     half = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     worst = ((got - ref).abs() / (half * ref.abs() + 2.0 ** -20 * size)).max().item()
     assert worst <= 1, f"{worst:.2f} of the bound"
+
+
+def test_a_length_past_the_histories():
+    """Device lengths beyond the rows of K and V (ahead of the host's, from which the rows
+    were counted) count as that many rows."""
+    from winnow_amd import packed_attention as pa
+    from winnow_amd import packed_backend as pb
+    B, Hq, Hkv, Q, D, Lmax = 2, 4, 2, 3, 64, 70
+    g = torch.Generator().manual_seed(7)
+    q = torch.randn(B, Hq, Q, D, generator=g).to(DEV, torch.bfloat16)
+    k, v = (torch.randn(B, Hkv, Lmax, D, generator=g).to(DEV, torch.bfloat16) for _ in range(2))
+
+    def run(lens):
+        kv = pa.PackedKV(torch.empty(0, Hkv, 16, D, dtype=torch.uint8, device=DEV), None, None, None, None,
+                         torch.tensor(lens, dtype=torch.int32, device=DEV), None, None, D)
+        return pb._history_attention(q, kv, k, v, Lmax, 0.1)
+    assert torch.equal(run((Lmax + 1, Lmax + 100)), run((Lmax, Lmax)))

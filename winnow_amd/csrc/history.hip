@@ -175,7 +175,7 @@ __global__ __launch_bounds__(64 * kHtWaves) void history_kernel(HistArgs a) {
   const int rows = a.n_rep * a.Q;
   const int r_first = cg * kHtRows + wig * kHtBlock;
   const bool live = r_first < rows;
-  const int L = const_view(a.seq_lens)[b];
+  const int L = int(min(int64_t(const_view(a.seq_lens)[b]), a.Lpad));  // no row past the histories' own
   // the chunks that the group's last row sees
   const int g_last = min((cg + 1) * kHtRows, rows) - 1;
   const int seen = max(0, min(L, L - a.Q + g_last / a.n_rep + 1));
