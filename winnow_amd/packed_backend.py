@@ -418,7 +418,14 @@ def dequantize_history(kv: pa.PackedKV, pages, norms, quant, b: int, dtype) -> t
 
     Contiguous page rows: one launch reads the pool pages through the table row,
     ``wn_dequantize_history`` at head_dim 128 and ``wn_dequantize_pages`` at the others.
-    Other layouts gather the rows, unpack and dequantize with the standalone kernels."""
+    Other layouts gather the rows, unpack and dequantize with the standalone kernels. Raises
+    ``UnsupportedLayout`` for a length or page id out of range."""
+    pa.check_page_ranges(_host_lens(kv)[b:b + 1], _host_table(kv)[b:b + 1], pages.shape[0], kv.page_size)
+    return _history(kv, pages, norms, quant, b, dtype)
+
+
+def _history(kv: pa.PackedKV, pages, norms, quant, b: int, dtype) -> torch.Tensor:
+    """``dequantize_history`` of a handle whose ranges are checked."""
     L = int(_host_lens(kv)[b])
     S, D, Hkv = kv.page_size, kv.head_dim, pages.shape[1]
     odt = dtype if dtype in _lib.DTYPE_CODE else torch.float32
@@ -509,6 +516,7 @@ def _history_kernel(query, kv: pa.PackedKV, Lmax: int) -> bool:
     return (D in (64, 128) and kv.head_dim == D and _lib.is_hip(query) and Hq % Hkv == 0 and Q > 0
             and query.device == kv.k_pages.device == lens.device and lens.dtype == torch.int32 and lens.shape == (B,)
             and lens.is_contiguous() and kv.page_table.dtype == torch.int32 and kv.page_table.stride(-1) == 1
+            and kv.page_table.shape[0] >= B and kv.page_table.device == query.device
             and Hq // Hkv * Q <= 1 << 24 and B * Hkv * Lmax < 1 << 31)
 
 
@@ -530,7 +538,7 @@ def _histories(kv: pa.PackedKV, pages, norms, quant, lens, Lmax: int, dtype) -> 
         return buf
     for b in range(B):
         if lens[b]:
-            buf[b, :, :int(lens[b])] = dequantize_history(kv, pages, norms, quant, b, dtype)[0]
+            buf[b, :, :int(lens[b])] = _history(kv, pages, norms, quant, b, dtype)[0]
     return buf
 
 
@@ -562,6 +570,8 @@ def _reconstruct_sdpa(query, kv: pa.PackedKV, scaling):
     Lmax = int(lens.max()) if B else 0
     if Lmax == 0:
         return torch.zeros(B, Hq, Q, D, dtype=query.dtype, device=query.device)
+    # the kernels read pages by the table's ids, unchecked
+    pa.check_page_ranges(_host_lens(kv)[:B], _host_table(kv)[:B], kv.k_pages.shape[0], kv.page_size)
     sides = ((kv.k_pages, kv.k_norms, kv.k_quant), (kv.v_pages, kv.v_norms, kv.v_quant))
     if _history_kernel(query, kv, Lmax):
         k, v = (_histories(kv, *side, lens, Lmax, query.dtype) for side in sides)
@@ -571,7 +581,7 @@ def _reconstruct_sdpa(query, kv: pa.PackedKV, scaling):
         buf = torch.zeros(B, kv.num_kv_heads, Lmax, D, dtype=query.dtype, device=query.device)
         for b in range(B):
             if lens[b]:
-                buf[b, :, :int(lens[b])] = dequantize_history(kv, pages, norms, quant, b, query.dtype)[0]
+                buf[b, :, :int(lens[b])] = _history(kv, pages, norms, quant, b, query.dtype)[0]
         hist.append(buf)
     return _padded_sdpa(query, hist[0], hist[1], lens, scaling)
 
