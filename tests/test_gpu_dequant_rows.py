@@ -165,3 +165,32 @@ def test_pages_of_whole_sequences(D, bw):
     pb._dequantize_pages(dkv, *side, dkv.page_table, None, L, got)
     for b in range(B):
         assert torch.equal(got[b], pb.dequantize_history(dkv, *side, b, torch.float32)[0])
+
+
+@pytest.mark.parametrize("D,n_out,span", [(320, 64, 1024), (288, 40, 10), (512, 256, 1024)])
+def test_heads_wider_than_the_rows_kernel(D, n_out, span):
+    """Outlier channels beside at most 256 regular ones: group by group, by chunks."""
+    from winnow_amd.packing import unpack
+    B, H, n = 2, 2, 37
+    loud = torch.randperm(D, generator=torch.Generator().manual_seed(D))[:n_out].to(DEV)
+    layer = _layer(D, 4, n_out, 8, n + 3, chunk=span)
+    for step, m in enumerate((n - 1, 1)):
+        got = layer.update(*_kv(B, H, m, D, loud, torch.float32, step))
+    for x, groups in zip(got, (layer._k_groups, layer._v_groups)):
+        want = torch.zeros(B, H, n, D, dtype=torch.float64, device=DEV)
+        for grp, tq, w, dim, mask in ((groups[0], layer._quant, 4, D - n_out, ~layer._outlier_channels),
+                                      (groups[1], layer._quant_outlier, 8, n_out, layer._outlier_channels)):
+            want[..., mask] = _closed(unpack(grp.codes[:, :, :n].contiguous(), w, dim), grp.norms[:, :, :n], tq)
+        assert ((x.double() - want).abs() <= 2e-6 * want.abs().max()).all()
+
+
+def test_histories_past_the_row_limit_go_group_by_group(monkeypatch):
+    """The rows kernel counts rows in 31 bits: with the limit lowered, the same values."""
+    from winnow_amd import cache as wc
+    D, n = 64, 50
+    loud = torch.arange(8, device=DEV)
+    k, v = _kv(2, 3, n, D, loud, torch.float32, 3)
+    whole = _layer(D, 4, 8, 8, n).update(k, v)
+    monkeypatch.setattr(wc, "_ROWS_LIMIT", 2 * 3 * n)
+    for a, b in zip(_layer(D, 4, 8, 8, n, chunk=16).update(k, v), whole):
+        assert torch.allclose(a, b, rtol=0, atol=2e-6 * b.abs().max().item())

@@ -20,13 +20,15 @@ On MI355X:
   group width up to 256);
 * the history comes back through ``wn_tq_dequant`` (the fused kernel, read in place
   from the ``max_cache_len`` buffer) at head_dim 128 without outlier channels, else
-  through ``wn_dequantize_rows`` at fp32 accuracy, K and V in one launch.
+  through ``wn_dequantize_rows`` at fp32 accuracy, K and V in one launch, up to
+  head_dim 256; wider heads (outlier channels beside at most 256 regular ones) through
+  ``wn_unpack`` + ``wn_dequantize`` per group in chunks of ``chunk`` positions.
 
 ``kernel_backend`` keeps the reference's names: ``"triton_fp32"`` and
 ``"native_cuda_fp32"`` select the fused kernel at fp32 accuracy, ``"triton_tf32"``
 the fused kernel's fast mode (one fp16 product per term), ``"torch_fp32"`` the
 fp32-accurate rows kernel (the reference's chunked path, recorded under that name;
-``chunk`` is accepted and ignored), and ``"auto"`` the fused kernel where it applies
+``chunk`` matters above head_dim 256 only), and ``"auto"`` the fused kernel where it applies
 (fast when ``allow_tf32``) and the rows kernel elsewhere. The reference's dispatcher
 (``dispatch.py``) is not used: ``native_kernel`` and ``dispatcher`` are accepted
 and ignored, and ``last_dispatch_decision`` records the path taken.
@@ -40,13 +42,15 @@ from transformers.cache_utils import DynamicCache, DynamicLayer
 
 from winnow_amd import _lib
 from winnow_amd.kernel import tq_dequant
-from winnow_amd.packing import pack, packed_bytes
+from winnow_amd.packing import pack, packed_bytes, unpack
 from winnow_amd.quantizer import get_quantizer
 
 KERNEL_BACKENDS = ("auto", "torch_fp32", "triton_fp32", "triton_tf32", "native_cuda_fp32")
 _FUSED_HEAD_DIM = 128   # wn_tq_dequant's head_dim
 _APPEND_HEAD_DIMS = (16, 32, 64, 128, 256)
 _SPLIT_HEAD_DIMS = (64, 128)   # wn_append_split's
+_ROWS_HEAD_DIM = 256           # wn_dequantize_rows' largest
+_ROWS_LIMIT = 1 << 31          # rows per side of wn_append_split and wn_dequantize_rows
 
 
 @dataclass
@@ -75,13 +79,13 @@ class TQPackedLayer(DynamicLayer):
                  use_kernel: bool = True, allow_tf32: bool = True, kernel_backend: str = "auto",
                  native_kernel=None, dispatcher=None):
         super().__init__()
-        del native_kernel, dispatcher, chunk  # not used here
+        del native_kernel, dispatcher  # planner objects of the reference, not used here
         backend = kernel_backend if use_kernel else "torch_fp32"
         if backend not in KERNEL_BACKENDS:
             raise ValueError(f"unknown kernel_backend={kernel_backend!r}")
         self.use_kernel, self.allow_tf32, self.kernel_backend = use_kernel, allow_tf32, backend
         self.last_dispatch_decision: DequantChoice | None = None
-        self._head_dim, self._bits, self._capacity = head_dim, bit_width, max_cache_len
+        self._head_dim, self._bits, self._capacity, self._span = head_dim, bit_width, max_cache_len, chunk
         split = num_outlier_channels > 0 and outlier_bits > bit_width
         self._n_outlier = num_outlier_channels if split else 0
         self._n_regular = head_dim - self._n_outlier
@@ -169,7 +173,7 @@ class TQPackedLayer(DynamicLayer):
         """One wn_append_split launch writes both sides and groups: a compiled head_dim,
         K/V rows that 16-byte loads read."""
         return (bool(self._n_outlier) and self._head_dim in _SPLIT_HEAD_DIMS and k.dtype in _lib.DTYPE_CODE
-                and v.dtype == k.dtype and all(
+                and v.dtype == k.dtype and k.numel() < _ROWS_LIMIT * self._head_dim and all(
                     x.stride(-1) == 1 and x.data_ptr() % 16 == 0
                     and all(s * x.element_size() % 16 == 0 for s in x.stride()[:3]) for x in (k, v)))
 
@@ -232,6 +236,10 @@ class TQPackedLayer(DynamicLayer):
                 tq_dequant(g.codes[:, :, :length], g.norms[:, :, :length], self._quant.centroids, self._quant.Pi,
                            self._bits, D, out=out, allow_tf32=choice.fast)
             return k, v
+        if D > _ROWS_HEAD_DIM or B * H * length >= _ROWS_LIMIT:
+            for groups, out in ((self._k_groups, k), (self._v_groups, v)):
+                self._group_history(groups, length, out)
+            return k, v
         exact = self.dtype in _lib.DTYPE_CODE   # else through fp32
         ok, ov = (k, v) if exact else (k.float(), v.float())
         kg, vg, q = self._k_groups[0], self._v_groups[0], self._quant
@@ -248,6 +256,21 @@ class TQPackedLayer(DynamicLayer):
                       B * H, length, self._capacity, D, _lib.ptr(ok), _lib.ptr(ov), _lib.DTYPE_CODE[ok.dtype],
                       _lib.stream_of(self.device))
         return (ok, ov) if exact else (ok.to(self.dtype), ov.to(self.dtype))
+
+    def _group_history(self, groups, length: int, out: torch.Tensor) -> None:
+        """One side's first ``length`` positions, group by group: each has at most 256 channels."""
+        quants = [(self._quant, self._bits, self._n_regular)] + \
+            ([(self._quant_outlier, self._outlier_bits, self._n_outlier)] if self._n_outlier else [])
+        for s in range(0, length, self._span):
+            e = min(s + self._span, length)
+            pieces = []
+            for g, (q, bw, dim) in zip(groups, quants):
+                pieces.append(torch.empty(*out.shape[:2], e - s, dim, dtype=out.dtype, device=out.device))
+                q.dequantize_into(unpack(g.codes[:, :, s:e].contiguous(), bw, dim), g.norms[:, :, s:e], pieces[-1])
+            if self._n_outlier:
+                out[:, :, s:e, ~self._outlier_channels], out[:, :, s:e, self._outlier_channels] = pieces
+            else:
+                out[:, :, s:e] = pieces[0]
 
     # ---------------------------------------------------------------- cache protocol
     def _check_step(self, k: torch.Tensor, v: torch.Tensor) -> None:
