@@ -190,12 +190,17 @@ def lib() -> ctypes.CDLL:
                 handle = ctypes.CDLL(str(LIB_PATH))
             except OSError as e:
                 raise HipLibraryMissing(f"cannot load {LIB_PATH}: {e}") from e
+            # the version before the entry points: a version gains some, so that a library of
+            # the same one may still lack the newest
+            version = getattr(handle, "wn_abi_version", lambda: None)()
+            if version != ABI_VERSION:
+                raise HipLibraryMissing(f"{LIB_PATH} has ABI {version}, expected {ABI_VERSION}; rebuild it")
+            missing = [name for name in SIGNATURES if not hasattr(handle, name)]
+            if missing:
+                raise HipLibraryMissing(f"{LIB_PATH} lacks {', '.join(missing)}; rebuild it")
             for name, (res, args) in SIGNATURES.items():
                 fn = getattr(handle, name)
                 fn.restype, fn.argtypes = res, args
-            if handle.wn_abi_version() != ABI_VERSION:
-                raise HipLibraryMissing(
-                    f"{LIB_PATH} has ABI {handle.wn_abi_version()}, expected {ABI_VERSION}; rebuild it")
             _lib = handle
     return _lib
 
