@@ -80,7 +80,8 @@ const char* wn_last_error(void);
  * share the flattened (sequence, kv head, 64-token chunk) space equally, ragged
  * batches included. Otherwise (any other pair of widths in {2,3,4,5,6,8}, head_dim
  * 16, 32, 64 or 256, any other n_rep, run as groups of <= 16 query heads) fixed
- * splits sized to fill the GPU (head_dim 64 with n_rep <= 4 runs the row scan on them). Head dims: the powers of two 16 .. 256. */
+ * splits sized to fill the GPU (on them, head_dim 64 with n_rep <= 4 runs the row scan where
+ * B * Hq * S * max_pages is 786,432 or more). Head dims: the powers of two 16 .. 256. */
 int wn_decode_plan(int B, int Hq, int Hkv, int D, int S, int bw_k, int bw_v, int max_pages,
                    int requested_splits, int* pages_per_split, int* num_splits);
 

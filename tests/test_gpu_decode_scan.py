@@ -79,6 +79,47 @@ def test_norms_off_the_word(Hq=8, Hkv=2, D=64, S=16):
         assert float((got - ref).abs().max()) <= tol
 
 
+def _room(dev, tokens=3 << 18):
+    """The handle with a page table that has room for ``tokens`` (token, query head) pairs at
+    three heads and more: the size from which head_dim 64 runs two tokens to a row."""
+    B, width = dev.page_table.shape
+    pad = torch.full((B, -(-tokens // (3 * B * dev.page_size)) + 1 - width), -1, dtype=torch.int32)
+    dev.page_table_host = torch.cat([dev.page_table_host, pad], 1)
+    dev.page_table = dev.page_table_host.cuda()
+    return dev
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,bwk,bwv", [(16, 8, 2, 4, 4), (32, 12, 4, 4, 4), (128, 3, 3, 8, 8), (16, 4, 2, 5, 5), (64, 8, 2, 6, 4),
+                                              (16, 6, 2, 3, 3), (16, 8, 4, 2, 2), (32, 8, 2, 6, 6), (16, 4, 1, 4, 6), (64, 6, 2, 4, 8),
+                                              (16, 8, 2, 8, 8)])
+@pytest.mark.parametrize("apart", [False, True])
+def test_two_tokens_to_a_row(S, Hq, Hkv, bwk, bwv, apart):
+    """head_dim 64 in a table large enough for the row scan, at the lengths where a row, a
+    chunk, a page or a split ends, and with a head's pages and norms apart from the next
+    one's (strides larger than a block)."""
+    from winnow_amd import packed_attention as pa
+    D = 64
+    lens = (0, 1, 2, 3, 63, 64, 65, 127, 128, 129, 130, 255, 257, 2049)
+    q, kv = build(900 + S + bwk + bwv, len(lens), Hq, Hkv, D, lens, S, bwk, bw_v=bwv)
+    scale = oa.default_scale(D)
+    ref, tol = _float64(q, kv, scale)
+    dev = _room(to_device(kv, "cuda"))
+    if apart:
+        for name in ("k_pages", "v_pages", "k_norms", "v_norms"):
+            x = getattr(dev, name)
+            wide = torch.full((x.shape[0], 2 * Hkv, *x.shape[2:]), 0x55, dtype=torch.uint8, device="cuda").to(x.dtype)
+            wide[:, 1::2] = x
+            setattr(dev, name, wide[:, 1::2])
+    plan = pa.plan_for(q.cuda(), dev)
+    assert plan[1] <= 256 and plan[0] * dev.page_size >= 128
+    for splits in (None, 1, 7, 2000):
+        got = pa.packed_decode_attention(q.cuda(), dev, scale, num_splits=splits, out_dtype=torch.float32).cpu().double()
+        assert torch.isfinite(got).all()
+        err = float((got - ref).abs().max())
+        assert err <= tol, (err, tol)
+        assert (got[0] == 0).all()
+
+
 @pytest.mark.parametrize("D,S,Hq,Hkv,bwk,bwv,tf32", [(128, 16, 28, 4, 8, 8, False), (128, 16, 8, 8, 4, 8, False),
                                                      (128, 32, 16, 4, 4, 4, False), (128, 16, 16, 2, 6, 6, False),
                                                      (128, 16, 8, 8, 4, 6, True), (64, 16, 8, 2, 4, 4, False),
@@ -92,6 +133,8 @@ def test_value_norms_of_any_size(D, S, Hq, Hkv, bwk, bwv, tf32):
     q, kv = build(800 + S + bwv + D, len(lens), Hq, Hkv, D, lens, S, bwk, bw_v=bwv)
     scale = oa.default_scale(D)
     dev = to_device(kv, "cuda")
+    if D == 64:
+        _room(dev)
     norms, outs = dev.v_norms.clone(), {}
     for e in (0, -15, 11):
         dev.v_norms.copy_((norms.float() * 2.0 ** e).half())

@@ -7,7 +7,7 @@
 //   2. page scan         the row-per-lane matrix-core scan (decode_rows.hip) where
 //                        it applies (head_dim 128, a width pair it compiles, and
 //                        n_rep that 2^s virtual heads per kv head bring to <= 8;
-//                        head_dim 64 with n_rep <= 4, two tokens to a row),
+//                        large batches at head_dim 64 with n_rep <= 4, two tokens to a row),
 //                        else decode_split_kernel (wn_split.h): one work-group per
 //                        (split, kv head, sequence), score phase (lane = token),
 //                        online softmax, value phase (16 lanes per token row),
@@ -405,6 +405,8 @@ int valu_groups(int n_rep) {
   return n_rep > 0 ? n_rep : 1;
 }
 
+constexpr int64_t kPairMin = 3 << 18;
+
 // The scan wn_decode_attention runs for this shape: the row-per-lane matrix-core
 // scan where it applies (head_dim 128, page size >= 16, a compiled width pair, any
 // n_rep that 2^s virtual heads bring to <= 8), else the vector-ALU scan (any
@@ -412,7 +414,8 @@ int valu_groups(int n_rep) {
 // tf32: the TF32-class row scan where it is compiled (4 and 6-bit K and V, alike or
 // mixed, on the row scan: n_rep up to 8, or up to 16 in virtual kv heads of eight),
 // else the same choice as without it.
-SplitKernel choose_scan(int Hq, int Hkv, int D, int S, int bw_k, int bw_v, bool tf32 = false, bool norm_words = true) {
+SplitKernel choose_scan(int B, int Hq, int Hkv, int D, int S, int max_pages, int bw_k, int bw_v, bool tf32 = false,
+                        bool norm_words = true) {
   SplitKernel sk;
   const int n_rep = Hq / Hkv;
   const int shift = row_shift(n_rep);
@@ -425,11 +428,15 @@ SplitKernel choose_scan(int Hq, int Hkv, int D, int S, int bw_k, int bw_v, bool 
     }
   }
   // head_dim 64, two tokens to a row, for up to four heads of a kv head (the scan's eight
-  // columns are heads x 2 tokens), pages of whole blocks of eight rows, and norms that
-  // can be read by the word: 48 us against the vector-ALU scan's 87 with 32 heads over 8
-  // (16 sequences of 3,000 to 12,000 tokens, 4/4 bits), 67 against 84 with 16 over 8
-  // (32 of 8,000, 6/6), level at 300 tokens (40 and 42, host time).
-  if (D == 64 && S >= 16 && norm_words && rows_allowed()) sk = pick_split_pair(bw_k, bw_v, n_rep);
+  // columns are heads x 2 tokens), pages of whole blocks of eight rows, norms that can be
+  // read by the word, and a batch whose table holds kPairMin (token, query head) pairs:
+  // below them the vector-ALU scan's shorter start wins. Measured (us, a call by itself,
+  // vector ALU -> row scan): 32 heads over 8, 4/4 bits, 8 x 300 tokens 60 -> 64, 64 x 300 76 -> 68,
+  // 64 x 2,000 129 -> 86, 16 x 3,000 84 -> 72; 8 over 8, 8/8 bits, 8 x 4,096 66 -> 73,
+  // 8 x 8,192 77 -> 81; 16 over 8, 4/4, 8 x 4,096 65 -> 69, 8 x 8,192 78 -> 74; 8 over 2, 8/8, 131,072
+  // tokens 104 -> 98.
+  if (D == 64 && S >= 16 && norm_words && int64_t(B) * Hq * S * max_pages >= kPairMin && rows_allowed())
+    sk = pick_split_pair(bw_k, bw_v, n_rep);
   if (!sk.fn) {
     const int g = valu_groups(n_rep);
     const int nrp = pad_nrep(n_rep / g);
@@ -524,15 +531,18 @@ static void fixed_plan(int B, int units_per_seq, int mp, int* pages_per_split, i
 }
 
 // Fixed splits for the row scan of head_dim 64: at most kPairWaves waves, the chip's two
-// per SIMD, each of whole chunks of 128 tokens. Every wave costs about 12 us before its
+// per SIMD, each of whole chunks of 128 tokens (or pages, where they are larger). Every wave costs about 12 us before its
 // first product, so a second round of them is dear: 2,048 / 3,072 / 4,096 waves take
 // 48 / 53 / 49 us (16 sequences of 3,000 to 12,000 tokens, 8 kv heads) and
-// 67 / 90 / 78 us (32 of 8,000).
-static constexpr int64_t kPairWaves = 2048;
+// 67 / 90 / 78 us (32 of 8,000). At most kPairSplits per unit, which the merge reads one after
+// another: one sequence of 131,072 tokens, 2 kv heads, 4/4 bits takes 45 / 46 / 68 us with
+// 256 / 512 / 1,024 of them (8/8 bits 49 / 53 / 73). At least two chunks per split: 4 sequences
+// of 32,768, 2 kv heads, 8/8 bits take 83 us a call by itself with two and 88 with one.
+static constexpr int64_t kPairWaves = 2048, kPairSplits = 256;
 static void pair_plan(int B, int Hkv, int S, int mp, int* pages_per_split, int* num_splits) {
   const int64_t units = int64_t(B > 0 ? B : 1) * Hkv, chunk = S < 128 ? 128 / S : 1;
-  const int64_t want = std::max<int64_t>(kPairWaves / units, 1);
-  const int64_t pps = std::min<int64_t>(((mp + want - 1) / want + chunk - 1) / chunk * chunk, mp);
+  const int64_t want = std::min(std::max<int64_t>(kPairWaves / units, 1), kPairSplits);
+  const int64_t pps = std::min<int64_t>(std::max(((mp + want - 1) / want + chunk - 1) / chunk, int64_t(2)) * chunk, mp);
   *pages_per_split = int(pps);
   *num_splits = int((mp + pps - 1) / pps);
 }
@@ -554,7 +564,7 @@ int decode_plan(int B, int Hq, int Hkv, int D, int S, int bw_k, int bw_v, int ma
     *pages_per_split = (mp + ns - 1) / ns;
     return WN_OK;
   }
-  const SplitKernel sk = choose_scan(Hq, Hkv, D, S, bw_k, bw_v, tf32);
+  const SplitKernel sk = choose_scan(B, Hq, Hkv, D, S, mp, bw_k, bw_v, tf32);
   if (sk.pair) {
     pair_plan(B, Hkv, S, mp, pages_per_split, num_splits);
     return WN_OK;
@@ -642,7 +652,7 @@ int decode_attention(
 
   const bool norm_words = aligned(k_norms, 4) && aligned(v_norms, 4) &&
                           (kn_stride_p | kn_stride_h | vn_stride_p | vn_stride_h) % 2 == 0;
-  const SplitKernel sk = choose_scan(Hq, Hkv, D, S, bw_k, bw_v, tf32, norm_words);
+  const SplitKernel sk = choose_scan(B, Hq, Hkv, D, S, max_pages, bw_k, bw_v, tf32, norm_words);
   RotFn rot = pick_rot_d(D, max(sk.nrep, 1));
   WN_REQUIRE(sk.fn && rot, WN_E_UNSUPPORTED, "decode: (D=%d, bw_k=%d, bw_v=%d) not compiled", D, bw_k,
              bw_v);
