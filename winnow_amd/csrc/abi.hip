@@ -1,4 +1,5 @@
 // Version, error reporting and split planning of the C ABI.
+#include <atomic>
 #include <cstdarg>
 
 #include "wn_common.h"
@@ -27,6 +28,16 @@ int check_launch(const char* what) {
     return WN_E_LAUNCH;
   }
   return WN_OK;
+}
+
+int device_cus() {
+  static std::atomic<int> known[64];
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 0;
+  if (dev < 64 && (cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
+  if (dev < 64) known[dev].store(cus, std::memory_order_relaxed);
+  return cus;
 }
 
 }  // namespace wn

@@ -211,10 +211,8 @@ int launch_rows(RowsArgs& a, int sides, hipStream_t st, const char* what) {
   WN_REQUIRE(a.rows < (int64_t(1) << 31), WN_E_INVALID, "%s: too many rows", what);
   a.vec = a.D % 4 == 0;
   for (int i = 0; i < sides; ++i) a.vec = a.vec && aligned(a.side[i].out, a.out_dtype == WN_F32 ? 16 : 8);
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
+  const int cus = device_cus();
+  WN_REQUIRE(cus > 0, WN_E_LAUNCH, "%s: cannot query the device", what);
   const int KD = a.D <= 64 ? 64 : a.D <= 128 ? 128 : 256, NR = KD == 64 ? 64 : 32;
   // three work-groups of four waves fit a CU (registers): each reads M once
   const int64_t tiles = (a.rows + NR - 1) / NR;

@@ -48,6 +48,7 @@
 // dot products; a launch of one pass per wave adds the staging and the latency of its
 // loads. Measured without gain: a touch of the next pass's rows ahead of it (40 us).
 #include <algorithm>
+#include <type_traits>
 
 #include "wn_quant.h"
 
@@ -165,8 +166,11 @@ __device__ __forceinline__ uint8_t* code8(TileWave<D>& w, int r, int k) {
   return w.code[r] + 8 * (k ^ ((r >> 1) & (D / 8 - 1)));
 }
 
+template <bool G2>
+using TileArgs = std::conditional_t<G2, QuantSplitArgs, QuantArgs>;
+
 template <int D, int DT, bool G2>
-__global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(QuantArgs a) {
+__global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(TileArgs<G2> a) {
   constexpr int WV = tile_waves<G2>();
   constexpr int KS = D / 32;  // K-steps of 32 input dims
   constexpr int U = D / 32;   // eights of output dims per lane (two MFMA row tiles each)
@@ -183,9 +187,13 @@ __global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(Qu
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int wig = __builtin_amdgcn_readfirstlane(tid >> 6);
   TileWave<D>& wv = waves[wig];
-  const int bw = sd.bw, split = G2 ? a.split : D;
+  const int bw = sd.bw;
+  QuantGroup2 s2{};
+  int split = D;
   uint32_t outl = 0;  // bit 8s + k: channel 32s + 8g + k is an outlier
   if constexpr (G2) {
+    s2 = a.second[blockIdx.y];
+    split = a.split;
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
@@ -197,7 +205,7 @@ __global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(Qu
   int64_t pass = int64_t(wig) * gridDim.x + blockIdx.x;
 #pragma unroll
   for (int q = 0; q < NG; ++q)
-    for (int i = tid; i < (1 << (q ? sd.bw2 : bw)) - 1; i += NTHR) bnd[q][i] = (q ? sd.bnd2 : sd.bnd)[i];
+    for (int i = tid; i < (1 << (q ? s2.bw : bw)) - 1; i += NTHR) bnd[q][i] = (q ? s2.bnd : sd.bnd)[i];
   for (int i = tid; i < D; i += NTHR) rowsq[i] = 0.f;
   __syncthreads();
   // operand (t, s, lane 16g + c): row r = c of tile t = 2u + h is output dim
@@ -228,7 +236,7 @@ __global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(Qu
   float eps[NG], inv_w[NG], at0[NG];
 #pragma unroll
   for (int q = 0; q < NG; ++q) {
-    const int qbw = q ? sd.bw2 : bw, nb = (1 << qbw) - 1;
+    const int qbw = q ? s2.bw : bw, nb = (1 << qbw) - 1;
     const float* bd = bnd[q];
     float rmax = 0.f;  // largest squared row norm (a NaN row is left out: its own dims' y are NaN, hence flagged)
 #pragma unroll
@@ -267,7 +275,7 @@ __global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(Qu
       o.x = b * sd.sb + h * sd.sh + i * sd.sn;
       int64_t page = -1, norm = 0;
       if (vec < a.total) {
-        if (G2) {
+        if constexpr (G2) {
           page = norm = (int64_t(b) * a.H + h) * a.cap + a.pos0 + i;  // the row's number
         } else if (!a.scatter) {
           page = vec * D;
@@ -411,29 +419,29 @@ __global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(Qu
       }
       sum += __shfl_xor(sum, 16, 64);
       sum += __shfl_xor(sum, 32, 64);
-      if (g == 0) code8<D>(wv, rr, dim >> 3)[dim & 7] = uint8_t(count_below(bnd[q2], q2 ? sd.bw2 : bw, float(sum)));
+      if (g == 0) code8<D>(wv, rr, dim >> 3)[dim & 7] = uint8_t(count_below(bnd[q2], q2 ? s2.bw : bw, float(sum)));
     }
     wave_lds_sync();
     if constexpr (G2) {
       // byte by byte: the bytes of both groups' rows, neighbouring lanes neighbouring bytes
-      const int nb1 = split * bw / 8, nb2 = (D - split) * sd.bw2 / 8, nball = nb1 + nb2;
+      const int nb1 = split * bw / 8, nb2 = (D - split) * s2.bw / 8, nball = nb1 + nb2;
       for (int i = lane; i < NR * nball; i += 64) {
         const int rr = i / nball, k = i % nball, q = k >= nb1;
         const int64_t row = wv.row[rr].page;
         if (row < 0) continue;
-        const int w = q ? sd.bw2 : bw, first = q ? split : 0, end = q ? D : split, bit0 = 8 * (q ? k - nb1 : k);
+        const int w = q ? s2.bw : bw, first = q ? split : 0, end = q ? D : split, bit0 = 8 * (q ? k - nb1 : k);
         uint32_t v = 0;
         for (int d = bit0 / w; first + d < end && d * w < bit0 + 8; ++d) {
           const int j = first + d, sh = d * w - bit0;
           const uint32_t cd = code8<D>(wv, rr, j >> 3)[j & 7];
           v |= sh >= 0 ? cd << sh : cd >> -sh;
         }
-        if (q) sd.pages2[row * nb2 + k - nb1] = uint8_t(v);
+        if (q) s2.pages[row * nb2 + k - nb1] = uint8_t(v);
         else sd.pages[row * nb1 + k] = uint8_t(v);
       }
       if (lane < NR && wv.row[lane].page >= 0) {
         sd.norms[wv.row[lane].norm] = f32_to_f16(wv.row[lane].n[0]);
-        sd.norms2[wv.row[lane].norm] = f32_to_f16(wv.row[lane].n[1]);
+        s2.norms[wv.row[lane].norm] = f32_to_f16(wv.row[lane].n[1]);
       }
       continue;
     }
@@ -466,10 +474,11 @@ __global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(Qu
   }
 }
 
-using TileFn = void (*)(QuantArgs);
+template <bool G2>
+using TileFn = void (*)(TileArgs<G2>);
 
 template <int D, bool G2>
-TileFn pick_tile(int dtype) {
+TileFn<G2> pick_tile(int dtype) {
   return dtype == WN_F32   ? quantize_tile_kernel<D, WN_F32, G2>
          : dtype == WN_F16 ? quantize_tile_kernel<D, WN_F16, G2>
                            : quantize_tile_kernel<D, WN_BF16, G2>;
@@ -497,22 +506,21 @@ bool quantize_tiles_ok(const QuantArgs& a, int sides, int D) {
   return a.total * sides >= (wide ? 16384 : 12288);
 }
 
-static int launch_tiles(TileFn fn, int waves, const QuantArgs& a, int sides, hipStream_t st) {
+template <bool G2>
+static int launch_tiles(TileFn<G2> fn, const TileArgs<G2>& a, int sides, hipStream_t st) {
   // one work-group per CU; its passes are dealt out from there
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return WN_E_LAUNCH;
+  const int cus = device_cus();
+  if (cus <= 0) return WN_E_LAUNCH;
   const int64_t groups = std::min<int64_t>((a.total + kTileVecs - 1) / kTileVecs, std::max(1, cus / sides));
-  hipLaunchKernelGGL(fn, dim3(unsigned(groups), sides), dim3(64 * waves), 0, st, a);
+  hipLaunchKernelGGL(fn, dim3(unsigned(groups), sides), dim3(64 * tile_waves<G2>()), 0, st, a);
   return WN_OK;
 }
 
 int launch_quantize_tiles(const QuantArgs& a, int sides, int D, hipStream_t st) {
-  return launch_tiles(D == 64 ? pick_tile<64, false>(a.x_dtype) : pick_tile<128, false>(a.x_dtype), tile_waves<false>(), a, sides, st);
+  return launch_tiles<false>(D == 64 ? pick_tile<64, false>(a.x_dtype) : pick_tile<128, false>(a.x_dtype), a, sides, st);
 }
 
-bool quantize_split_ok(const QuantArgs& a, int sides, int D) {
+bool quantize_split_ok(const QuantSplitArgs& a, int sides, int D) {
   if ((D != 64 && D != 128) || a.total >= (int64_t(1) << 31)) return false;
   const int es = a.x_dtype == WN_F32 ? 4 : 2;
   for (int i = 0; i < sides; ++i)
@@ -520,8 +528,8 @@ bool quantize_split_ok(const QuantArgs& a, int sides, int D) {
   return true;
 }
 
-int launch_quantize_split(const QuantArgs& a, int sides, int D, hipStream_t st) {
-  return launch_tiles(D == 64 ? pick_tile<64, true>(a.x_dtype) : pick_tile<128, true>(a.x_dtype), tile_waves<true>(), a, sides, st);
+int launch_quantize_split(const QuantSplitArgs& a, int sides, int D, hipStream_t st) {
+  return launch_tiles<true>(D == 64 ? pick_tile<64, true>(a.x_dtype) : pick_tile<128, true>(a.x_dtype), a, sides, st);
 }
 
 }  // namespace wn

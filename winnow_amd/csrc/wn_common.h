@@ -25,6 +25,9 @@ void clear_error();
 
 int check_launch(const char* what);
 
+// Compute units of the current device, asked for once per device; 0: the query failed.
+int device_cus();
+
 inline bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 inline int ilog2(int64_t x) {
   int r = 0;

@@ -18,11 +18,6 @@ struct QuantSide {
   int64_t nsp, nsh;
   uint8_t* codes_out;  // flat mode
   float* norms_out;
-  // outlier channels (launch_quantize_split): boundaries, width, rows and norms of the second group
-  const float* bnd2;
-  int bw2;
-  uint8_t* pages2;
-  uint16_t* norms2;
 };
 
 struct QuantArgs {
@@ -32,10 +27,21 @@ struct QuantArgs {
   int64_t tsb;
   int64_t total;  // vectors per side = B*H*n
   int H, n, log2S, num_pages, max_pages, x_dtype, scatter;
-  // launch_quantize_split: group of each channel, codes of group 0, rows per (sequence, head), first position
-  const uint8_t* chan;
-  int split, pos0;
-  int64_t cap;
+};
+
+// Outlier channels (launch_quantize_split): boundaries, width, rows and norms of the second group.
+struct QuantGroup2 {
+  const float* bnd;
+  int bw;
+  uint8_t* pages;
+  uint16_t* norms;
+};
+
+struct QuantSplitArgs : QuantArgs {
+  QuantGroup2 second[2];  // K, V
+  const uint8_t* chan;    // group of each channel
+  int split, pos0;        // codes of group 0, first position
+  int64_t cap;            // rows per (sequence, head)
 };
 
 // pos[k] = #{b < y[k]} over the 2^bw - 1 ascending boundaries (torch.bucketize,
@@ -77,7 +83,7 @@ bool quantize_tiles_ok(const QuantArgs& a, int sides, int D);
 int launch_quantize_tiles(const QuantArgs& a, int sides, int D, hipStream_t st);
 // The same kernel with two groups of channels, rows of a contiguous cache (quant.hip's
 // wn_append_split).
-bool quantize_split_ok(const QuantArgs& a, int sides, int D);
-int launch_quantize_split(const QuantArgs& a, int sides, int D, hipStream_t st);
+bool quantize_split_ok(const QuantSplitArgs& a, int sides, int D);
+int launch_quantize_split(const QuantSplitArgs& a, int sides, int D, hipStream_t st);
 
 }  // namespace wn
