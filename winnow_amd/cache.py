@@ -276,6 +276,9 @@ class TQPackedLayer(DynamicLayer):
     def _check_step(self, k: torch.Tensor, v: torch.Tensor) -> None:
         """The kernels address the buffers by K's sizes: K and V have one shape, the buffers'
         batch, heads and head_dim (``reset`` keeps the buffers), and lie on their device."""
+        if (self.is_initialized and v.shape == k.shape and len(k.shape) == 4 and (*k.shape[:2], k.shape[3]) == self._dims
+                and k.device == v.device == self.device):
+            return
         if k.dim() != 4 or v.shape != k.shape:
             raise ValueError(f"TQPackedLayer: K {tuple(k.shape)} and V {tuple(v.shape)} must be (B, H, n, D) alike")
         if v.device != k.device:

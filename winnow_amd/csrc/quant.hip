@@ -557,10 +557,10 @@ extern "C" int wn_append_split(
              WN_E_INVALID, "append_split: null operand");
   WN_REQUIRE(aligned(m, 16), WN_E_INVALID, "append_split: the rotations need 16-byte aligned rows");
   QuantSplitArgs a{};
-  a.side[0] = QuantSide{k, ks_b, ks_h, ks_n, m, boundaries, bw, k_codes, 0, 0, k_norms, 0, 0, nullptr, nullptr};
-  a.side[1] = QuantSide{v, vs_b, vs_h, vs_n, m, boundaries, bw, v_codes, 0, 0, v_norms, 0, 0, nullptr, nullptr};
-  a.second[0] = QuantGroup2{boundaries2, bw2, k_codes2, k_norms2};
-  a.second[1] = QuantGroup2{boundaries2, bw2, v_codes2, v_norms2};
+  a.side[0] = QuantSplitSide{{k, ks_b, ks_h, ks_n, m, boundaries, bw, k_codes, 0, 0, k_norms, 0, 0, nullptr, nullptr},
+                             {boundaries2, bw2, k_codes2, k_norms2}};
+  a.side[1] = QuantSplitSide{{v, vs_b, vs_h, vs_n, m, boundaries, bw, v_codes, 0, 0, v_norms, 0, 0, nullptr, nullptr},
+                             {boundaries2, bw2, v_codes2, v_norms2}};
   a.total = int64_t(B) * H * n;
   a.H = H;
   a.n = n;

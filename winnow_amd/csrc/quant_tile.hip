@@ -168,6 +168,9 @@ __device__ __forceinline__ uint8_t* code8(TileWave<D>& w, int r, int k) {
 
 template <bool G2>
 using TileArgs = std::conditional_t<G2, QuantSplitArgs, QuantArgs>;
+// The second group of a side that has one; else `none`.
+__device__ __forceinline__ const QuantGroup2& second_group(const QuantSplitSide& s, const QuantGroup2&) { return s.second; }
+__device__ __forceinline__ const QuantGroup2& second_group(const QuantSide&, const QuantGroup2& none) { return none; }
 
 template <int D, int DT, bool G2>
 __global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(TileArgs<G2> a) {
@@ -183,16 +186,16 @@ __global__ __launch_bounds__(64 * tile_waves<G2>()) void quantize_tile_kernel(Ti
   __shared__ float rowsq[D];
   __shared__ TileWave<D> waves[WV];
 
-  const QuantSide& sd = a.side[blockIdx.y];
+  const auto& sd = a.side[blockIdx.y];
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15;
   const int wig = __builtin_amdgcn_readfirstlane(tid >> 6);
   TileWave<D>& wv = waves[wig];
   const int bw = sd.bw;
-  QuantGroup2 s2{};
+  const QuantGroup2 none{};
+  const QuantGroup2& s2 = second_group(sd, none);
   int split = D;
   uint32_t outl = 0;  // bit 8s + k: channel 32s + 8g + k is an outlier
   if constexpr (G2) {
-    s2 = a.second[blockIdx.y];
     split = a.split;
 #pragma unroll
     for (int s = 0; s < KS; ++s)

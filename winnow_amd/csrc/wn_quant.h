@@ -20,14 +20,16 @@ struct QuantSide {
   float* norms_out;
 };
 
-struct QuantArgs {
-  QuantSide side[2];
+template <class Side>
+struct QuantArgsOf {
+  Side side[2];  // K, V
   const int32_t* table;
   const int32_t* start_pos;
   int64_t tsb;
   int64_t total;  // vectors per side = B*H*n
   int H, n, log2S, num_pages, max_pages, x_dtype, scatter;
 };
+using QuantArgs = QuantArgsOf<QuantSide>;
 
 // Outlier channels (launch_quantize_split): boundaries, width, rows and norms of the second group.
 struct QuantGroup2 {
@@ -37,8 +39,11 @@ struct QuantGroup2 {
   uint16_t* norms;
 };
 
-struct QuantSplitArgs : QuantArgs {
-  QuantGroup2 second[2];  // K, V
+struct QuantSplitSide : QuantSide {
+  QuantGroup2 second;
+};
+
+struct QuantSplitArgs : QuantArgsOf<QuantSplitSide> {
   const uint8_t* chan;    // group of each channel
   int split, pos0;        // codes of group 0, first position
   int64_t cap;            // rows per (sequence, head)
