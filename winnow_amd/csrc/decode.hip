@@ -928,8 +928,8 @@ extern "C" int wn_dense_decode_attention(
   da.balanced = balanced ? 1 : 0;
   da.qrows = pad_nrep(n_rep_s);
   const int64_t waves = balanced ? int64_t(num_splits) : int64_t(num_splits) * Hkv_s * B;
-  // the MFMA scan numbers its waves across work-groups of sk.wpb waves; the fp32 scan
-  // runs one work-group per (split, virtual kv head, sequence)
+  // the MFMA scan numbers its waves across work-groups of sk.wpb waves; the scan of fp32
+  // pages runs one work-group per (split, virtual kv head, sequence)
   const dim3 grid = sk.rows ? dim3(unsigned((waves + sk.wpb - 1) / sk.wpb)) : dim3(num_splits, Hkv_s, B);
   if (ev_begin) hipEventRecord(static_cast<hipEvent_t>(ev_begin), st);
   hipLaunchKernelGGL(sk.fn, grid, dim3(sk.block), 0, st, da);

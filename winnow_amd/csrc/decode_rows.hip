@@ -1,44 +1,31 @@
-// Row-per-lane matrix-core page scan of the packed decode attention (head_dim 128,
-// power-of-two page size >= 16, up to eight query heads per (virtual) kv head in one
-// or two groups of four; the host runs an even n_rep of 10..16 as two virtual kv
-// heads per kv head, kvshift), gfx950.
+// Row-per-lane matrix-core page scan of the packed decode attention (power-of-two page
+// size >= 16), gfx950: head_dim 128 with up to eight query heads per (virtual) kv head in
+// one or two groups of four (the host runs an even n_rep of 10..16 as two virtual kv
+// heads per kv head, kvshift), and head_dim 64 with up to four, two tokens to a 128-wide
+// row (PAIR). Every product runs on v_mfma_f32_16x16x32_f16, on fp16 pairs
+// (decode_rows16_kernel) or, for allow_tf32, on single fp16 operands
+// (decode_rows_tf_kernel).
 //
 // Waves are independent of each other; the waves of a work-group only share the
 // codebook tables staged in LDS. With fixed splits a wave owns a range of pages of
 // one (sequence, kv head); with a balanced plan
 // the resident waves split the flattened (sequence, kv head, chunk) space into
-// equal shares. Either way a wave walks its tokens in 64-token chunks.
+// equal shares. Either way a wave walks its tokens in 64-token chunks: scores, online
+// softmax, values.
 //
-//   scores  lane l holds the packed K row of token c0+l. For each dim k one
-//           v_mfma_f32_4x4x1_16b_f32 per group of four heads, with A = q_rot[head i][k]
-//           broadcast to all 16 blocks (CBSZ=4, ABID=k%16) and B = c_K[code(token, k)],
-//           gives D[block][i][j] = partial s(head i, token 4*block+j): lane l ends
-//           with its own token's scores. 128 MFMAs per chunk and head group; each
-//           codebook lookup feeds every group.
 //   softmax per head in log2 units (q_rot carries log2 e), lane = token, with a
 //           lazy reference maximum: it moves (rescaling the accumulators) only
 //           when a score exceeds it by more than kRescale, so 2^(s - m) <= 2^kRescale.
-//   values  p * n_V goes through a 1.3 KB LDS tile so that lanes 16G+i hold
-//           p(head i, token c0+4q+G) for the 16 token quads q. Lanes 16G..16G+15
-//           hold the packed V codes of dims 8p..8p+7 (p = lane%16) of that token.
-//           A v_mfma_f32_4x4x1_16b_f32 with CBSZ=2 broadcasts A inside each group of
-//           four blocks, so block group G accumulates token c0+4q+G into
-//           acc[m] register i = (head i, dim 8p+m). 8 MFMAs per quad, 128 per chunk;
-//           the four groups are folded once per split.
 //
-// Codebooks sit in LDS; every product is an exact fp32 multiply-add. 4-bit codes
-// are looked up two at a time in a byte-indexed table of (c[lo nibble], c[hi nibble])
-// pairs that is replicated once per lane of a half-wave, so that the 32 lanes LDS
-// serves together always read 32 distinct bank pairs: a lookup never waits on a
-// bank conflict, whatever the codes. Twelve waves per work-group (eight with two
-// head groups or wider codes) share the tables.
+// 4-bit codes are looked up two at a time in a byte-indexed table of (c[lo nibble], c[hi
+// nibble]) pairs that is replicated once per lane of a half-wave, so that the 32 lanes
+// LDS serves together always read 32 distinct bank pairs: a lookup never waits on a
+// bank conflict, whatever the codes.
 // Page ids run two chunks ahead and the packed rows of chunk c+1 load while chunk c
 // computes.
 // Algebra: turboquant_kv/packed_attention.py:260-334 (the schedule of the
 // reference kernel packed_attention_triton.py:51-134).
 #include <cfloat>
-#include <cstdlib>
-#include <cstring>
 #include <type_traits>
 #include <utility>
 
@@ -48,24 +35,7 @@
 namespace wn {
 namespace {
 
-
-
 constexpr float kRescale = 8.0f;
-constexpr int kPStride = 20;  // floats per (head, token group) row of the p tile (16 + pad, 16-B rows)
-
-template <int K>
-__device__ __forceinline__ float comp(const float4& x) {
-  if constexpr (K == 0) return x.x;
-  else if constexpr (K == 1) return x.y;
-  else if constexpr (K == 2) return x.z;
-  else return x.w;
-}
-
-// Row of the p tile lane 16G+i reads its value-MFMA operands of head group g from:
-// p(head 4g+i, token c0+4q+G) * n_V sits at row 16g + 4i + G, column q.
-__device__ __forceinline__ const float4* tile_row(const float* pt, int g, int lane) {
-  return reinterpret_cast<const float4*>(pt + (16 * g + (lane & 3) * 4 + (lane >> 4)) * kPStride);
-}
 
 constexpr int kPairTableBytes = 256 * 32 * 8;  // 256 byte values x 32 lanes x float2
 
@@ -75,18 +45,18 @@ constexpr int kPairTableBytes = 256 * 32 * 8;  // 256 byte values x 32 lanes x f
 template <int BW>
 constexpr bool pair_coded() { return BW == 2 || BW == 3 || BW == 5 || BW == 6; }
 
-// LDS bytes the codebook of BW-bit codes occupies: the replicated pair table for
-// 4-bit codes, the pair table of pair_coded widths, else the plain 2^BW-entry table
-// (padded to 16 bytes).
+// LDS bytes of the table of BW-bit codes: the replicated pair table for 4-bit codes, else the
+// pair table of pair_coded widths.
 template <int BW>
 constexpr int table_bytes() {
-  return BW == 4 ? kPairTableBytes : pair_coded<BW>() ? (8 << (2 * BW)) : (4 << BW) < 16 ? 16 : (4 << BW);
+  static_assert(BW == 4 || pair_coded<BW>());
+  return BW == 4 ? kPairTableBytes : 8 << (2 * BW);
 }
 
 // A codebook in LDS as one lane reads it.
 template <int BW>
 struct Tab {
-  const float* t;  // plain table: lanes sharing a code share an address (LDS broadcasts)
+  const float* t;  // pair table: lanes sharing a pair share an address (LDS broadcasts)
 };
 template <>
 struct Tab<4> {
@@ -98,64 +68,6 @@ struct Tab<4> {
     for (int k = 0; k < 4; ++k) r[k] = uint32_t(8 * (lane & 31)) | (uint32_t(slot) << 16);
   }
 };
-
-// Stages a codebook into LDS at `dst` with all `nthr` threads of the work-group:
-// the replicated pair table for 4-bit codes (entry (b, r) at byte 256*b + 8*r holds
-// (c[b & 15], c[b >> 4])), the pair table of pair_coded widths (entry i holds
-// (c[i mod 2^BW], c[i >> BW]): two consecutive codes, LSB first, read as one
-// 2*BW-bit index), else the plain table.
-template <int BW, int NTHR>
-__device__ __forceinline__ void stage_table(const float* cb, char* dst, int tid) {
-  if constexpr (BW == 4) {
-    float2* t = reinterpret_cast<float2*>(dst);
-    for_strided<256 * 32, NTHR>(tid, [&](int i) {
-      const int b = i >> 5;
-      t[i] = make_float2(cb[b & 15], cb[b >> 4]);
-    });
-  } else if constexpr (pair_coded<BW>()) {
-    float2* t = reinterpret_cast<float2*>(dst);
-    for_strided<(1 << (2 * BW)), NTHR>(tid, [&](int i) { t[i] = make_float2(cb[i & ((1 << BW) - 1)], cb[i >> BW]); });
-  } else {
-    float* t = reinterpret_cast<float*>(dst);
-    for_strided<(1 << BW), NTHR>(tid, [&](int i) { t[i] = cb[i]; });
-  }
-}
-
-// Codebook values of the 8 codes starting at bit BIT0 of the word array (LSB-first,
-// BW bits each) into v[0..7]: one SDWA move and one 8-byte LDS read per two 4-bit
-// codes; one 2*BW-bit extract and one 8-byte read per two codes of a pair_coded
-// width; 8-bit codes are read one by one from the plain table.
-template <int BW, int BIT0, int NW>
-__device__ __forceinline__ void lookup8(const uint32_t (&w)[NW], Tab<BW>& tab, float (&v)[8]) {
-  if constexpr (BW == 4) {
-    static_assert(BIT0 % 32 == 0, "4-bit groups are word aligned");
-    static_for<0, 4>([&](auto kc) {
-      constexpr int k = decltype(kc)::value;
-      tab.r[k] = put_byte1<k>(tab.r[k], w[BIT0 / 32]);
-      const float2 e = *reinterpret_cast<const float2*>(tab.lds + tab.r[k]);
-      v[2 * k] = e.x;
-      v[2 * k + 1] = e.y;
-    });
-  } else if constexpr (pair_coded<BW>()) {
-    static_for<0, 4>([&](auto kc) {
-      constexpr int k = decltype(kc)::value;
-      constexpr int bit = BIT0 + 2 * BW * k, wi = bit >> 5, sh = bit & 31;
-      uint32_t x = w[wi] >> sh;
-      if constexpr (sh + 2 * BW > 32) x |= w[wi + 1] << (32 - sh);
-      const float2 e = reinterpret_cast<const float2*>(tab.t)[x & ((1u << (2 * BW)) - 1u)];
-      v[2 * k] = e.x;
-      v[2 * k + 1] = e.y;
-    });
-  } else {
-    static_for<0, 8>([&](auto jc) {
-      constexpr int j = decltype(jc)::value;
-      constexpr int bit = BIT0 + j * BW, wi = bit >> 5, sh = bit & 31;
-      uint32_t x = w[wi] >> sh;
-      if constexpr (sh + BW > 32) x |= w[wi + 1] << (32 - sh);
-      v[j] = tab.t[x & ((1u << BW) - 1u)];
-    });
-  }
-}
 
 // s_waitcnt vmcnt(0) (expcnt and lgkmcnt left at their maxima): every vector
 // memory load this wave issued has returned.
@@ -174,8 +86,9 @@ struct VWords {
   static constexpr int N = BWV <= 4 ? 1 : 2;
 };
 
-// One buffer of packed rows. As a K buffer it holds the packed K row of token
-// c0 + lane (words [0, KW)) and that token's fp16 K and V norms (words KW, KW+1);
+// One buffer of packed rows. As a K buffer it holds, for each tile t, the 4 BWK bytes of
+// quarter g of token 16t + 4(c%4) + c/4 (lane 16g + c; words [t*BWK, t*BWK + BWK)) and the
+// fp16 K and V norms of token c0 + lane (words KW, KW+1);
 // as a V buffer, for each token quad q, the codes 8p..8p+7 of token c0 + 4q + G
 // (G = lane/16, p = lane%16) at words [q*VW, q*VW + VW). A chunk's K buffer is
 // refilled with the next chunk's V codes once the softmax has used the norms.
@@ -245,34 +158,6 @@ __device__ __forceinline__ void load_vcodes(const uint8_t* p, bool odd_lane, uin
   }
 }
 
-// Running state of NG groups of four query heads (head 4g+i is register i of group g).
-template <int NG>
-struct RowState {
-  f32x4 acc[NG][8];  // acc[g][m] register i: head 4g+i, dim 8p+m (partial over this lane's token group)
-  float m[4 * NG];   // reference maxima (wave-uniform), log2 units
-  float l[4 * NG];   // sum of 2^(s - m) over this lane's tokens
-};
-
-// K side of chunk [c0, c0+64): the packed K row and both norms of token c0+lane,
-// whose page is pid_lane.
-template <int BWK, int BWV>
-__device__ __forceinline__ void load_k(const DecodeArgs& a, int kvh, int lane, int c0, int pid_lane,
-                                       RowBuf<BWK, BWV>& r) {
-  constexpr int NBK = 16 * BWK, KW = RowBuf<BWK, BWV>::KW;
-  const int slot = (c0 + lane) & ((1 << a.log2S) - 1);
-  const uint8_t* krow = a.k_pages + int64_t(pid_lane) * a.ksp + (kvh >> a.kvshift) * a.ksh + slot * NBK;
-#pragma unroll
-  for (int i = 0; i < NBK / 16; ++i) {
-    const uint4 x = reinterpret_cast<const uint4*>(krow)[i];
-    r.w[4 * i] = x.x;
-    r.w[4 * i + 1] = x.y;
-    r.w[4 * i + 2] = x.z;
-    r.w[4 * i + 3] = x.w;
-  }
-  r.w[KW] = a.k_norms[int64_t(pid_lane) * a.knp + (kvh >> a.kvshift) * a.knh + slot];
-  r.w[KW + 1] = a.v_norms[int64_t(pid_lane) * a.vnp + (kvh >> a.kvshift) * a.vnh + slot];
-}
-
 // A page-block address formed on the device (block_bases) as a pointer into global memory: the address space is
 // stated, so loads through it stay global loads (a plain pointer rebuilt from an integer
 // would make them flat loads, which also count against the LDS wait counter).
@@ -316,299 +201,6 @@ __device__ __forceinline__ void load_v(const DecodeArgs& a, int kvh, int lane, i
     });
   });
 }
-
-// Score lookups of dims [8g, 8g+8) of this lane's K row.
-template <int BWK, int G, int NW>
-__device__ __forceinline__ void score_look(const uint32_t (&k)[NW], Tab<BWK>& cbk, float (&kv)[8]) {
-  lookup8<BWK, 8 * G * BWK>(k, cbk, kv);
-}
-
-// The score MFMAs of dims [8g, 8g+8), eight per head group: A = q_rot[head][k]
-// broadcast from block k%16; every lookup feeds one MFMA per group.
-template <int G, int NG>
-__device__ __forceinline__ void score_mfma(const float (&qb)[NG][8], const float (&kv)[8], f32x4 (&s0)[NG],
-                                           f32x4 (&s1)[NG]) {
-  static_for<0, 8>([&](auto jc) {
-    constexpr int j = decltype(jc)::value, k = 8 * G + j;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      if constexpr (j & 1)
-        s1[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(qb[g][k >> 4], kv[j], s1[g], 4, k & 15, 0);
-      else
-        s0[g] = __builtin_amdgcn_mfma_f32_4x4x1f32(qb[g][k >> 4], kv[j], s0[g], 4, k & 15, 0);
-    }
-  });
-}
-
-// Value lookups of quad q (this lane's 8 dims of token c0+4q+G).
-template <int BWV, int Q, int NW>
-__device__ __forceinline__ void value_look(const uint32_t (&v)[NW], Tab<BWV>& cbv, float (&vv)[8]) {
-  lookup8<BWV, 32 * VWords<BWV>::N * Q>(v, cbv, vv);
-}
-
-// The value MFMAs of quad q, eight per head group: A = p*n_V broadcast inside each
-// group of four blocks.
-template <int NG>
-__device__ __forceinline__ void value_mfma(const float (&a_q)[NG], const float (&vv)[8], f32x4 (&acc)[NG][8]) {
-  static_for<0, 8>([&](auto mc) {
-    constexpr int mm = decltype(mc)::value;
-#pragma unroll
-    for (int g = 0; g < NG; ++g) acc[g][mm] = __builtin_amdgcn_mfma_f32_4x4x1f32(a_q[g], vv[mm], acc[g][mm], 2, 0, 0);
-  });
-}
-
-// Scores of the chunk's 64 tokens (lane = token, register i = head i). The
-// lookups of group g+2 are issued before the MFMAs of group g, so every LDS read
-// has sixteen of this wave's MFMAs to land before its value is needed; the sched
-// barriers keep the compiler from sinking the reads next to their consumers.
-template <int BWK, int NG, int NW>
-__device__ __forceinline__ void score_phase(const uint32_t (&kc)[NW], Tab<BWK>& cbk, const float (&qb)[NG][8],
-                                            f32x4 (&out)[NG]) {
-  f32x4 s0[NG], s1[NG];
-#pragma unroll
-  for (int g = 0; g < NG; ++g) s0[g] = s1[g] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float kv[3][8];
-  score_look<BWK, 0>(kc, cbk, kv[0]);
-  score_look<BWK, 1>(kc, cbk, kv[1]);
-  __builtin_amdgcn_sched_barrier(0);
-  static_for<0, 16>([&](auto gc) {
-    constexpr int g = decltype(gc)::value;
-    if constexpr (g + 2 < 16) {
-      score_look<BWK, g + 2>(kc, cbk, kv[(g + 2) % 3]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    score_mfma<g, NG>(qb, kv[g % 3], s0, s1);
-    __builtin_amdgcn_sched_barrier(0);
-  });
-#pragma unroll
-  for (int g = 0; g < NG; ++g) out[g] = s0[g] + s1[g];
-}
-
-// Lookups of the first two value quads, issued before the softmax so that they
-// land while it runs.
-template <int BWV, int NW>
-__device__ __forceinline__ void value_prime(const uint32_t (&vc)[NW], Tab<BWV>& cbv, float (&vv)[3][8]) {
-  value_look<BWV, 0>(vc, cbv, vv[0]);
-  value_look<BWV, 1>(vc, cbv, vv[1]);
-  __builtin_amdgcn_sched_barrier(0);
-}
-
-// Values of a chunk; lookups of quad q+2 are issued before the MFMAs of quad q,
-// and the p * n_V operands of four quads are read from the tile two quads before
-// the first of them.
-template <int BWV, int NG, int NW>
-__device__ __forceinline__ void value_phase(const uint32_t (&vc)[NW], Tab<BWV>& cbv, const float* pt, int lane,
-                                            f32x4 (&acc)[NG][8], float (&vv)[3][8]) {
-  const float4* arow[NG];
-  float4 ab[NG][2];
-#pragma unroll
-  for (int g = 0; g < NG; ++g) {
-    arow[g] = tile_row(pt, g, lane);
-    ab[g][0] = arow[g][0];
-  }
-  static_for<0, 16>([&](auto qc) {
-    constexpr int q = decltype(qc)::value;
-    if constexpr ((q & 3) == 2 && q + 2 < 16) {
-#pragma unroll
-      for (int g = 0; g < NG; ++g) ab[g][((q >> 2) + 1) & 1] = arow[g][(q >> 2) + 1];
-    }
-    if constexpr (q + 2 < 16) value_look<BWV, q + 2>(vc, cbv, vv[(q + 2) % 3]);
-    __builtin_amdgcn_sched_barrier(0);
-    float aq[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) aq[g] = comp<q & 3>(ab[g][(q >> 2) & 1]);
-    value_mfma<NG>(aq, vv[q % 3], acc);
-    __builtin_amdgcn_sched_barrier(0);
-  });
-}
-
-// Online softmax of one chunk (lane = token) and the p * n_V transposition: on
-// return the tile holds p(head 4g+i, token c0+4q+G) * n_V at row 16g+4i+G, column q,
-// and lane 16G+i finds its value-MFMA operands of group g for quads 4j..4j+3 at
-// float4 j of row 16g + 4(lane%4) + lane/16 (tile_row).
-template <int NG>
-__device__ __forceinline__ void softmax_phase(const f32x4 (&s)[NG], uint32_t nk_h, uint32_t nv_h, bool valid,
-                                              int lane, float* pt, RowState<NG>& st) {
-  constexpr int H = 4 * NG;
-  const float nk = half_lo(nk_h);
-  const float nv = valid ? half_lo(nv_h) : 0.f;
-  float sv[H];
-#pragma unroll
-  for (int i = 0; i < H; ++i) sv[i] = valid ? s[i >> 2][i & 3] * nk : -INFINITY;
-  bool move = st.m[0] == -INFINITY;
-#pragma unroll
-  for (int i = 0; i < H; ++i) move = move || __any(sv[i] > st.m[i] + kRescale);
-  if (move) {  // wave-uniform
-#pragma unroll
-    for (int i = 0; i < H; ++i) {
-      // wave-uniform: kept in a scalar register, which frees a VGPR per head
-      const float m_new = uniform(fmaxf(st.m[i], wave_max(sv[i])));
-      const float alpha = __builtin_amdgcn_exp2f(st.m[i] - m_new);  // 0 on the first chunk
-      st.m[i] = m_new;
-      st.l[i] *= alpha;
-#pragma unroll
-      for (int mm = 0; mm < 8; ++mm) st.acc[i >> 2][mm][i & 3] *= alpha;
-    }
-  }
-  float pv[H];
-#pragma unroll
-  for (int i = 0; i < H; ++i) {
-    const float p = __builtin_amdgcn_exp2f(sv[i] - st.m[i]);  // 0 for masked tokens
-    st.l[i] += p;
-    pv[i] = p * nv;
-  }
-  wave_lds_sync();  // the previous chunk's reads of the tile are done
-  {
-    const int G = lane & 3, q = lane >> 2;
-#pragma unroll
-    for (int i = 0; i < H; ++i) pt[(16 * (i >> 2) + (i & 3) * 4 + G) * kPStride + q] = pv[i];
-  }
-  wave_lds_sync();
-}
-
-
-
-// Folds the four token groups and the per-lane sums and writes the (acc, m, l)
-// partial of each query head h < n_rep to row prow * n_rep + h.
-template <int NG>
-__device__ __forceinline__ void write_partial(const DecodeArgs& a, RowState<NG>& st, int64_t prow, int lane) {
-  constexpr int D = 128, H = 4 * NG;
-#pragma unroll
-  for (int g = 0; g < NG; ++g)
-#pragma unroll
-    for (int mm = 0; mm < 8; ++mm)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        float x = st.acc[g][mm][i];
-        x += __shfl_xor(x, 16, 64);
-        x += __shfl_xor(x, 32, 64);
-        st.acc[g][mm][i] = x;
-      }
-#pragma unroll
-  for (int i = 0; i < H; ++i) st.l[i] = wave_sum(st.l[i]);
-  const int64_t row0 = prow * a.n_rep;
-  if (lane < 16) {  // lane p: dims 8p..8p+7 of every head
-#pragma unroll
-    for (int i = 0; i < H; ++i) {
-      if (i < a.n_rep) {
-        const f32x4* ac = st.acc[i >> 2];
-        float* dst = a.part_acc + (row0 + i) * D + 8 * lane;
-        *reinterpret_cast<float4*>(dst) = make_float4(ac[0][i & 3], ac[1][i & 3], ac[2][i & 3], ac[3][i & 3]);
-        *reinterpret_cast<float4*>(dst + 4) = make_float4(ac[4][i & 3], ac[5][i & 3], ac[6][i & 3], ac[7][i & 3]);
-      }
-    }
-  }
-  // m and l are wave-uniform: lane 0 writes every head's (a lane-indexed pick would
-  // turn the register arrays into an indexed stack object)
-  if (lane == 0) {
-#pragma unroll
-    for (int i = 0; i < H; ++i) {
-      if (i < a.n_rep) {
-        a.part_ml[2 * (row0 + i)] = st.m[i];
-        a.part_ml[2 * (row0 + i) + 1] = st.l[i];
-      }
-    }
-  }
-}
-
-// Scans tokens [t_lo, t_hi) of (sequence b, kv head kvh) in 64-token chunks (t_lo a
-// multiple of 16) and writes one partial at row prow. Each chunk runs score,
-// softmax and values in turn; the packed codes of chunk c+1 load while chunk c
-// computes and page ids run two chunks ahead.
-template <int BWK, int BWV, int NG>
-__device__ __forceinline__ void scan_range(const DecodeArgs& a, int b, int kvh, int t_lo, int t_hi, int64_t prow,
-                                           int lane, Tab<BWK>& cbk, Tab<BWV>& cbv, float* ptile) {
-  constexpr int D = 128;
-  const int page_hi = (t_hi + (1 << a.log2S) - 1) >> a.log2S;
-  const int n = (t_hi - t_lo + 63) >> 6;
-
-  // register m of group g of lane 4j+i holds q_rot[head 4g+i][16m + j]
-  float qb[NG][8];
-#pragma unroll
-  for (int g = 0; g < NG; ++g) {
-    const float* qp = a.q_rot + ((int64_t(b) * a.Hkv + kvh) * (4 * NG) + 4 * g + (lane & 3)) * D + (lane >> 2);
-#pragma unroll
-    for (int m = 0; m < 8; ++m) qb[g][m] = qp[16 * m];
-  }
-  const int32_t* trow = a.table + b * a.tsb;
-  // page of this lane's token in chunk c (tokens past the range read its last page and are masked)
-  auto pid_of = [&](int c) {
-    const int col = min((t_lo + 64 * c + lane) >> a.log2S, page_hi - 1);
-    return trow[col];
-  };
-
-  RowState<NG> st;
-#pragma unroll
-  for (int g = 0; g < NG; ++g)
-#pragma unroll
-    for (int mm = 0; mm < 8; ++mm) st.acc[g][mm] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int i = 0; i < 4 * NG; ++i) {
-    st.m[i] = -INFINITY;
-    st.l[i] = 0.f;
-  }
-  using Buf = RowBuf<BWK, BWV>;
-  // Chunk c with its K rows in X and its V codes in Y; Z is free. The K rows of
-  // chunk c+1 load into Z at the start, its V codes into X once the softmax has
-  // read the norms, so each load has about one chunk of compute to land, and
-  // three buffers rotate through the roles: (X, Y, Z) -> (Z, X, Y).
-  int pid_next;
-  auto step = [&](int c, Buf& X, Buf& Y, Buf& Z) {
-    const int c0 = t_lo + 64 * c;
-    // page ids two chunks ahead, issued before the next chunk's rows, so the wait
-    // for them never waits for those rows; clamped, so always a valid read
-    const int pid_after = pid_of(c + 2);
-    const bool more = c + 1 < n;
-    if (more) load_k(a, kvh, lane, c0 + 64, pid_next, Z);
-    float vv[3][8];
-    f32x4 s[NG];
-    score_phase<BWK, NG>(X.w, cbk, qb, s);
-    value_prime<BWV>(Y.w, cbv, vv);
-    softmax_phase<NG>(s, X.w[Buf::KW], X.w[Buf::KW + 1], c0 + lane < t_hi, lane, ptile, st);
-    if (more) load_v(a, kvh, lane, c0 + 64, pid_next, X);
-    value_phase<BWV, NG>(Y.w, cbv, ptile, lane, st.acc, vv);
-    pid_next = pid_after;
-  };
-
-  Buf b0, b1, b2;
-  load_k(a, kvh, lane, t_lo, pid_of(0), b0);
-  load_v(a, kvh, lane, t_lo, pid_of(0), b1);
-  pid_next = pid_of(1);
-  // The prologue's loads land before the loop: the compiler's wait analysis then
-  // sees nothing outstanding at the loop head, so no wait inside the body covers
-  // a load issued for a later chunk.
-  wait_vmem_all();
-  for (int c = 0; c < n; c += 3) {
-    step(c, b0, b1, b2);
-    if (c + 1 >= n) break;
-    step(c + 1, b2, b0, b1);
-    if (c + 2 >= n) break;
-    step(c + 2, b1, b2, b0);
-  }
-  write_partial(a, st, prow, lane);
-}
-
-// LDS of a work-group of WPB waves: the codebook tables (a replicated 4-bit pair table
-// at a 64 KB slot, so that its address registers need no base add), then one p tile
-// per wave.
-template <int BWK, int BWV, int NG, int WPB>
-struct RowsLds {
-  // A 4-bit table takes a 64 KB slot of its own: its address registers carry the slot.
-  // Beside a pair-coded table (2, 3, 5, 6 bits) it takes slot 1 and the pair table
-  // offset 0, where its entry offsets (below 64 KB) need no base added: the read's
-  // 16-bit offset field cannot hold a base of 64 KB, which would cost an add per lookup.
-  static constexpr bool k4 = BWK == 4, v4 = BWV == 4;
-  static constexpr int k_off = k4 ? (pair_coded<BWV>() ? kPairTableBytes : 0)
-                                  : (v4 && !pair_coded<BWK>() ? kPairTableBytes : 0);
-  static constexpr int v_off = v4 ? (k4 || pair_coded<BWK>() ? kPairTableBytes : 0)
-                                  : (k4 ? (pair_coded<BWV>() ? 0 : kPairTableBytes) : table_bytes<BWK>());
-  static constexpr int k_slot = k_off >> 16, v_slot = v_off >> 16;
-  static constexpr int tiles = k_off + table_bytes<BWK>() > v_off + table_bytes<BWV>() ? k_off + table_bytes<BWK>()
-                                                                                       : v_off + table_bytes<BWV>();
-  static constexpr int tile_bytes = NG * 16 * kPStride * 4;
-  static constexpr int total = tiles + WPB * tile_bytes;
-  static_assert(total <= 160 * 1024, "LDS of a work-group exceeds 160 KB");
-};
 
 template <int BW>
 __device__ __forceinline__ Tab<BW> make_tab(const char* lds, int off, int lane) {
@@ -775,40 +367,10 @@ struct RangeWalk {
   }
 };
 
-template <class Scan>
-__device__ __forceinline__ void for_each_range(const DecodeArgs& a, int64_t w, int lane, Scan&& scan) {
-  RangeWalk rw;
-  if (rw.init(a, w, lane)) rw.run(a, w, lane, scan);
-}
-
-// Work-group of WPB independent waves sharing the codebook tables; wave w =
-// blockIdx.x * WPB + wave-in-group walks the work list of for_each_range.
-template <int BWK, int BWV, int NG, int WPB>
-__global__ __launch_bounds__(64 * WPB) void decode_rows_kernel(DecodeArgs a) {
-  using Lay = RowsLds<BWK, BWV, NG, WPB>;
-  __shared__ __align__(16) char lds[Lay::total];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wig = __builtin_amdgcn_readfirstlane(tid >> 6);
-  stage_table<BWK, 64 * WPB>(a.cb_k, lds + Lay::k_off, tid);
-  stage_table<BWV, 64 * WPB>(a.cb_v, lds + Lay::v_off, tid);
-  __syncthreads();  // the only block-wide barrier: waves run independently from here
-  // Work-groups are dealt to the eight XCDs round robin (group p on XCD p % 8); the
-  // logical group index gives each XCD a contiguous stretch of the flattened work,
-  // so the kv heads of a sequence run on one XCD and share the 128-byte lines that
-  // hold their norms in its L2.
-  const int64_t w = int64_t(xcd_major(blockIdx.x, gridDim.x)) * WPB + wig;
-  float* ptile = reinterpret_cast<float*>(lds + Lay::tiles + wig * Lay::tile_bytes);
-  Tab<BWK> cbk = make_tab<BWK>(lds, Lay::k_off, lane);
-  Tab<BWV> cbv = make_tab<BWV>(lds, Lay::v_off, lane);
-  for_each_range(a, w, lane, [&](int b, int kvh, int t_lo, int t_hi, int64_t prow, uint32_t) {
-    scan_range<BWK, BWV, NG>(a, b, kvh, t_lo, t_hi, prow, lane, cbk, cbv, ptile);
-  });
-}
-
 // ------------------------------------------------------------------ 16-bit matrix-core scan
 //
-// The page scan on v_mfma_f32_16x16x32_f16 (16 times the MAC rate of the fp32 4x4x1
-// MFMA on gfx950), for 2, 3, 4, 5 and 6-bit codes, 8-bit ones, and 4 with 8. Every fp32 factor x is carried as
+// The page scan on v_mfma_f32_16x16x32_f16 (16 times the MAC rate of the fp32 4x4x1 MFMA
+// on gfx950), for 2, 3, 4, 5, 6 and 8-bit codes and the pairs 4/6, 6/4 and 4/8. Every fp32 factor x is carried as
 // an fp16 pair x = H + L (H = fp16(x), L = fp16(x - H)) after an exact power-of-two
 // scaling that takes the largest of a factor's values to the top of fp16's range: values
 // above 2^-3 keep 22 bits, smaller ones an error of 2^-25, 2^-32 or less of the largest.
@@ -836,11 +398,10 @@ __global__ __launch_bounds__(64 * WPB) void decode_rows_kernel(DecodeArgs a) {
 //            8..15 are zero. 8 K-steps x 4 tiles = 32 MFMAs per chunk. Output lane
 //            16g+c register i holds token 16r + 4i + g of column c.
 //   softmax  the two column halves are added (row rotate by NH), the scores pass
-//            through a per-wave LDS tile to lane = token, and the online softmax runs as
-//            in the fp32 scan. p n_V 2^-gs goes back to the same tile as H | L << 16
-//            words.
+//            through a per-wave LDS tile to lane = token, and p n_V 2^-gs goes back to the
+//            same tile as H | L << 16 words.
 //   values   M-tile mt: row c of lane 16g+c is dim 8c + mt, so a lane needs codes
-//            8c..8c+7 of each token: the V loads of the fp32 scan, unchanged. K-step ks:
+//            8c..8c+7 of each token (load_v). K-step ks:
 //            k-slots of group g are tokens 16ks + 4j + g, j = 0..3; the codes of dim
 //            8c + mt of tokens (j = 0, 1) and (2, 3) are merged into pair indices (4-bit:
 //            a bit-field insert per four dims), whose entries form the A operand. B =
@@ -1066,11 +627,6 @@ __device__ __forceinline__ void merge_value_pairs(RowBuf<BWK, BWV>& V, int lane)
     }
   }
 }
-
-// The 16-bit scan keeps its rows in RowBuf words too. As a K buffer: for each tile
-// t, the 4 BWK bytes of quarter g of token 16t + 4(c%4) + c/4 (words [t*BWK, t*BWK +
-// BWK)), then the fp16 K and V norms of token c0 + lane (words KW, KW+1). As a V
-// buffer: the layout of the fp32 scan.
 
 // Token (within its 16-token tile) whose scores row c of a score MFMA holds.
 __device__ __forceinline__ int tile_token(int c) { return 4 * (c & 3) + (c >> 2); }
@@ -1811,9 +1367,13 @@ __device__ __forceinline__ void scan_range16(const DecodeArgs& a, int b, int kvh
 }
 
 // LDS of a work-group: the tables (4 and 8-bit ones in 64 KB slots of their own, slot 1
-// beside a pair-coded table, as in RowsLds), then one tile per wave.
+// beside a pair-coded table: its entry offsets, below 64 KB, then need no base added, which
+// the read's 16-bit offset field could not hold), then one tile per wave.
 template <int BW>
-constexpr int table16_bytes() { return BW == 8 ? 256 * 64 * 4 : table_bytes<BW>(); }
+constexpr int table16_bytes() {
+  if constexpr (BW == 8) return 256 * 64 * 4;
+  else return table_bytes<BW>();
+}
 template <int BWK, int BWV, int NG, int WPB>
 struct Rows16Lds {
   static constexpr bool ks = BWK == 4 || BWK == 8, vs = BWV == 4 || BWV == 8;
@@ -1888,44 +1448,6 @@ __global__ __launch_bounds__(64 * WPB) void decode_rows_tf_kernel(DecodeArgs a) 
   pace.publish(0);
 }
 
-// Waves per work-group: three per SIMD where the scan fits in 168 VGPRs, else two.
-template <int BWK, int BWV, int NG>
-constexpr int rows_wpb() { return NG == 1 && BWK <= 4 && BWV <= 4 ? 12 : 8; }
-
-template <int BWK, int BWV, int NG>
-SplitKernel rows_kernel() {
-  constexpr int wpb = rows_wpb<BWK, BWV, NG>();
-  SplitKernel k;
-  k.fn = decode_rows_kernel<BWK, BWV, NG, wpb>;
-  k.block = 64 * wpb;
-  k.wpb = wpb;
-  k.nrep = 4 * NG;
-  k.log2_units = true;
-  k.rows = true;
-  return k;
-}
-
-template <int NG>
-SplitKernel rows_for(int bw_k, int bw_v) {
-  if (bw_k == bw_v) {
-    switch (bw_k) {
-      case 2: return rows_kernel<2, 2, NG>();
-      case 3: return rows_kernel<3, 3, NG>();
-      case 4: return rows_kernel<4, 4, NG>();
-      case 5: return rows_kernel<5, 5, NG>();
-      case 6: return rows_kernel<6, 6, NG>();
-      case 8: return rows_kernel<8, 8, NG>();
-    }
-  } else if (bw_k == 4 && bw_v == 6) {
-    return rows_kernel<4, 6, NG>();
-  } else if (bw_k == 6 && bw_v == 4) {
-    return rows_kernel<6, 4, NG>();
-  } else if (bw_k == 4 && bw_v == 8) {
-    return rows_kernel<4, 8, NG>();
-  }
-  return SplitKernel{};
-}
-
 template <int BWK, int BWV, int NG, bool PAIR>
 SplitKernel rows16_kernel() {
   constexpr int wpb = 8;  // two waves per SIMD: the 16-bit scan needs up to 256 VGPRs
@@ -1990,38 +1512,23 @@ SplitKernel rows_tf_for(int bw_k, int bw_v) {
   return SplitKernel{};
 }
 
-// WN_DECODE_SCAN=rows32 keeps the fp32-product row scan for every width (the two
-// compute the same result to fp32 rounding; the knob exists to compare them on one
-// machine). Read once.
-bool rows16_allowed() {
-  static const bool allowed = [] {
-    const char* e = getenv("WN_DECODE_SCAN");
-    return !(e && !strcmp(e, "rows32"));
-  }();
-  return allowed;
-}
-
 }  // namespace
 
 SplitKernel pick_split_rows_tf(int bw_k, int bw_v, int n_rep) {
   const int ng = n_rep >= 1 && n_rep <= 4 ? 1 : n_rep >= 5 && n_rep <= 8 ? 2 : 0;
-  if (ng == 0 || !rows16_allowed()) return SplitKernel{};
+  if (ng == 0) return SplitKernel{};
   return ng == 1 ? rows_tf_for<1>(bw_k, bw_v) : rows_tf_for<2>(bw_k, bw_v);
 }
 
 SplitKernel pick_split_pair(int bw_k, int bw_v, int n_rep) {
-  if (n_rep < 1 || n_rep > 4 || !rows16_allowed()) return SplitKernel{};
+  if (n_rep < 1 || n_rep > 4) return SplitKernel{};
   return rows16_for<2, true>(bw_k, bw_v);
 }
 
 SplitKernel pick_split_rows(int bw_k, int bw_v, int n_rep) {
   const int ng = n_rep <= 4 ? 1 : n_rep <= 8 ? 2 : 0;
   if (ng == 0) return SplitKernel{};
-  if (rows16_allowed()) {
-    const SplitKernel k = ng == 1 ? rows16_for<1>(bw_k, bw_v) : rows16_for<2>(bw_k, bw_v);
-    if (k.fn) return k;
-  }
-  return ng == 1 ? rows_for<1>(bw_k, bw_v) : rows_for<2>(bw_k, bw_v);
+  return ng == 1 ? rows16_for<1>(bw_k, bw_v) : rows16_for<2>(bw_k, bw_v);
 }
 
 }  // namespace wn
