@@ -972,21 +972,17 @@ struct PfRotArgs {
   int vec;  // rows of q are aligned to four elements
 };
 
-// Waves that share a row tile, row tiles a work-group of four waves takes at a time.
-template <int D>
-struct RotShape {
-  static constexpr int CW = D / 32, TW = 4 / CW, S = D / 16;
-};
+constexpr int kRotD = 128, kRotSteps = kRotD / 16;  // head_dim, K-steps of sixteen columns
 
 // acc[rt][t] += M x^T: columns 16t + 4g + i of row c of half rt of the tile.
-template <int S>
-__device__ __forceinline__ void rot_product(const f32x4 (&m)[2][S], const f32x4 (&x)[2][S], f32x4 (&acc)[2][2]) {
+__device__ __forceinline__ void rot_product(const f32x4 (&m)[2][kRotSteps], const f32x4 (&x)[2][kRotSteps],
+                                            f32x4 (&acc)[2][2]) {
 #pragma unroll
   for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
     for (int t = 0; t < 2; ++t) acc[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int s = 0; s < S; ++s)
+  for (int s = 0; s < kRotSteps; ++s)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -1032,32 +1028,31 @@ __device__ __forceinline__ void store4(void* out, int64_t i, int dtype, bool vec
 }
 
 // q_rot = scale * q Pi_K^T, zero for rows past n_rep Q of a (sequence, kv head).
-template <int D>
 __global__ __launch_bounds__(256) void pf_rotate_kernel(PfRotArgs a) {
-  using Sh = RotShape<D>;
+  constexpr int D = kRotD;
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15, w = threadIdx.x >> 6;
-  const int j0 = 32 * (w % Sh::CW);
-  f32x4 m[2][Sh::S];  // rows j of Pi_K
+  const int j0 = 32 * w;
+  f32x4 m[2][kRotSteps];  // rows j of Pi_K
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int s = 0; s < Sh::S; ++s) m[t][s] = *reinterpret_cast<const f32x4*>(a.pi + (j0 + 16 * t + c) * D + 16 * s + 4 * g);
+    for (int s = 0; s < kRotSteps; ++s) m[t][s] = *reinterpret_cast<const f32x4*>(a.pi + (j0 + 16 * t + c) * D + 16 * s + 4 * g);
   const int rows = a.n_rep * a.Q;
-  for (int64_t tile = int64_t(blockIdx.x) * Sh::TW + w / Sh::CW; tile < a.tiles; tile += int64_t(gridDim.x) * Sh::TW) {
+  for (int64_t tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
     const int64_t row0 = tile * kRotRows;
     const uint32_t unit = uint32_t(row0) / uint32_t(a.nrp);  // kRotRows divides nrp
     const int r0 = int(uint32_t(row0) % uint32_t(a.nrp)), kvh = int(unit % uint32_t(a.Hkv));
     const int64_t b = unit / uint32_t(a.Hkv);
-    f32x4 x[2][Sh::S], acc[2][2];
+    f32x4 x[2][kRotSteps], acc[2][2];
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) {
       const int r = r0 + 16 * rt + c;
       const int qi = r / a.n_rep, h = kvh * a.n_rep + r % a.n_rep;
       const int64_t o = b * a.qsb + h * a.qsh + qi * a.qsq + 4 * g;
 #pragma unroll
-      for (int s = 0; s < Sh::S; ++s) x[rt][s] = r < rows ? load_q4(a, o + 16 * s) : f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < kRotSteps; ++s) x[rt][s] = r < rows ? load_q4(a, o + 16 * s) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    rot_product<Sh::S>(m, x, acc);
+    rot_product(m, x, acc);
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
@@ -1081,54 +1076,50 @@ struct PfMergeArgs {
 // threads merge a row tile into LDS, then its waves multiply. The splits' maxima are
 // read in one pass and their weighted rows in a second, so neither pass chains a load
 // behind another.
-template <int D>
 __global__ __launch_bounds__(256) void pf_merge_kernel(PfMergeArgs a) {
-  using Sh = RotShape<D>;
-  constexpr int NR = kRotRows * Sh::TW, STRIDE = D + 4;  // rows at a time; floats per LDS row (bank-skewed)
+  constexpr int D = kRotD, NR = kRotRows, STRIDE = D + 4;  // floats per LDS row (bank-skewed)
   __shared__ __align__(16) float xt[NR * STRIDE];
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, c = lane & 15, w = tid >> 6;
-  const int j0 = 32 * (w % Sh::CW);
-  f32x4 m[2][Sh::S];  // columns j of Pi_V ([k][j])
+  const int j0 = 32 * w;
+  f32x4 m[2][kRotSteps];  // columns j of Pi_V ([k][j])
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int s = 0; s < Sh::S; ++s)
+    for (int s = 0; s < kRotSteps; ++s)
 #pragma unroll
       for (int e = 0; e < 4; ++e) m[t][s][e] = a.pi_v[(16 * s + 4 * g + e) * D + j0 + 16 * t + c];
   const int rows = a.n_rep * a.Q, Hq = a.Hkv * a.n_rep;
-  for (int64_t tile0 = int64_t(blockIdx.x) * Sh::TW; tile0 < a.tiles; tile0 += int64_t(gridDim.x) * Sh::TW) {
+  for (int64_t tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
     {
       // thread: row rr, dims DPT (tid % TPR) .. (TPR threads per row)
       constexpr int TPR = 256 / NR, DPT = D / TPR;
       const int rr = tid / TPR, d0 = DPT * (tid % TPR);
-      const int64_t row = tile0 * kRotRows + rr;
+      const int64_t row = tile * kRotRows + rr;
       float den = 0.f, num[DPT];
 #pragma unroll
       for (int k = 0; k < DPT; ++k) num[k] = 0.f;
-      if (row < a.tiles * kRotRows) {
-        const uint32_t unit = uint32_t(row) / uint32_t(a.nrp);
-        const int r = int(uint32_t(row) % uint32_t(a.nrp));
-        const int64_t part = (int64_t(unit) * a.nsplit * a.ncb + r / a.nr) * a.nr + r % a.nr;
-        const int64_t step = int64_t(a.ncb) * a.nr;  // rows between a row's consecutive splits
-        float M = -INFINITY;
+      const uint32_t unit = uint32_t(row) / uint32_t(a.nrp);
+      const int r = int(uint32_t(row) % uint32_t(a.nrp));
+      const int64_t part = (int64_t(unit) * a.nsplit * a.ncb + r / a.nr) * a.nr + r % a.nr;
+      const int64_t step = int64_t(a.ncb) * a.nr;  // rows between a row's consecutive splits
+      float M = -INFINITY;
 #pragma unroll 8
-        for (int s = 0; s < a.nsplit; ++s) M = fmaxf(M, a.part_ml[2 * (part + s * step)]);
-        if (M != -INFINITY) {
+      for (int s = 0; s < a.nsplit; ++s) M = fmaxf(M, a.part_ml[2 * (part + s * step)]);
+      if (M != -INFINITY) {
 #pragma unroll 4
-          for (int s = 0; s < a.nsplit; ++s) {
-            const int64_t pr = part + s * step;
-            const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * pr);
-            const float wt = __builtin_amdgcn_exp2f(ml.x - M);  // 0 for a split without keys (m = -inf)
-            den = fmaf(wt, ml.y, den);
-            const float4* src = reinterpret_cast<const float4*>(a.part_acc + pr * D + d0);
+        for (int s = 0; s < a.nsplit; ++s) {
+          const int64_t pr = part + s * step;
+          const float2 ml = *reinterpret_cast<const float2*>(a.part_ml + 2 * pr);
+          const float wt = __builtin_amdgcn_exp2f(ml.x - M);  // 0 for a split without keys (m = -inf)
+          den = fmaf(wt, ml.y, den);
+          const float4* src = reinterpret_cast<const float4*>(a.part_acc + pr * D + d0);
 #pragma unroll
-            for (int k = 0; k < DPT / 4; ++k) {
-              const float4 v = src[k];
-              num[4 * k] = fmaf(wt, v.x, num[4 * k]);
-              num[4 * k + 1] = fmaf(wt, v.y, num[4 * k + 1]);
-              num[4 * k + 2] = fmaf(wt, v.z, num[4 * k + 2]);
-              num[4 * k + 3] = fmaf(wt, v.w, num[4 * k + 3]);
-            }
+          for (int k = 0; k < DPT / 4; ++k) {
+            const float4 v = src[k];
+            num[4 * k] = fmaf(wt, v.x, num[4 * k]);
+            num[4 * k + 1] = fmaf(wt, v.y, num[4 * k + 1]);
+            num[4 * k + 2] = fmaf(wt, v.z, num[4 * k + 2]);
+            num[4 * k + 3] = fmaf(wt, v.w, num[4 * k + 3]);
           }
         }
       }
@@ -1138,26 +1129,23 @@ __global__ __launch_bounds__(256) void pf_merge_kernel(PfMergeArgs a) {
         *reinterpret_cast<f32x4*>(xt + rr * STRIDE + d0 + k) = f32x4{num[k], num[k + 1], num[k + 2], num[k + 3]} * inv;
     }
     __syncthreads();
-    const int64_t tile = tile0 + w / Sh::CW;
-    if (tile < a.tiles) {
-      f32x4 x[2][Sh::S], acc[2][2];
+    f32x4 x[2][kRotSteps], acc[2][2];
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt)
+    for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
-        for (int s = 0; s < Sh::S; ++s)
-          x[rt][s] = *reinterpret_cast<const f32x4*>(xt + ((w / Sh::CW) * kRotRows + 16 * rt + c) * STRIDE + 16 * s + 4 * g);
-      rot_product<Sh::S>(m, x, acc);
-      const uint32_t row0 = uint32_t(tile * kRotRows), unit = row0 / uint32_t(a.nrp);
-      const int kvh = int(unit % uint32_t(a.Hkv));
-      const int64_t b = unit / uint32_t(a.Hkv);
+      for (int s = 0; s < kRotSteps; ++s)
+        x[rt][s] = *reinterpret_cast<const f32x4*>(xt + (16 * rt + c) * STRIDE + 16 * s + 4 * g);
+    rot_product(m, x, acc);
+    const uint32_t row0 = uint32_t(tile * kRotRows), unit = row0 / uint32_t(a.nrp);
+    const int kvh = int(unit % uint32_t(a.Hkv));
+    const int64_t b = unit / uint32_t(a.Hkv);
 #pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
-        const int r = int(row0 % uint32_t(a.nrp)) + 16 * rt + c;
-        if (r >= rows) continue;
-        const int qi = r / a.n_rep, h = kvh * a.n_rep + r % a.n_rep;
+    for (int rt = 0; rt < 2; ++rt) {
+      const int r = int(row0 % uint32_t(a.nrp)) + 16 * rt + c;
+      if (r >= rows) continue;
+      const int qi = r / a.n_rep, h = kvh * a.n_rep + r % a.n_rep;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) store4(a.out, ((b * Hq + h) * a.Q + qi) * D + j0 + 16 * t + 4 * g, a.out_dtype, a.vec, acc[rt][t]);
-      }
+      for (int t = 0; t < 2; ++t) store4(a.out, ((b * Hq + h) * a.Q + qi) * D + j0 + 16 * t + 4 * g, a.out_dtype, a.vec, acc[rt][t]);
     }
     __syncthreads();  // the tile is read; the next one may overwrite it
   }
@@ -1343,7 +1331,7 @@ extern "C" int wn_prefill_attention(
                float(double(scale) * 1.4426950408889634), tiles, Hkv, n_rep, Q, nrp, q_dtype, qvec};
   // work-groups that take a few row tiles each: Pi is read once per work-group
   const unsigned rot_groups = unsigned(std::min<int64_t>(tiles, kRotGroups));
-  hipLaunchKernelGGL(pf_rotate_kernel<128>, dim3(rot_groups), dim3(256), 0, st, ra);
+  hipLaunchKernelGGL(pf_rotate_kernel, dim3(rot_groups), dim3(256), 0, st, ra);
 
   PrefillArgs pa;
   pa.q_rot = ra.q_rot;
@@ -1385,6 +1373,6 @@ extern "C" int wn_prefill_attention(
 
   PfMergeArgs ma{pa.part_acc, pa.part_ml, pi_v, out, tiles, out_dtype, Hkv, n_rep, Q, nrp, ncb, num_splits, nr,
                  aligned(out, o4)};
-  hipLaunchKernelGGL(pf_merge_kernel<128>, dim3(rot_groups), dim3(256), 0, st, ma);
+  hipLaunchKernelGGL(pf_merge_kernel, dim3(rot_groups), dim3(256), 0, st, ma);
   return check_launch("wn_prefill_attention");
 }
