@@ -194,3 +194,48 @@ def test_histories_past_the_row_limit_go_group_by_group(monkeypatch):
     monkeypatch.setattr(wc, "_ROWS_LIMIT", 2 * 3 * n)
     for a, b in zip(_layer(D, 4, 8, 8, n, chunk=16).update(k, v), whole):
         assert torch.allclose(a, b, rtol=0, atol=2e-6 * b.abs().max().item())
+
+
+def test_split_append_of_mixed_dtypes():
+    """K and V of different types, and rows that 16-byte loads cannot read, take the
+    per-group kernels: the same codes as the values alike."""
+    D, n = 128, 21
+    loud = torch.arange(0, D, 16, device=DEV)
+    k, v = _kv(2, 3, n, D, loud, torch.bfloat16, 4)
+    shifted = torch.empty(k.numel() + 1, dtype=k.dtype, device=DEV)[1:].view(k.shape)
+    shifted.copy_(k)
+    layers = []
+    for kk, vv in ((k, v), (k, v.float()), (shifted, v)):
+        layers.append(_layer(D, 4, 8, 8, n))
+        layers[-1].update(kk, vv)
+    for other in layers[1:]:
+        assert not other._split_append_ok(k, v.float()) and not other._split_append_ok(shifted, v)
+        for a, b in zip(layers[0]._k_groups + layers[0]._v_groups, other._k_groups + other._v_groups):
+            assert torch.equal(a.codes, b.codes) and torch.equal(a.norms, b.norms)
+
+
+@pytest.mark.parametrize("bw,off", [(4, 2), (8, 4), (4, 1), (6, 3)])
+def test_sides_at_different_alignments(bw, off):
+    """One side's codes a few bytes off the width that whole eights are read by: both sides
+    byte by byte, the same values."""
+    from winnow_amd import _lib
+    from winnow_amd.quantizer import TurboQuantMSE
+    D, rows = 64, 70
+    tq = TurboQuantMSE(bw, D, DEV)
+    nb = D * bw // 8
+    g = torch.Generator(device=DEV).manual_seed(bw)
+    sides = torch.randint(0, 256, (2, rows, nb), generator=g, device=DEV, dtype=torch.uint8)
+    norms = torch.rand(2, rows, generator=g, device=DEV).half()
+    room = torch.empty(rows * nb + off, dtype=torch.uint8, device=DEV)[off:].view(rows, nb)
+    room.copy_(sides[1])
+
+    def run(k, v):
+        out = torch.empty(2, rows, D, device=DEV)
+        _lib.call("wn_dequantize_rows", _lib.ptr(k), _lib.ptr(v), _lib.ptr(norms[0]), _lib.ptr(norms[1]), bw, _lib.ptr(tq.centroids),
+                  None, None, None, None, 0, None, 0, _lib.ptr(tq.Pi), None, 1, rows, rows, D, _lib.ptr(out[0]), _lib.ptr(out[1]),
+                  _lib.WN_F32, _lib.stream_of(out.device))
+        return out
+    want = run(sides[0], sides[1])
+    assert torch.equal(run(sides[0], room), want)
+    norms = norms.flip(0).contiguous()
+    assert torch.equal(run(room, sides[0]), want.flip(0))
