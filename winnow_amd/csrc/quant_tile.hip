@@ -12,8 +12,9 @@
 //
 //   operands  Pi 2^8 = H + L, an fp16 pair per entry (22 bits), in LDS in the order the
 //             MFMAs read it, staged once by a persistent work-group of sixteen waves; x
-//             2^(8-e), e the exponent of the norm: exact in fp16 for bf16 and fp16
-//             inputs, an fp16 pair for fp32 inputs.
+//             2^(8-e), e the exponent of the norm: one fp16 for bf16 and fp16 inputs
+//             (exact but for elements below 2^-22 of the norm, which end as fp16 subnormals,
+//             2^-33 of it off at most), an fp16 pair for fp32 inputs.
 //   product   y^T = Pi x^T on v_mfma_f32_16x16x32_f16, A = rows of Pi, B = sixteen
 //             vectors; a wave takes one such tile of vectors at a time (with two, half
 //             the LDS reads, the kernel spilled and ran slower: 34 us against 30).
@@ -21,7 +22,8 @@
 //             products of fp16 values are exact, each of a sum's D additions errs by at
 //             most one ulp (2^-23, truncation allowed) of a partial sum, all of which
 //             are below |x / n| R <= R (Cauchy-Schwarz); 2^-20 covers the two splits
-//             (2^-22 each), the product with 1 / n and the last rounding.
+//             (2^-22 each), the subnormal elements (sqrt(D) 2^-33), the product with 1 / n
+//             and the last rounding.
 //   buckets   y's cell of a 512-cell grid over the boundaries gives the number of
 //             boundaries below the cell and the one boundary in reach of it: one 8-byte
 //             LDS read, against a search of bw reads. A cell with two or more in reach

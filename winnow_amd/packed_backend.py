@@ -16,10 +16,12 @@ Names, arguments and errors are those of ``turboquant_kv/packed_backend.py``
   and every page it names inside the pool, on host copies of the metadata before
   the launch, raising ``UnsupportedLayout`` as the reference raises in its gather.
 * Decode (one query token) runs the HIP compressed-domain operator on packed pages,
-  the HIP dense operator on unquantized pages. A prefill chunk dequantizes the
-  batch's histories on the GPU (``wn_dequantize_history``) into one padded tensor
-  and runs ONE SDPA call with a per-sequence offset-causal mask (the reference loops
-  over sequences, packed_backend.py:210-246).
+  the HIP dense operator on unquantized pages. A prefill chunk runs the fused prefill
+  over the packed pages where it is compiled (``prefill_fused``); other packed shapes
+  dequantize the batch's histories on the GPU into one padded tensor and attend to it
+  under a per-sequence offset-causal mask in one HIP operator (``wn_history_attention``:
+  16-bit queries at head_dim 64 and 128 of which only the values are wanted) or one SDPA
+  call (the reference loops over sequences, packed_backend.py:210-246).
 * There is no host fallback: a decode on a non-HIP tensor raises.
 """
 from __future__ import annotations
@@ -498,18 +500,18 @@ def _plain(t: torch.Tensor) -> bool:
 def _observed() -> bool:
     """Whether something records or rewrites the torch operators called here: a compiler, a
     trace (``torch.jit.trace``, ``make_fx``, export), a dispatch mode, or a function mode
-    other than a default device's."""
-    return (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
-            or torch._ops._len_torch_dispatch_stack_pre_dispatch() > 0
+    other than a default device's (tracing before dispatch runs under one too)."""
+    return (torch._C._len_torch_dispatch_stack() > 0 or torch._C._get_tracing_state() is not None
             or (torch._C._len_torch_function_stack() > 0
-                and not all(isinstance(m, DeviceContext) for m in _get_current_function_mode_stack())))
+                and not all(isinstance(m, DeviceContext) for m in _get_current_function_mode_stack()))
+            or torch.compiler.is_compiling())
 
 
 def _history_kernel(query, kv: pa.PackedKV, Lmax: int) -> bool:
-    """Whether ``wn_history_attention`` serves the SDPA of a reconstruct step: a 16-bit
-    query at head_dim 64 or 128 on the handle's device, only its values wanted (the
-    library's operator serves gradients, tangents and traces), sizes within its limits."""
-    if query.dtype not in (torch.bfloat16, torch.float16) or query.dim() != 4 or not _plain(query):
+    """Whether ``wn_history_attention`` serves the SDPA of a reconstruct step whose query is
+    wanted for its values alone (``_plain``): a 16-bit query at head_dim 64 or 128 on the
+    handle's device, sizes within the operator's limits."""
+    if query.dtype not in (torch.bfloat16, torch.float16) or query.dim() != 4:
         return False
     B, Hq, Q, D = query.shape
     Hkv, lens = kv.num_kv_heads, kv.seq_lens
@@ -522,19 +524,17 @@ def _history_kernel(query, kv: pa.PackedKV, Lmax: int) -> bool:
 
 def _histories(kv: pa.PackedKV, pages, norms, quant, lens, Lmax: int, dtype) -> torch.Tensor:
     """(B, Hkv, Lmax, D) histories of the batch; what lies past a length is not meant to be
-    read. Contiguous page rows: one launch; else sequence by sequence."""
+    read. Contiguous page rows: one launch, on the current device; else sequence by sequence."""
     B, S, D, Hkv = lens.shape[0], kv.page_size, kv.head_dim, kv.num_kv_heads
     buf = torch.empty(B, Hkv, Lmax, D, dtype=dtype, device=pages.device)
     if D == 128 and pages.stride(-1) == 1 and pages.stride(-2) == pages.shape[-1] and norms.stride(-1) == 1:
-        with torch.cuda.device(pages.device):
-            _lib.call("wn_dequantize_histories", _lib.ptr(pages), pages.stride(0), pages.stride(1), _lib.ptr(norms),
-                      norms.stride(0), norms.stride(1), _lib.ptr(kv.page_table), kv.page_table.stride(0),
-                      _lib.ptr(kv.seq_lens), B, Lmax, Hkv, S, _lib.ptr(quant.centroids), _lib.ptr(quant.Pi),
-                      quant.bit_width, D, _lib.ptr(buf), _lib.DTYPE_CODE[dtype], 0, _lib.stream_of(pages.device))
+        _lib.call("wn_dequantize_histories", _lib.ptr(pages), pages.stride(0), pages.stride(1), _lib.ptr(norms),
+                  norms.stride(0), norms.stride(1), _lib.ptr(kv.page_table), kv.page_table.stride(0),
+                  _lib.ptr(kv.seq_lens), B, Lmax, Hkv, S, _lib.ptr(quant.centroids), _lib.ptr(quant.Pi),
+                  quant.bit_width, D, _lib.ptr(buf), _lib.DTYPE_CODE[dtype], 0, _lib.stream_of(pages.device))
         return buf
     if D != 128 and _paged_rows(kv, pages, norms):
-        with torch.cuda.device(pages.device):
-            _dequantize_pages(kv, pages, norms, quant, kv.page_table, kv.seq_lens, Lmax, buf)
+        _dequantize_pages(kv, pages, norms, quant, kv.page_table, kv.seq_lens, Lmax, buf)
         return buf
     for b in range(B):
         if lens[b]:
@@ -543,22 +543,42 @@ def _histories(kv: pa.PackedKV, pages, norms, quant, lens, Lmax: int, dtype) -> 
 
 
 def _history_attention(query, kv: pa.PackedKV, k, v, Lmax: int, scaling):
-    """The offset-causal SDPA of ``_padded_sdpa`` in one HIP operator, as a (B, Hq, Q, D)
-    view of (B, Q, Hq, D) memory, the order in which the model's attention returns it."""
+    """The offset-causal SDPA of ``_padded_sdpa`` in one HIP operator on the current device, as
+    a (B, Hq, Q, D) view of (B, Q, Hq, D) memory, the order in which the model's attention
+    returns it."""
     B, Hq, Q, D = query.shape
     Hkv, code = kv.num_kv_heads, _lib.DTYPE_CODE[query.dtype]
     if query.stride(-1) != 1 or query.data_ptr() % 16 or any(s % 8 for s in query.stride()[:3]):
         query = query.clone(memory_format=torch.contiguous_format)
     out = torch.empty(B, Q, Hq, D, dtype=query.dtype, device=query.device)
     ns = ctypes.c_int(0)
-    with torch.cuda.device(query.device):
-        _lib.call("wn_history_plan", B, Hq, Hkv, Q, D, code, Lmax, ctypes.byref(ns))
-        ws = torch.empty(int(_lib.lib().wn_history_workspace_bytes(B, Hq, Hkv, Q, D, ns.value)), dtype=torch.uint8,
-                         device=query.device)
-        _lib.call("wn_history_attention", _lib.ptr(query), code, query.stride(0), query.stride(1), query.stride(2),
-                  _lib.ptr(k), _lib.ptr(v), _lib.ptr(kv.seq_lens), _lib.ptr(out), _lib.ptr(ws), ws.numel(),
-                  B, Hq, Hkv, Q, D, Lmax, float(scaling), ns.value, _lib.stream_of(query.device))
+    _lib.call("wn_history_plan", B, Hq, Hkv, Q, D, code, Lmax, ctypes.byref(ns))
+    ws = torch.empty(int(_lib.lib().wn_history_workspace_bytes(B, Hq, Hkv, Q, D, ns.value)), dtype=torch.uint8,
+                     device=query.device)
+    _lib.call("wn_history_attention", _lib.ptr(query), code, query.stride(0), query.stride(1), query.stride(2),
+              _lib.ptr(k), _lib.ptr(v), _lib.ptr(kv.seq_lens), _lib.ptr(out), _lib.ptr(ws), ws.numel(),
+              B, Hq, Hkv, Q, D, Lmax, float(scaling), ns.value, _lib.stream_of(query.device))
     return out.transpose(1, 2)
+
+
+def _check_histories(lens: torch.Tensor, table: torch.Tensor, num_pages: int, page_size: int) -> None:
+    """``check_page_ranges`` of the histories about to be read: the kernels read pages by the
+    table's ids, unchecked. Looked over in few steps first (four sequences of one page 3 us
+    against 17, eight of 94 pages 8 against 18); whatever is odd goes the long way and raises."""
+    if table.dtype == torch.int32 and table.dim() == 2 and table.shape[0] == lens.numel() > 0:
+        lengths = lens.tolist()
+        used = [-(-L // page_size) for L in lengths]
+        if min(lengths) >= 0 and max(used) <= table.shape[1]:
+            if table.numel() <= 128:
+                rows = [row[:n] for row, n in zip(table.tolist(), used) if n]
+                if all(min(row) >= 0 and max(row) < num_pages for row in rows):
+                    return
+            else:
+                bad = table.numpy().view(np.uint32) >= num_pages   # a negative id is a large one
+                first = bad.argmax(1).tolist()                     # 0 where none is bad
+                if all(f >= n or not (f or b) for f, b, n in zip(first, bad[:, 0].tolist(), used)):
+                    return
+    pa.check_page_ranges(lens, table, num_pages, page_size)
 
 
 def _reconstruct_sdpa(query, kv: pa.PackedKV, scaling):
@@ -566,16 +586,19 @@ def _reconstruct_sdpa(query, kv: pa.PackedKV, scaling):
     pair, then one offset-causal SDPA over the batch (packed_backend.py:211-226): the HIP
     operator for 16-bit queries (``_history_kernel``), else the library's."""
     B, Hq, Q, D = query.shape
-    lens = _host_lens(kv).to(torch.int64)
-    Lmax = int(lens.max()) if B else 0
+    host = _host_lens(kv)
+    plain = _plain(query)
+    # under a trace the read of the longest length is what refuses it
+    Lmax = 0 if not B else max(host.tolist(), default=0) if plain else int(host.to(torch.int64).max())
     if Lmax == 0:
         return torch.zeros(B, Hq, Q, D, dtype=query.dtype, device=query.device)
-    # the kernels read pages by the table's ids, unchecked
-    pa.check_page_ranges(_host_lens(kv)[:B], _host_table(kv)[:B], kv.k_pages.shape[0], kv.page_size)
+    _check_histories(host[:B], _host_table(kv)[:B], kv.k_pages.shape[0], kv.page_size)
     sides = ((kv.k_pages, kv.k_norms, kv.k_quant), (kv.v_pages, kv.v_norms, kv.v_quant))
-    if _history_kernel(query, kv, Lmax):
-        k, v = (_histories(kv, *side, lens, Lmax, query.dtype) for side in sides)
-        return _history_attention(query, kv, k, v, Lmax, scaling)
+    if plain and _history_kernel(query, kv, Lmax):
+        with torch.cuda.device(query.device):
+            k, v = (_histories(kv, *side, host, Lmax, query.dtype) for side in sides)
+            return _history_attention(query, kv, k, v, Lmax, scaling)
+    lens = host.to(torch.int64)
     hist = []
     for pages, norms, quant in sides:
         buf = torch.zeros(B, kv.num_kv_heads, Lmax, D, dtype=query.dtype, device=query.device)
