@@ -41,7 +41,7 @@
 // order, zero between the groups; the norms, thresholds, grids and exact dot products
 // are taken per group, and the rows are packed byte by byte (a group's codes need not
 // fill eights). A prompt of 2,048 tokens (2 sequences, 8 heads; 120 channels at 4 bits, 8 at
-// 8) took sixteen launches and copies, a single token 25 us now, the prompt 53 us.
+// 8) took sixteen launches and copies; now the prompt takes 54 us, a single token 26 (traces).
 //
 // Measured (K and V of 8 kv heads in one launch, head_dim 128, quantize_kernel -> this):
 // 8,191 tokens 4 bits bf16 128 -> 30 us, 8 bits 133 -> 47 us, 4 bits fp32 119 -> 34 us;
