@@ -653,7 +653,7 @@ def prefill_bench(w, Q: int, nseq: int | None = None, steps: int = 10, warmup: i
     lengths count the Q tokens (the cache holds them before attention, as on the
     reference's Q > 1 route), query bf16 ~N(0, 1) seeded, output bf16. Beside it the
     reference's route on the same pages and GPU: each history dequantized to bf16, then
-    SDPA with the offset causal mask (``_reconstruct_sdpa``, packed_backend.py:211-226).
+    the library's SDPA with the offset causal mask (packed_backend.py:211-226).
 
     The scan is timed with HIP events on its stream; the call (rotate + scan + merge)
     with events around the calls. Its roofline, both ways: HBM, the packed K/V rows and
@@ -697,11 +697,13 @@ def prefill_bench(w, Q: int, nseq: int | None = None, steps: int = 10, warmup: i
     end.record()
     torch.cuda.synchronize()
     ms = start.elapsed_time(end) / steps
-    pb._reconstruct_sdpa(q, kv, scale)
+    host_lens = kv.seq_lens_host.long()
+    route = lambda: pb._library_sdpa(q, kv, host_lens, max(lens), scale)  # noqa: E731
+    route()
     torch.cuda.synchronize()
     start.record()
     for _ in range(ref_steps):
-        pb._reconstruct_sdpa(q, kv, scale)
+        route()
     end.record()
     torch.cuda.synchronize()
     ref_ms = start.elapsed_time(end) / ref_steps
@@ -716,7 +718,7 @@ def prefill_bench(w, Q: int, nseq: int | None = None, steps: int = 10, warmup: i
                    "frac": nbytes / (scan_ms * 1e-3) / 1e9 / HBM_PEAK_GBPS},
            "mfma": {"flops": flops, "achieved_TFLOPs": flops / (scan_ms * 1e-3) / 1e12,
                     "frac": flops / (scan_ms * 1e-3) / 1e12 / MFMA_F16_PEAK_TFLOPS},
-           "reference_route": "history dequantized to bf16, then SDPA with the offset causal mask "
+           "reference_route": "history dequantized to bf16, then the library's SDPA with the offset causal mask "
                               "(_reconstruct_sdpa, packed_backend.py:211-226)",
            "reference_route_us": ref_ms * 1e3, "speedup_vs_reference_route": ref_ms / ms,
            "products": "single fp16 operands (11 significant bits, rounded to nearest), fp32 accumulation"}
@@ -734,7 +736,8 @@ def prefill_bench(w, Q: int, nseq: int | None = None, steps: int = 10, warmup: i
         ref = oa.reconstruct_attention(qs.float().cpu(), host, scale)
         rr = tf32_class_reference(qs.float().cpu(), host, scale,
                                   q_log2=prefill_q_log2(wsc, len(seqs), Hq, c["Hkv"], Q)).float()
-        route = pb._reconstruct_sdpa(qs, sub2, scale).float().cpu()
+        cut = sub2.seq_lens_host.long()
+        route = pb._library_sdpa(qs, sub2, cut, int(cut.max()), scale).float().cpu()
         out["parity"] = {
             "sequences": seqs, "cut_to": check_len,
             "rounded_operand_ref_max_abs_err": (got - rr).abs().max().item(),

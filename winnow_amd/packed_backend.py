@@ -593,16 +593,23 @@ def _reconstruct_sdpa(query, kv: pa.PackedKV, scaling):
     if Lmax == 0:
         return torch.zeros(B, Hq, Q, D, dtype=query.dtype, device=query.device)
     _check_histories(host[:B], _host_table(kv)[:B], kv.k_pages.shape[0], kv.page_size)
-    sides = ((kv.k_pages, kv.k_norms, kv.k_quant), (kv.v_pages, kv.v_norms, kv.v_quant))
     if plain and _history_kernel(query, kv, Lmax):
         with torch.cuda.device(query.device):
-            k, v = (_histories(kv, *side, host, Lmax, query.dtype) for side in sides)
+            k, v = (_histories(kv, *side, host, Lmax, query.dtype) for side in _sides(kv))
             return _history_attention(query, kv, k, v, Lmax, scaling)
-    lens = host.to(torch.int64)
+    return _library_sdpa(query, kv, host.to(torch.int64), Lmax, scaling)
+
+
+def _sides(kv: pa.PackedKV):
+    return (kv.k_pages, kv.k_norms, kv.k_quant), (kv.v_pages, kv.v_norms, kv.v_quant)
+
+
+def _library_sdpa(query, kv: pa.PackedKV, lens: torch.Tensor, Lmax: int, scaling):
+    """The route with the library's SDPA, a history at a time into zeroed buffers; ranges checked."""
     hist = []
-    for pages, norms, quant in sides:
-        buf = torch.zeros(B, kv.num_kv_heads, Lmax, D, dtype=query.dtype, device=query.device)
-        for b in range(B):
+    for pages, norms, quant in _sides(kv):
+        buf = torch.zeros(query.shape[0], kv.num_kv_heads, Lmax, query.shape[-1], dtype=query.dtype, device=query.device)
+        for b in range(query.shape[0]):
             if lens[b]:
                 buf[b, :, :int(lens[b])] = _history(kv, pages, norms, quant, b, query.dtype)[0]
         hist.append(buf)
