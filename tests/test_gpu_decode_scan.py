@@ -143,6 +143,11 @@ def test_value_norms_of_any_size(D, S, Hq, Hkv, bwk, bwv, tf32):
     assert float(outs[0].abs().max()) > 0
     for e in (-15, 11):
         assert torch.equal(outs[e], outs[0])
+    # the scale is the magnitude's: negative norms give the attention negated, up to the sums'
+    # rounding, which is not the same for both signs (some thousand sums of 2^-24 each)
+    dev.v_norms.copy_(-norms)
+    out = pa.packed_decode_attention(q.cuda(), dev, scale, out_dtype=torch.float32, allow_tf32=tf32)
+    assert float((out + outs[0]).abs().max()) <= 2.0 ** -16 * float(outs[0].abs().max())
     dev.v_norms.zero_()
     out = pa.packed_decode_attention(q.cuda(), dev, scale, out_dtype=torch.float32, allow_tf32=tf32)
     assert (out == 0).all()

@@ -776,7 +776,7 @@ __device__ __forceinline__ void score_phase_mx(const RowBuf<BWK, BWV>& K, Tab16<
   wave_lds_sync();
 }
 
-// Value scale: 2^kRescale * max(n_V) * 2^-gs < 2^15, i.e. every n_V < 2^(7 + gs), with the
+// Value scale (nv: a lane's |n_V|): 2^kRescale * max|n_V| * 2^-gs < 2^15, i.e. every |n_V| < 2^(7 + gs), with the
 // smallest such gs, negative for small norms: an fp16 pair keeps 22 bits of a weight only
 // above 2^-3 (its low half ends at 2^-24), so the weights of a range go as far up as they
 // fit. The scale only grows, so the wave's maximum is taken only when a norm reaches
@@ -809,13 +809,13 @@ __device__ __forceinline__ void softmax_phase_mx(float sc, uint32_t nk_h, uint32
   // head i weighs token T of this lane, T = 0 except for PAIR's second four heads
   constexpr int NT = PAIR ? 2 : 1;
   bool valid[NT];
-  float nk[NT], nvt[NT], nv = 0.f;
+  float nk[NT], nvt[NT], nv = 0.f;  // nv: the larger magnitude, for the value scale
 #pragma unroll
   for (int T = 0; T < NT; ++T) {
     valid[T] = left > T;
     nk[T] = half_lo(nk_h >> (16 * T)) * sc;
     nvt[T] = valid[T] ? half_lo(nv_h >> (16 * T)) : 0.f;
-    nv = T ? fmaxf(nv, nvt[T]) : nvt[T];
+    nv = T ? fmaxf(nv, fabsf(nvt[T])) : fabsf(nvt[T]);
   }
   float sv[H];
   if constexpr (kTileHalves<NG>) {
@@ -1031,7 +1031,7 @@ __device__ __forceinline__ void softmax_phase_tf(float sc, uint32_t nk_h, uint32
   read_unconditionally(x);
 #pragma unroll
   for (int i = 0; i < H; ++i) sv[i] = valid ? x[i] * nk : -INFINITY;
-  raise_value_scale(nv, st);
+  raise_value_scale(fabsf(nv), st);
   float d[H], dmax = -INFINITY;
 #pragma unroll
   for (int i = 0; i < H; ++i) {
